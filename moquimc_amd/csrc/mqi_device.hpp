@@ -175,6 +175,7 @@ MQI_DI float momentum(const rel_q& r) {
 #endif
 }
 
+#if MQI_EXACT   // the production build's are in mqi_prod.hpp
 MQI_DI float intpl(float x, float x0, float x1, float y0, float y1) {
     return (x1 == x0) ? y0 : y0 + (x - x0) * (y1 - y0) / (x1 - x0);
 }
@@ -209,18 +210,11 @@ MQI_DI float radiation_length(float rho_mass) {
     } else if (density > 0.26 && density <= 0.9) {
         f = 1.0446 - 0.2180 * density;
     } else if (density > 0.9) {
-#if MQI_EXACT
         f = 1.19 + 0.44 * MQ_LOGD((double) (density - 0.44));
-#else
-        f = 1.19f + 0.44f * __logf(density - 0.44f);   // production: float
-#endif
     }
-#if MQI_EXACT
     return (float) ((units::water_density * units::X0_water) / (density * 0.001 * f));
-#else
-    return (units::water_density * units::X0_water) / (density * 0.001f * f);
-#endif
 }
+#endif
 
 // hu_to_density (mqi_patient_materials.hpp:515-542)
 MQI_DI float hu_to_density(int hu_in, const float* corr) {
@@ -313,6 +307,7 @@ MQI_DI void index3(const grid_view& g, v3 p, v3 d, int& cx, int& cy, int& cz) {
     cz = scan_axis(g.ze, g.sz, g.nz, p.z, d.z);
 }
 
+#if MQI_EXACT   // production: exit_distance (mqi_prod.hpp)
 // one axis of intersect(p, d, idx) (mqi_grid3d.hpp:519-545); mutates dcomp
 MQI_DI void axis_in(float& dcomp, float p, float v1, float v2, int i, int n, float& tmax) {
     MQI_NO_CONTRACT
@@ -352,6 +347,7 @@ MQI_DI float intersect_in(const grid_view& g, v3 p, v3& d, int& cx, int& cy, int
     cx = cy = cz = -1;
     return -1.0f;
 }
+#endif
 
 MQI_DI void axis_out(float& dcomp, float p, float lo, float hi, float& tmin, float& tmax) {
     MQI_NO_CONTRACT
@@ -572,7 +568,7 @@ struct rng_t {
         // last two take revolutions: sin(2 pi u))
         const float u1 = mqi_rng::stream::to_uniform(w.v[1]);
         const float u2 = mqi_rng::stream::to_uniform(w.v[2]);
-        const float r  = __builtin_sqrtf(-2.0f * 0.693147180559945309f * __builtin_amdgcn_logf(u1));
+        const float r  = __builtin_amdgcn_sqrtf(-2.0f * 0.693147180559945309f * __builtin_amdgcn_logf(u1));
         st_z0          = r * __builtin_amdgcn_cosf(u2);
         st_z1          = r * __builtin_amdgcn_sinf(u2);
 #endif

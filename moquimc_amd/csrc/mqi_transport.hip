@@ -16,6 +16,12 @@
 // (namespace mqi_fast, device math library, FMA contraction).
 #include "mqi_device.hpp"
 #include "mqi_kernels.h"
+#if MQI_EXACT
+#define MQI_VOXEL_EXIT mqi_dev::intersect_in
+#else
+#include "mqi_prod.hpp"
+#define MQI_VOXEL_EXIT mqi_dev::exit_distance
+#endif
 
 #define MQI_TABLE_QUALIFIER static __constant__
 #include "mqi_tables.inc"
@@ -48,6 +54,7 @@ struct ctx {
     const float* blxf;     // their transforms (fwd[9], inv[9], translation[3] each), HBM
 };
 
+#if MQI_EXACT
 // p_ionization_tabulated::cross_section (mqi_p_ionization.hpp:254-268): Ei=0.1, Ef=299.6, step 0.5
 MQI_DI float cs_ion(const ctx& c, float Ek, float rho) {
     float cs = 0;
@@ -104,36 +111,12 @@ MQI_DI float energy_loss(ctx& c, const rel_q& rel, float rho, float step_length,
     float r = intpl(rel.Ek, x0, x1, R[n], R[n + 1]);
     if (r < L_w) return rel.Ek;
     r -= L_w;
-#if MQI_EXACT
     for (;;) {
         if (r >= R[n]) break;
         if (n == 0) break;
         --n;
         if (n == 0) break;
     }
-#else
-    // The walk above ends at the largest n in [1, n0] with R[n] <= r (0 if
-    // none), R being non-decreasing.  Walking from the current bin takes one
-    // LDS round trip per 0.5 MeV lost, the longest lane setting the wave's
-    // count (8.3 per step on the 2000-spot CT plan); here the walk starts at
-    // the bin the range slope of the current bin predicts, and goes up or
-    // down from there to the same n.
-    {
-        const int n0 = n;
-        const float slope = R[n0 + 1] - R[n0];   // mm per 0.5 MeV
-        int         k     = slope > 0.0f ? (int) (L_w / slope) : 0;
-        int         m     = n0 - (k < n0 ? k : n0);
-        if (m >= 1 && R[m] > r) {
-            do {
-                --m;
-            } while (m >= 1 && R[m] > r);
-            if (m < 1) m = 0;
-        } else {
-            while (m < n0 && R[m + 1] <= r) ++m;
-        }
-        n = (uint16_t) m;
-    }
-#endif
     x0            = 0.1f + n * 0.5f;
     x1            = x0 + 0.5f;
     float dE_mean = rel.Ek - intpl(r, R[n], R[n + 1], x0, x1);
@@ -167,6 +150,113 @@ MQI_DI void along_step(ctx& c, trk& t, float len, float rho, float sp) {
     update_pos(t, r * len);
     t.ke1 -= dE * r;
 }
+
+#else
+// Cross sections per density of the four processes at Ek (cs_ion, cs_tab)
+// and, with DEDX, dEdx: the two index grids of the tables (0.1 + 0.5 i and
+// 0.5 + 0.5 i MeV) are evaluated once for the tables that share them.
+struct q_cs {
+    float ion, pp, poe, poi;
+};
+template<bool DEDX>
+MQI_DI q_cs q_cross(const float* T, float Ek, float* pw) {
+    MQI_NO_CONTRACT
+    q_cs         c;
+    const bool   in = Ek >= 0.1f && Ek <= 299.6f;
+    const int    i  = in ? (int) ((Ek - 0.1f) * 2.0f) : 0;
+    const float  x0 = __builtin_fmaf((float) i, 0.5f, 0.1f);
+    const float  dx = Ek - x0;
+    const float  rw = __builtin_amdgcn_rcpf((x0 + 0.5f) - x0);
+    const float* t  = T + i;
+    c.ion           = t[T_CS_ION] + dx * (t[T_CS_ION + 1] - t[T_CS_ION]) * rw;
+    if (DEDX) {
+        *pw = t[T_DEDX] + dx * (t[T_DEDX + 1] - t[T_DEDX]) * rw;
+        if (!in) *pw = (Ek < 0.1f && Ek > 0) ? T[T_DEDX] : 0.0f;
+    }
+    const bool   jn = Ek >= 0.5f && Ek <= 300.0f;
+    const int    j  = jn ? (int) ((Ek - 0.5f) * 2.0f) : 0;
+    const float  dy = Ek - __builtin_fmaf((float) j, 0.5f, 0.5f);
+    const float* u  = T + j;
+    // the bins are 0.5 wide exactly: the quotient is a doubling
+    c.pp  = __builtin_fmaf(dy * (u[T_CS_PP + 1] - u[T_CS_PP]), 2.0f, u[T_CS_PP]);
+    c.poe = __builtin_fmaf(dy * (u[T_CS_POE + 1] - u[T_CS_POE]), 2.0f, u[T_CS_POE]);
+    c.poi = __builtin_fmaf(dy * (u[T_CS_POI + 1] - u[T_CS_POI]), 2.0f, u[T_CS_POI]);
+    if (!in) c.ion = 0.0f;
+    if (!jn) c.pp = c.poe = c.poi = 0.0f;
+    return c;
+}
+MQI_DI float q_sum(const q_cs& c, float rho) {
+    MQI_NO_CONTRACT
+    return __builtin_fmaf(rho, c.poi, __builtin_fmaf(rho, c.poe, __builtin_fmaf(rho, c.ion, rho * c.pp)));
+}
+
+// energy_loss + energy_straggling: the residual-range walk of the
+// verification build ends at the largest n in [1, n0] with R[n] <= r (0 if
+// none), R being non-decreasing.  Walking from the current bin takes one LDS
+// round trip per 0.5 MeV lost, the longest lane setting the wave's count (8.3
+// per step on the 2000-spot CT plan); here the walk starts at the bin the
+// range slope of the current bin predicts, and goes down or up from there to
+// the same n (1.7 round trips).
+MQI_DI float q_energy_loss(ctx& c, const q_rel& rel, float Ek, float rho, float L_w) {
+    MQI_NO_CONTRACT
+    const float* R  = c.T + T_RANGE;
+    int          n  = (int) ((Ek - 0.1f) * 2.0f);
+    const float  x0 = __builtin_fmaf((float) n, 0.5f, 0.1f);
+    const float  x1 = x0 + 0.5f;
+    if (x0 > Ek) n -= 1;
+    if (x1 < Ek) n += 1;
+    const float slope = R[n + 1] - R[n];   // mm per 0.5 MeV
+    float       r     = R[n] + q_div((Ek - x0) * slope, x1 - x0);
+    if (r < L_w) return Ek;
+    r -= L_w;
+    int k = slope > 0.0f ? (int) q_div(L_w, slope) : 0;
+    k     = k < 0 ? 0 : k;
+    int   m = n - (k < n ? k : n);
+    float a = R[m], b = R[m + 1];
+    while (m >= 1 && a > r) {
+        --m;
+        b = a;
+        a = R[m];
+    }
+    while (m < n && b <= r) {
+        ++m;
+        a = b;
+        b = R[m + 1];
+    }
+    const float y0 = __builtin_fmaf((float) m, 0.5f, 0.1f);
+    const float w  = b - a;
+    const float E1 = w == 0.0f ? y0 : y0 + q_div((r - a) * ((y0 + 0.5f) - y0), w);
+    const float te = q_te_max(rel);
+    const float Te = te >= at_least(0.08511) ? 0.08511f : te;
+    const float  O = q_div(units::two_pi_re2_mc2_h2o * rho, units::water_density) * L_w;
+    const double g = __builtin_fma((double) rel.beta_sq, -0.5, 1.0) * (double) q_div(Te, rel.beta_sq);
+    const float  O_sq = (float) (g * (double) O);
+    return fabsf(__builtin_fmaf(c.rng.st_z0, q_sqrt(O_sq), Ek - E1));
+}
+
+// along_step (mqi_p_ionization.hpp:348-420) from the step's sp * len
+template<bool DBG>
+MQI_DI void q_along_step(ctx& c, trk& t, float len, float rho, float sp) {
+    MQI_NO_CONTRACT
+    const q_rel rel = q_relq(t.ke0);
+    const float L_w = q_div(len * sp * rho, units::water_density);
+    const float dE  = q_energy_loss(c, rel, t.ke0, rho, L_w);
+    float       r   = 1.0f;
+    if (dE >= t.ke0) {
+        r         = r_div(t.ke0, dE);
+        t.stopped = true;
+    }
+    const float q     = q_div(13.9f, q_sqrt(rel.pp));
+    const float th_sq = q_div(q_div(q * q, rel.beta_sq) * len, q_radiation_length<DBG>(rho));
+    const float th    = fabsf(c.rng.st_z1 * (0x1.6a09e6p+0f * q_sqrt(th_sq)));   // sqrt(2)
+    const float phi   = (float) (2.0 * 3.14159265358979323846 * (double) c.rng.st_u1);
+    q_rotate(t.d1, th, phi);
+    t.dE = __builtin_fmaf(dE, r, t.dE);
+    update_pos(t, r * len);
+    t.ke1 = __builtin_fmaf(-dE, r, t.ke1);
+}
+
+#endif
 
 // secondary placement: pos -> fwd (pos - T) + T, dir -> fwd dir (e.g.
 // mqi_pp_elastic.hpp:190-196), with the transform of the child the track is
@@ -218,6 +308,7 @@ MQI_DI void push_placed(ctx& c, float ke0, v3 p, v3 d, float ke1, float dE) {
         push(c, ke0, place(c, p), turn(c, d), ke1, dE, -1.0f);
 }
 
+#if MQI_EXACT
 // p_ionization_tabulated::post_step: delta-ray (mqi_p_ionization.hpp:424-477)
 template<bool DBG>
 MQI_DI void post_ion(ctx& c, trk& t) {
@@ -240,6 +331,39 @@ MQI_DI void post_ion(ctx& c, trk& t) {
     }
     t.ke1 -= Te;
 }
+#else
+// p_ionization_tabulated::post_step: delta-ray (mqi_p_ionization.hpp:424-477).
+// The first trial's numbers come from the interaction's block; the later
+// ones (acceptance is above 1/2) from the history's stream.
+template<bool DBG>
+MQI_DI void post_ion(ctx& c, trk& t) {
+    MQI_NO_CONTRACT
+    const q_rel  rel    = q_relq(t.ke1);
+    const float  te_max = q_te_max(rel);
+    const float  T_cut  = DBG ? 0.08511 * 1.0 : 0.0815 * 1.0;
+    const double num    = (double) (T_cut * te_max);
+    const double temd   = (double) te_max;
+    const float  rte    = __builtin_amdgcn_rcpf(te_max);
+    const double e2     = 2.0 * (double) rel.Et_sq;
+    const double re2    = d_recip(e2);
+    float        n = c.rng.it_u1, acc = c.rng.it_u2, Te;
+    // the bound only ends the loop for non-finite input
+    for (int it = 0;; ++it) {
+        const double den = __builtin_fma(1.0 - (double) n, temd, (double) (n * T_cut));
+        Te               = (float) d_quot(num, den, d_recip(den));
+        const double a   = 1.0 - (double) (rel.beta_sq * Te * rte);
+        if ((double) acc < a + d_quot((double) (Te * Te), e2, re2) || it == 4095) break;
+        n   = c.rng.uniform();
+        acc = c.rng.uniform();
+    }
+    if (DBG) {
+        push_placed(c, 0.0f, t.p0, t.d0, 0.0f, Te);
+    } else {
+        t.dE += Te;
+    }
+    t.ke1 -= Te;
+}
+#endif
 
 // pp_elastic_tabulated::post_step (mqi_pp_elastic.hpp:119-219)
 MQI_DI void post_pp(ctx& c, trk& t) {
@@ -366,6 +490,7 @@ MQI_DI void post_poi(ctx& c, trk& t) {
     t.stopped = true;
 }
 
+#if MQI_EXACT
 // fippel_physics::stepping (mqi_fippel_physics.hpp:68-216).  The three
 // branches' along_step calls are merged into one call with the branch's
 // length; the random-number order is unchanged.  The stopping power ratio
@@ -446,6 +571,78 @@ MQI_DI void stepping(ctx& c, trk& t, float rho, float d2b, float& sp) {
         post_poi<DBG>(c, t);
     }
 }
+#else
+// The same with the step's common terms formed once (mqi_prod.hpp): one
+// stopping power ratio for every kind of step, both energies' cross sections
+// from shared table indices.
+template<bool DBG>
+MQI_DI void stepping(ctx& c, trk& t, float rho, float d2b, float& sp) {
+    MQI_NO_CONTRACT
+    if (rho < at_least(1.0e-7)) {
+        sp = 0.0f;   // vacuum: the dose hit returns before reading it
+        update_pos(t, d2b);
+        return;
+    }
+    const bool block = rho > at_most(99.9);
+    if (!block && t.ke0 < 0) t.ke0 = 0;
+    sp = q_spr<DBG>(rho, t.ke0);
+    if (block) {
+        t.stopped = true;
+        return;
+    }
+    if (t.ke0 <= 0.5f) {
+        t.dE += t.ke0;
+        t.ke1 -= t.ke0;
+        // last_step (mqi_p_ionization.hpp:481-490)
+        float L_w = 0;
+        if (t.dE > 0) {
+            float pw;
+            q_cross<true>(c.T, t.ke0, &pw);
+            L_w = geo_div(t.dE, pw);
+        }
+        update_pos(t, q_div(L_w * units::water_density, sp * rho));
+        t.stopped = true;
+        return;
+    }
+    const float sr  = sp * rho;
+    const float cms = q_div(sr, units::water_density);
+    float       pw;
+    const q_cs  c1   = q_cross<true>(c.T, t.ke0, &pw);
+    const q_cs  c2   = q_cross<false>(c.T, t.ke0 - cms * pw, nullptr);
+    const float sum1 = q_sum(c1, rho), sum2 = q_sum(c2, rho);
+    const bool  first  = sum1 >= sum2;
+    const float cs_sum = first ? sum1 : sum2;
+    const float ion = first ? c1.ion : c2.ion, pp = first ? c1.pp : c2.pp, poe = first ? c1.poe : c2.poe,
+                poi = first ? c1.poi : c2.poi;
+    c.rng.begin_step();
+    const float mfp        = q_div(-q_log(c.rng.st_u0), cs_sum);
+    const float step_limit = q_div(cms * units::water_density, sr);
+    float       len        = step_limit;
+    bool        interact   = false;
+    if (d2b < mfp && d2b < step_limit) {
+        len = d2b;
+    } else if ((mfp < d2b || fabsf(mfp - d2b) < 1e-3f) &&
+               (mfp < step_limit || fabsf(mfp - step_limit) < 1e-3f)) {
+        len      = mfp;
+        interact = true;
+    }
+    q_along_step<DBG>(c, t, len, rho, sp);
+    if (!interact || t.ke1 <= 0.5f) return;
+    c.rng.begin_interaction();
+    const float u  = cs_sum * c.rng.it_u0;
+    const float s0 = rho * ion, s1 = s0 + rho * pp, s2 = s1 + rho * poe, s3 = s2 + rho * poi;
+    t.d1           = t.d0;
+    if (u < s0) {
+        post_ion<DBG>(c, t);
+    } else if (u < s1) {
+        post_pp(c, t);
+    } else if (u < s2) {
+        post_poe<DBG>(c, t);
+    } else if (u < s3) {
+        post_poi<DBG>(c, t);
+    }
+}
+#endif
 
 // ------------------------------------------------------------------ scoring
 // hit functions (mqi_scorer_energy_deposit.hpp:43-139)
@@ -950,12 +1147,12 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
         const int*     m   = P.bl_meta + 8 * c.child;
         const uint64_t off = (uint64_t) (uint32_t) m[4] | ((uint64_t) (uint32_t) m[5] << 32);
         cnb                = (uint64_t) (int32_t) (t.cz * gb.nx * gb.ny + t.cy * gb.nx + t.cx);
-        t.its              = intersect_in(gb, t.p0, t.d0, t.cx, t.cy, t.cz);
+        t.its              = MQI_VOXEL_EXIT(gb, t.p0, t.d0, t.cx, t.cy, t.cz);
         rho                = P.bl_density[off + cnb];
     } else {
         cnb              = (uint64_t) (int32_t) (t.cz * c.g.nx * c.g.ny + t.cy * c.g.nx + t.cx);
         const float dens = P.density[cnb];
-        t.its            = intersect_in(c.g, t.p0, t.d0, t.cx, t.cy, t.cz);
+        t.its            = MQI_VOXEL_EXIT(c.g, t.p0, t.d0, t.cx, t.cy, t.cz);
         rho              = dens * L.scale;
         // The deposits gathered in the voxel the lane has left go out here,
         // after the wait for the density and ahead of the physics of the
@@ -1313,14 +1510,23 @@ __global__ void __launch_bounds__(256) k_physics_probe(int fn, const float* rho,
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     if (fn == 0) {
+#if MQI_EXACT
         out[i] = spr<DBG>(rho[i], ek[i]);
+#else
+        out[i] = q_spr<DBG>(rho[i], ek[i]);
+#endif
     } else if (fn == 1) {
+#if MQI_EXACT
         out[i] = radiation_length<DBG>(rho[i]);
+#else
+        out[i] = q_radiation_length<DBG>(rho[i]);
+#endif
     } else {
+        float* o = out + 10 * i;
+#if MQI_EXACT
         ctx c;
         c.T           = sh;
         const rel_q r = relq(ek[i]);
-        float*      o = out + 10 * i;
         o[0]          = cs_ion(c, r.Ek, rho[i]);
         o[1]          = cs_tab(c, T_CS_PP, r.Ek, rho[i]);
         o[2]          = cs_tab(c, T_CS_POE, r.Ek, rho[i]);
@@ -1331,6 +1537,21 @@ __global__ void __launch_bounds__(256) k_physics_probe(int fn, const float* rho,
         o[7]          = r.Et;
         o[8]          = r.Te_max;
         o[9]          = momentum(r);
+#else
+        float       pw;
+        const q_cs  c = q_cross<true>(sh, ek[i], &pw);
+        const q_rel r = q_relq(ek[i]);
+        o[0]          = c.ion * rho[i];
+        o[1]          = c.pp * rho[i];
+        o[2]          = c.poe * rho[i];
+        o[3]          = c.poi * rho[i];
+        o[4]          = -pw;
+        o[5]          = r.beta_sq;
+        o[6]          = q_div(r.Et, units::Mp);
+        o[7]          = r.Et;
+        o[8]          = q_te_max(r);
+        o[9]          = q_sqrt(r.pp);
+#endif
     }
 }
 
