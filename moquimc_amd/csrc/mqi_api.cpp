@@ -609,6 +609,13 @@ fill_params(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg) {
         P.dij_vals     = c->d_dij_vals;
         P.dij_off      = c->d_dij_off;
     }
+    P.dij_slot = -1;
+    for (int k = 0; k < P.n_scorers; ++k) {
+        const int kd = P.kinds[k];
+        if (kd == MQI_KIND_DIJ) P.dij_slot = k;
+        if (kd == MQI_KIND_LETD_NUM || kd == MQI_KIND_LETD_DEN || kd == MQI_KIND_LETT_NUM || kd == MQI_KIND_LETT_DEN)
+            P.let_kinds = 1;
+    }
     P.out_scenario_stride = c->per_scen ? nvox(c) : 0;
     P.loops               = cfg.scoring_loops;
     P.stack               = c->d_stack;

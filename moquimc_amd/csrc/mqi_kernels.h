@@ -99,6 +99,8 @@ struct transport_params {
     double*  out[MQI_MAX_SCORERS];
     uint64_t out_scenario_stride;   // 0: scenarios share the arrays; else per-scenario offset (elements)
     int      loops;
+    int      let_kinds;   // any LETd / LETt scorer
+    int      dij_slot;    // the Dij scorer's slot, -1: none
     // Grouped scoring (production kernels, each-scorer-once, no Dij): the
     // leading group_ns scorers (2 .. 4) add into one interleaved array with
     // pair (2 or 4; 0: off) doubles per element, element i of scorer s at

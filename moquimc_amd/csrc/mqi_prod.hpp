@@ -86,6 +86,19 @@ MQI_DI double d_quot(double a, double b, double r) {
     return __builtin_fma(__builtin_fma(-b, q, a), r, q);
 }
 
+// correctly rounded square root in double of a normal a > 0 (the compiler's
+// sequence without its range scaling)
+MQI_DI double d_sqrt(double a) {
+    MQI_NO_CONTRACT
+    const double y = __builtin_amdgcn_rsq(a);
+    double       g = a * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g              = __builtin_fma(g, r, g);
+    h              = __builtin_fma(h, r, h);
+    g              = __builtin_fma(__builtin_fma(-g, g, a), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, a), h, g);
+}
+
 MQI_DI void q_normalize(v3& a) {   // normalize_fast
     MQI_NO_CONTRACT
     const float r = __builtin_amdgcn_rcpf(q_sqrt(a.x * a.x + a.y * a.y + a.z * a.z));

@@ -656,34 +656,32 @@ MQI_DI double dose_hit(const trk& t, float density, float volume, float sp) {
     return (double) ((t.dE + t.ldE) * 1.60218e-10f / (volume * density * sp));
 #endif
 }
-// LETt_weight1 / LETt_weight2 (mqi_scorer_energy_deposit.hpp:141-177)
-MQI_DI double lett_hit(const trk& t, float density, bool numer) {
-    density *= 1000.0;
-    double length = (t.p1.x - t.p0.x) * (t.p1.x - t.p0.x);
-    length += (t.p1.y - t.p0.y) * (t.p1.y - t.p0.y);
-    length += (t.p1.z - t.p0.z) * (t.p1.z - t.p0.z);
-    length = MQ_SQRTD(length);
-    if (length <= 0) return 0.0;
-    if (!numer) return length;
-    double let = t.dE / length / density;
-    return length * let;
-}
 // energy_deposit (:14-20); dose_to_medium of primaries in J/kg (:80-92)
 MQI_DI double edep_hit(const trk& t) { return t.dE + t.ldE; }
 MQI_DI double dm_hit(const trk& t, float density, float volume) {
     return t.primary ? t.dE * 1.60218e-13 * 1000.0 / (volume * density) : 0.0;
 }
-
-MQI_DI double letd_hit(const trk& t, float density, bool numer) {
+// step length and dE / length / density of the LETd and LETt scorers
+// (LETd_weight1/2 :93-139, LETt_weight1/2 :141-177); false for no length.
+// One square root and two divisions in FP64: formed once per step, and only
+// for plans that score a LET (evaluated per scorer they were hoisted out of
+// the scorers' branches and ran for every plan, 90 FP64 instructions a step).
+MQI_DI bool let_terms(const trk& t, float density, double& length, double& let) {
     density *= 1000.0;
-    double length = (t.p1.x - t.p0.x) * (t.p1.x - t.p0.x);
+    length = (t.p1.x - t.p0.x) * (t.p1.x - t.p0.x);
     length += (t.p1.y - t.p0.y) * (t.p1.y - t.p0.y);
     length += (t.p1.z - t.p0.z) * (t.p1.z - t.p0.z);
+#if MQI_EXACT
     length = MQ_SQRTD(length);
-    if (length <= 0) return 0.0;
-    double let = t.dE / length / density;
-    if (let >= 25.0) return 0;
-    return numer ? t.dE * let : t.dE * 1.0;
+    if (length <= 0) return false;
+    let = t.dE / length / density;
+#else
+    if (length <= 0) return false;
+    length          = d_sqrt(length);
+    const double dn = (double) density;
+    let             = d_quot(d_quot((double) t.dE, length, d_recip(length)), dn, d_recip(dn));
+#endif
+    return true;
 }
 
 // Dij: per-spot open-addressing table of (voxel, dose) in HBM.  Keys are
@@ -725,33 +723,62 @@ MQI_DI void dij_insert(const transport_params& P, uint64_t item, uint32_t voxel,
 // and every scratch reload waits on the one counter the atomics in flight
 // also hold.
 struct pending {
-    int64_t  cnb;    // voxel of the pending sums, -1: none
-    uint64_t off;    // scenario offset of the pending sums
-    uint32_t item;   // Dij table (scenario, spot) of the pending sums
+    int32_t  cnb;    // voxel of the pending sums, -1: none
+    uint32_t scen;   // their scenario
+    uint32_t item;   // their Dij table (scenario, spot)
 };
+MQI_DI uint64_t pend_element(const transport_params& P, const pending& A) {
+    return P.out_scenario_stride * A.scen + (uint32_t) A.cnb;
+}
 
+// accumulated slots are positive, +inf or NaN (every value that is not <= 0
+// is added, NaN included); untouched slots are 0
 MQI_DI void flush(const transport_params& P, pending& A, double* v) {
     if (A.cnb >= 0) {
-        // accumulated slots are positive, +inf or NaN (the per-step path adds
-        // every value that is not <= 0, NaN included); untouched slots are 0
+        const uint64_t k  = pend_element(P, A);
+        double         dx = 0.0;   // the Dij slot's sum: inserted behind the loop, from one place
 #pragma unroll
         for (int s = 0; s < MQI_DEFER; ++s) {
+            if (s >= P.n_scorers) break;
             const double x = v[s * blockDim.x];
-            if (x == 0.0) continue;
-            if (P.kinds[s] == MQI_KIND_DIJ)
-                dij_insert(P, A.item, (uint32_t) A.cnb, x);
+            if (s == P.dij_slot) {
+                dx = x;
+            } else if (x != 0.0) {
 #if !MQI_EXACT
-            else if (P.pair && s < P.group_ns)
-                atomicAdd(P.pair_out + (uint64_t) P.pair * (A.off + (uint64_t) A.cnb) + s, x);
+                if (P.pair && s < P.group_ns)
+                    atomicAdd(P.pair_out + (uint64_t) P.pair * k + s, x);
+                else
 #endif
-            else
-                atomicAdd(P.out[s] + A.off + (uint64_t) A.cnb, x);
+                    atomicAdd(P.out[s] + k, x);
+            }
         }
+        if (dx != 0.0) dij_insert(P, A.item, (uint32_t) A.cnb, dx);
     }
     A.cnb = -1;
 }
 
 #if !MQI_EXACT
+// a lane's value from another lane of its group of four (DPP quad_perm: one
+// instruction, no LDS round trip as ds_bpermute has); lanes that are not
+// active read as `old`
+template<int CTRL>
+MQI_DI int quad_get(int old, int x) {
+    return __builtin_amdgcn_update_dpp(old, x, CTRL, 0xf, 0xf, false);
+}
+template<int CTRL>
+MQI_DI uint64_t quad_get(uint64_t x) {
+    const uint32_t lo = (uint32_t) quad_get<CTRL>(0, (int) (uint32_t) x);
+    const uint32_t hi = (uint32_t) quad_get<CTRL>(0, (int) (uint32_t) (x >> 32));
+    return (uint64_t) hi << 32 | lo;
+}
+template<int CTRL>
+MQI_DI double quad_get(double x) {
+    return __longlong_as_double((long long) quad_get<CTRL>((uint64_t) __double_as_longlong(x)));
+}
+#define QUAD_XOR1 0xB1          // quad_perm [1, 0, 3, 2]
+#define QUAD_XOR2 0x4E          // quad_perm [2, 3, 0, 1]
+#define QUAD_OF(j) ((j) * 0x55) // quad_perm [j, j, j, j]
+
 // The flush of the step with paired scoring, run by every lane that steps
 // (f: this lane leaves its voxel).  Lanes 2m and 2m+1 exchange their sums:
 // the first atomic instruction adds both of lane 2m's sums (scorer 0 from
@@ -759,138 +786,125 @@ MQI_DI void flush(const transport_params& P, pending& A, double* v) {
 // two adds of a voxel land in one line of the interleaved array in one
 // instruction.  A lane whose partner does not step adds both of its own.
 MQI_DI void flush_pair(const transport_params& P, pending& A, double* v, bool f) {
-    const bool     has = f && A.cnb >= 0;
-    const double   a   = has ? v[0] : 0.0;
-    const double   b   = has ? v[blockDim.x] : 0.0;
-    const uint64_t k   = has ? A.off + (uint64_t) A.cnb : 0;
-    const int      me  = __lane_id();
-    const bool     pact = (__ballot(1) >> (me ^ 1)) & 1ull;
-    const uint64_t kp  = __shfl_xor((unsigned long long) k, 1);
-    const double   ap  = __shfl_xor(a, 1);
-    const double   bp  = __shfl_xor(b, 1);
-    const bool     odd = me & 1;
-    uint64_t       eA = 2 * k, eB = 2 * k + 1;   // partner stepping: overwritten
-    double         xA = a, xB = b;
-    if (pact) {
-        eA = odd ? 2 * kp + 1 : 2 * k;
-        xA = odd ? bp : a;
-        eB = odd ? 2 * k + 1 : 2 * kp;
-        xB = odd ? b : ap;
-    }
+    const bool     has  = f && A.cnb >= 0;
+    const double   a    = has ? v[0] : 0.0;
+    const double   b    = has ? v[blockDim.x] : 0.0;
+    const uint64_t k    = 2 * (has ? pend_element(P, A) : 0);
+    const bool     pact = quad_get<QUAD_XOR1>(0, 1) != 0;
+    const uint64_t kp   = quad_get<QUAD_XOR1>(k);
+    const double   ap   = quad_get<QUAD_XOR1>(a);
+    const double   bp   = quad_get<QUAD_XOR1>(b);
+    const bool     odd  = __lane_id() & 1;
+    const bool     swA = pact && odd, swB = pact && !odd;
+    const uint64_t eA = swA ? kp + 1 : k, eB = swB ? kp : k + 1;
+    const double   xA = swA ? bp : a, xB = swB ? ap : b;
     if (xA != 0.0) atomicAdd(P.pair_out + eA, xA);
     if (xB != 0.0) atomicAdd(P.pair_out + eB, xB);
-    if (has) {
-#pragma unroll
-        for (int s = 2; s < MQI_DEFER; ++s) {
-            const double x = v[s * blockDim.x];
-            if (x != 0.0) atomicAdd(P.out[s] + A.off + (uint64_t) A.cnb, x);
-        }
-        A.cnb = -1;
-    }
+    if (has) A.cnb = -1;
+}
+
+// lanes q and q ^ D of each group exchange halves of (x, y): the even lane
+// keeps its x and gets the other's x as y, the odd one the reverse
+template<int CTRL>
+MQI_DI void quad_swap(bool up, double& x, double& y) {
+    const double t = quad_get<CTRL>(up ? x : y);
+    if (up)
+        x = t;
+    else
+        y = t;
 }
 
 // The same for three or four grouped scorers (interleaved four doubles per
 // element): in a group of four stepping lanes, instruction j adds the sums of
 // lane 4m+j's voxel, lane 4m+q adding that lane's sum of scorer q, so all of
-// a voxel's sums go out as one line request.  Lanes of a group with a lane
-// that does not step add their own sums.
+// a voxel's sums go out as one line request (the sums are transposed within
+// the group in two exchanges).  Lanes of a group with a lane that does not
+// step add their own sums.
 MQI_DI void flush_quad(const transport_params& P, pending& A, double* v, bool f) {
     const bool     has = f && A.cnb >= 0;
-    const double   x0  = has ? v[0] : 0.0;
-    const double   x1  = has ? v[blockDim.x] : 0.0;
-    const double   x2  = has ? v[2 * blockDim.x] : 0.0;
-    const double   x3  = (has && P.group_ns > 3) ? v[3 * blockDim.x] : 0.0;
-    const uint64_t k   = has ? A.off + (uint64_t) A.cnb : 0;
-    const int      me  = __lane_id();
-    const int      q   = me & 3;
-    const int      g0  = me & ~3;
-    if (((__ballot(1) >> g0) & 0xfull) == 0xfull) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint64_t kj = __shfl((unsigned long long) k, g0 + j);
-            const double   y0 = __shfl(x0, g0 + j);
-            const double   y1 = __shfl(x1, g0 + j);
-            const double   y2 = __shfl(x2, g0 + j);
-            const double   y3 = __shfl(x3, g0 + j);
-            const double   y  = q == 0 ? y0 : (q == 1 ? y1 : (q == 2 ? y2 : y3));
-            if (y != 0.0) atomicAdd(P.pair_out + 4 * kj + q, y);
-        }
+    double         x0  = has ? v[0] : 0.0;
+    double         x1  = has ? v[blockDim.x] : 0.0;
+    double         x2  = has ? v[2 * blockDim.x] : 0.0;
+    double         x3  = (has && P.group_ns > 3) ? v[3 * blockDim.x] : 0.0;
+    const uint64_t k   = 4 * (has ? pend_element(P, A) : 0);
+    const int      q   = __lane_id() & 3;
+    const int      all = quad_get<QUAD_OF(0)>(0, 1) & quad_get<QUAD_OF(1)>(0, 1) & quad_get<QUAD_OF(2)>(0, 1) &
+                    quad_get<QUAD_OF(3)>(0, 1);
+    if (all) {
+        const bool u1 = q & 1, u2 = q & 2;
+        quad_swap<QUAD_XOR1>(u1, x0, x1);
+        quad_swap<QUAD_XOR1>(u1, x2, x3);
+        quad_swap<QUAD_XOR2>(u2, x0, x2);
+        quad_swap<QUAD_XOR2>(u2, x1, x3);
+        // x_j: scorer q of lane 4m+j
+        const uint64_t k0 = quad_get<QUAD_OF(0)>(k), k1 = quad_get<QUAD_OF(1)>(k), k2 = quad_get<QUAD_OF(2)>(k),
+                       k3 = quad_get<QUAD_OF(3)>(k);
+        if (x0 != 0.0) atomicAdd(P.pair_out + k0 + q, x0);
+        if (x1 != 0.0) atomicAdd(P.pair_out + k1 + q, x1);
+        if (x2 != 0.0) atomicAdd(P.pair_out + k2 + q, x2);
+        if (x3 != 0.0) atomicAdd(P.pair_out + k3 + q, x3);
     } else if (has) {
-        if (x0 != 0.0) atomicAdd(P.pair_out + 4 * k, x0);
-        if (x1 != 0.0) atomicAdd(P.pair_out + 4 * k + 1, x1);
-        if (x2 != 0.0) atomicAdd(P.pair_out + 4 * k + 2, x2);
-        if (x3 != 0.0) atomicAdd(P.pair_out + 4 * k + 3, x3);
+        if (x0 != 0.0) atomicAdd(P.pair_out + k, x0);
+        if (x1 != 0.0) atomicAdd(P.pair_out + k + 1, x1);
+        if (x2 != 0.0) atomicAdd(P.pair_out + k + 2, x2);
+        if (x3 != 0.0) atomicAdd(P.pair_out + k + 3, x3);
     }
     if (has) A.cnb = -1;
 }
 #endif
 
 template<bool DBG>
-MQI_DI void score(const transport_params& P, const trk& t, uint64_t cnb, float density, float volume, float sp,
-                  uint64_t dij_item, uint64_t scen_off, pending& A, double* pv) {
-    const int     n   = P.n_scorers;
-    const int32_t roi = (int32_t) (uint32_t) cnb;   // roi_t DIRECT
+MQI_DI void score(const transport_params& P, const trk& t, uint32_t cnb, float density, float volume, float sp,
+                  uint32_t dij_item, uint32_t scen, pending& A, double* pv) {
+    const int n = P.n_scorers;
     // regular scorers score through roi_->idx(cnb) > 0, the statistics pair
-    // through get_mask_idx(cnb) >= 0 (mqi_transport.hpp:342-364); a CONTOUR
-    // ROI's answer per voxel is in roi_flags
-    const uint32_t fl      = P.roi_flags ? (uint32_t) P.roi_flags[cnb] : (roi > 0 ? 3u : 2u);
+    // through get_mask_idx(cnb) >= 0 (mqi_transport.hpp:342-364), under
+    // roi_t DIRECT every voxel but 0 and every voxel; a CONTOUR ROI's answer
+    // per voxel is in roi_flags
+    const uint32_t fl      = P.roi_flags ? (uint32_t) P.roi_flags[cnb] : ((int32_t) cnb > 0 ? 3u : 2u);
     const bool     in_reg  = fl & 1u;
     const bool     in_stat = fl & 2u;
-    // Both loops run over the fixed maximum with constant indices so that the
+    const uint64_t k       = P.out_scenario_stride * scen + cnb;
+    const double   d       = dose_hit<DBG>(t, density, volume, sp);
+    // the deposits of a voxel the lane has just entered start from 0
+    const bool fresh = (int32_t) cnb != A.cnb;
+    double     length = 0.0, let = 0.0;
+    bool       has_let = false;
+    if (P.let_kinds) has_let = let_terms(t, density, length, let);
+    double dv = 0.0;   // the Dij scorer's value and repeats when it is not deferred
+    int    dr = 0;
+    // The loop runs over the fixed maximum with constant indices so that the
     // scorer table stays in kernel arguments / registers (a runtime index
     // into it would move the whole argument block to private memory).
-    const double d = dose_hit<DBG>(t, density, volume, sp);
-    double       v[MQI_MAX_SCORERS];
 #pragma unroll
     for (int s = 0; s < MQI_MAX_SCORERS; ++s) {
-        v[s] = 0.0;
-        if (s >= n) continue;
-        const int k = P.kinds[s];
-        if (k == MQI_KIND_LETD_NUM)
-            v[s] = letd_hit(t, density, true);
-        else if (k == MQI_KIND_LETD_DEN)
-            v[s] = letd_hit(t, density, false);
-        else if (k == MQI_KIND_LETT_NUM)
-            v[s] = lett_hit(t, density, true);
-        else if (k == MQI_KIND_LETT_DEN)
-            v[s] = lett_hit(t, density, false);
-        else if (k == MQI_KIND_EDEP)
-            v[s] = edep_hit(t);
-        else if (k == MQI_KIND_DM)
-            v[s] = dm_hit(t, density, volume);
-        else
-            v[s] = (k == MQI_KIND_STAT_DOSE2) ? d * d : d;
-    }
-    if (P.loops == MQI_LOOPS_ONCE) {
-        if ((int64_t) cnb != A.cnb || scen_off != A.off || (uint32_t) dij_item != A.item) {
-            flush(P, A, pv);
-            A.cnb  = (int64_t) cnb;
-            A.off  = scen_off;
-            A.item = (uint32_t) dij_item;
-#pragma unroll
-            for (int s = 0; s < MQI_DEFER; ++s) pv[s * blockDim.x] = 0.0;
+        if (s >= n) break;
+        const int kind = P.kinds[s];
+        double    v    = d;
+        if (kind == MQI_KIND_STAT_DOSE2) {
+            v = d * d;
+        } else if (P.let_kinds && kind != MQI_KIND_DOSE) {
+            if (kind == MQI_KIND_LETD_NUM)
+                v = (!has_let || let >= 25.0) ? 0.0 : t.dE * let;
+            else if (kind == MQI_KIND_LETD_DEN)
+                v = (!has_let || let >= 25.0) ? 0.0 : (double) t.dE;
+            else if (kind == MQI_KIND_LETT_NUM)
+                v = has_let ? length * let : 0.0;
+            else if (kind == MQI_KIND_LETT_DEN)
+                v = has_let ? length : 0.0;
         }
-#pragma unroll
-        for (int s = 0; s < MQI_MAX_SCORERS; ++s) {
-            if (s >= n) continue;
-            const int  k    = P.kinds[s];
-            const bool stat = (k == MQI_KIND_STAT_DOSE || k == MQI_KIND_STAT_DOSE2);
-            if (!(stat ? in_stat : in_reg) || v[s] <= 0) continue;
-            if (s < MQI_DEFER)
-                pv[s * blockDim.x] += v[s];
-            else if (k == MQI_KIND_DIJ)
-                dij_insert(P, dij_item, (uint32_t) cnb, v[s]);
-            else
-                atomicAdd(P.out[s] + scen_off + cnb, v[s]);
+        if (kind == MQI_KIND_EDEP)
+            v = edep_hit(t);
+        else if (kind == MQI_KIND_DM)
+            v = dm_hit(t, density, volume);
+        const bool stat = (kind == MQI_KIND_STAT_DOSE || kind == MQI_KIND_STAT_DOSE2);
+        if (P.loops == MQI_LOOPS_ONCE && s < MQI_DEFER) {
+            double*      acc = pv + s * blockDim.x;
+            const double o   = fresh ? 0.0 : *acc;
+            *acc             = (!(stat ? in_stat : in_reg) || v <= 0) ? o : o + v;
+            continue;
         }
-        return;
-    }
-#pragma unroll
-    for (int s = 0; s < MQI_MAX_SCORERS; ++s) {
-        if (s >= n) continue;
-        const int  k    = P.kinds[s];
-        const bool stat = (k == MQI_KIND_STAT_DOSE || k == MQI_KIND_STAT_DOSE2);
-        int        reps = 0;
+        int reps = 0;
         if (P.loops == MQI_LOOPS_ONCE) {
             reps = (stat ? in_stat : in_reg) ? 1 : 0;
         } else if (P.loops == MQI_LOOPS_PLAIN) {
@@ -903,12 +917,20 @@ MQI_DI void score(const transport_params& P, const trk& t, uint64_t cnb, float d
             else if (n >= 2)
                 reps = in_stat ? 1 : 0;
         }
-        if (v[s] <= 0) continue;
-        if (k == MQI_KIND_DIJ) {
-            for (int r = 0; r < reps; ++r) dij_insert(P, dij_item, (uint32_t) cnb, v[s]);
+        if (v <= 0) continue;
+        if (kind == MQI_KIND_DIJ) {
+            dv = v;
+            dr = reps;
             continue;
         }
-        for (int r = 0; r < reps; ++r) atomicAdd(P.out[s] + scen_off + cnb, v[s]);
+        for (int r = 0; r < reps; ++r) atomicAdd(P.out[s] + k, v);
+    }
+    // one insert site for every slot and loop
+    for (int r = 0; r < dr; ++r) dij_insert(P, dij_item, cnb, dv);
+    if (P.loops == MQI_LOOPS_ONCE) {
+        A.cnb  = (int32_t) cnb;
+        A.scen = scen;
+        A.item = dij_item;
     }
 }
 
@@ -921,10 +943,11 @@ struct lane {
     uint64_t g;          // history index in the flattened list
     int      nsteps;     // trace mode: steps logged for this history
     float    scale;      // scenario density scale
-    uint64_t scen_off;   // scenario offset into the output arrays
-    uint64_t dij_item;   // Dij table of (scenario, spot): scenario * n_spots + spot
+    uint32_t scen;       // scenario
+    uint32_t dij_item;   // Dij table of (scenario, spot): scenario * n_spots + spot
     int      tsteps;     // steps of the current track
     pending  acc;        // deferred deposits of the current voxel
+    bool     newhist;    // the first step of a history: the pending deposits are another one's
     bool     reenter;    // left a beamline child: enter the next child
 };
 
@@ -1159,8 +1182,9 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
         // step: one counter tracks loads, stores and atomics alike, so atomics
         // issued just before the next wait on a load would add their round
         // trip to every step.
-        const bool leave = P.loops == MQI_LOOPS_ONCE && ((int64_t) cnb != L.acc.cnb || L.scen_off != L.acc.off ||
-                                                         (uint32_t) L.dij_item != L.acc.item);
+        // (A history's deposits are its own scenario's and Dij table's.)
+        const bool leave = P.loops == MQI_LOOPS_ONCE && ((int32_t) cnb != L.acc.cnb || L.newhist);
+        L.newhist        = false;
 #if !MQI_EXACT
         if (P.pair == 2)
             flush_pair(P, L.acc, pv, leave);
@@ -1210,7 +1234,7 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
         float     vol = c.g.X(i + 1) - c.g.X(i);
         vol *= c.g.Y(j + 1) - c.g.Y(j);
         vol *= c.g.Z(k + 1) - c.g.Z(k);
-        score<DBG>(P, t, cnb, rho, vol, sp, L.dij_item, L.scen_off, L.acc, pv);
+        score<DBG>(P, t, (uint32_t) cnb, rho, vol, sp, L.dij_item, L.scen, L.acc, pv);
     }
     if (!t.stopped) {
         step_axis(t.p1.x, t.d1.x, c.g.xe, c.g.sx, t.cx);
@@ -1281,6 +1305,8 @@ k_transport(transport_params P) {
     // the lane's pending deposit sums (MQI_DEFER doubles, blockDim.x apart),
     // after the beamline edges at an 8-byte boundary
     double* pv = reinterpret_cast<double*>(sh + mqi_pend_offset(P.nx, P.ny, P.nz, P.bl_n_edges)) + threadIdx.x;
+#pragma unroll
+    for (int s = 0; s < MQI_DEFER; ++s) pv[s * blockDim.x] = 0.0;
     const uint64_t tid      = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t nthreads = (uint64_t) gridDim.x * blockDim.x;
     c.stack                 = P.stack + tid * (uint64_t) P.stack_cap * MQI_STACK_FLOATS;
@@ -1299,14 +1325,15 @@ k_transport(transport_params P) {
     L.hist   = 0;
     L.nsteps   = 0;
     L.scale    = 1.0f;
-    L.scen_off = 0;
+    L.scen     = 0;
     L.dij_item = 0;
     L.acc.cnb  = -1;
-    L.acc.off  = 0;
+    L.acc.scen = 0;
     L.acc.item = 0;
+    L.newhist  = false;
     L.reenter  = false;
     c.g.sx = c.g.sy = c.g.sz = 0.0f;
-    unsigned long long done = 0, nstep = 0;
+    uint32_t           done = 0, nstep = 0;
     uint32_t           scen = 0;
     const uint64_t     hoff = P.hist_offset ? *P.hist_offset : 0;
     int                qx   = 0;   // work range this wave fetches from (dynamic form)
@@ -1388,8 +1415,9 @@ k_transport(transport_params P) {
             c.g.sy                 = P.scen_shift ? P.scen_shift[3 * scen + 1] : 0.0f;
             c.g.sz                 = P.scen_shift ? P.scen_shift[3 * scen + 2] : 0.0f;
             L.scale                = P.scen_scale ? P.scen_scale[scen] : 1.0f;
-            L.scen_off             = (uint64_t) scen * P.out_scenario_stride;
-            L.dij_item             = (uint64_t) scen * P.n_spots + spot_id;
+            L.scen                 = scen;
+            L.dij_item             = scen * (uint32_t) P.n_spots + spot_id;
+            L.newhist              = true;
             if (P.vertices) {
                 const float* v = P.vertices + 7 * g;
                 L.t.ke0        = v[0];
@@ -1428,8 +1456,8 @@ k_transport(transport_params P) {
         ++nstep;
     }
     flush(P, L.acc, pv);
-    atomicAdd(P.tracked, done);
-    atomicAdd(P.steps, nstep);
+    atomicAdd(P.tracked, (unsigned long long) done);
+    atomicAdd(P.steps, (unsigned long long) nstep);
     if (c.drops) atomicAdd(P.drops, (unsigned long long) c.drops);
 }
 

@@ -103,3 +103,30 @@ def test_production_vacuum_traversal_equals_the_oracle(ctx, shape, dx, dz):
     ctx.set_scorers(rb.SC_DOSE)
     cnb, rec, nst = ctx.trace(ctx.config(seed=5, exact=False, batched=False), len(rays), 400, vertices=rays)
     _assert_trace_equal(cnb, rec, nst, ref)
+
+
+@pytest.mark.parametrize("histories", [1, 3, 63, 65, 1025])
+@pytest.mark.parametrize("mask", [1, 4, 5, 2, 3, 18, 19, 16 + 32, 32 + 64])
+def test_grouped_flush_equals_the_plain_launch(ctx, histories, mask):
+    """Every number of grouped scorers (1, the pair, three and four, and five
+    with one beyond the deferred slots) at history counts around a group, a
+    wave and a workgroup: a batched pass adds the same deposits as one launch
+    per spot (the sums differ in FP64 order only)."""
+    import phantoms
+    g = phantoms.slab_box(9, 11, 90)
+    sp = phantoms.spots([90.0, 60.0], histories, sigma=3.0, sigma_e_frac=0.01, positions=[(0, 0, 0.5), (2, -1, 0.5)])
+    ctx.set_grid(g.xe, g.ye, g.ze, g.density)
+    ctx.set_scenarios([[0, 0, 0], [1, 0, 0]], [1.0, 0.9])
+    ctx.set_spots(sp)
+    for per_scenario in (False, True):
+        ctx.set_scorers(mask, per_scenario)
+        out = []
+        for batched in (True, False):
+            ctx.zero_scorers()
+            r = ctx.run(ctx.config(seed=3, batched=batched))
+            assert r.histories == 4 * histories
+            out.append([ctx.scorer(k, s) for k in range(ctx.scorer_count()) for s in range(2 if per_scenario else 1)])
+        for a, b in zip(*out):
+            assert b.sum() > 0
+            assert np.allclose(a, b, rtol=1e-12, atol=0)
+    ctx.set_scenarios()
