@@ -508,32 +508,129 @@ MQI_DI void rotate_direction(v3& d, float theta, float phi) {
 
 // ------------------------------------------------------------------ random numbers
 // The verification build draws every number from one lazily refilled stream
-// in the order the CPU restatement does.  The production build draws the four
-// numbers every step takes (mean free path, straggling and scattering
-// normals, azimuth) from one Philox block made for all lanes at the start of
-// the step, and the first three of an interaction (process, first delta-ray
-// trial) from one block made where the step ends in an interaction; the lazy
-// stream serves the rest (later delta-ray trials, nuclear interactions).
-// With the lazy stream alone, every draw site refilled for some lane of the
-// wave (8.3 block evaluations per wave step on the 2000-spot CT plan).
+// in the order the CPU restatement does.  The production build takes whole
+// Philox blocks, no word of which is kept between uses: one per step (mean
+// free path, straggling and scattering normals, azimuth), one per
+// interaction (process, first delta-ray trial) and, for later delta-ray
+// trials and the nuclear interactions, which draw in pairs, half a block per
+// pair.  (With a lazily refilled stream every draw site refilled for some
+// lane of the wave, 8.3 blocks per wave step on the 2000-spot CT plan, and
+// four unread words and their count stayed in registers.)
+#if MQI_EXACT
 struct rng_t {
     mqi_rng::stream s;
-#if !MQI_EXACT
-    uint32_t step_blk, int_blk;   // blocks of the two per-step streams used so far
-    float    st_u0, st_u1, st_z0, st_z1;   // the step's two uniforms and two normals
-    float    it_u0, it_u1, it_u2;          // the interaction's three uniforms
-#endif
-    MQI_DI void init(uint64_t seed, uint32_t history, uint32_t spot, uint32_t scenario, uint32_t purpose) {
-        s.init(seed, history, spot, scenario, purpose);
-#if !MQI_EXACT
-        step_blk = 0;
-        int_blk  = 0;
-#endif
+    MQI_DI void init(uint64_t seed, uint32_t history, uint32_t spot, uint32_t scenario) {
+        s.init(seed, history, spot, scenario, mqi_rng::STREAM_TRANSPORT);
     }
     MQI_DI float uniform() { return s.uniform(); }
-    // standard normal: the exact build evaluates Box-Muller as the CPU
-    // restatement does; the production build in float with the device library
-    MQI_DI float gauss() {
+    MQI_DI void  pair(float& a, float& b) {
+        a = s.uniform();
+        b = s.uniform();
+    }
+    MQI_DI float normal(float avg, float sig) {
+        float z = (float) s.gauss();
+        return z * sig + avg;
+    }
+};
+#else
+struct rng_t {
+    uint32_t key0, key1;                  // the seed: the same in every lane
+    uint32_t c1, c2, c3;                  // words 0 and 1 behind the first round (history and spot), scenario
+    uint32_t step_blk, int_blk, pairs;    // blocks and half blocks used
+    float    st_u0, st_u1, st_z0, st_z1;  // the step's two uniforms and two normals
+    float    it_u0, it_u1, it_u2;         // the interaction's three uniforms
+
+    // the seed is set once per launch, outside the history loop, so that the
+    // key schedule stays in scalar registers
+    MQI_DI void set_seed(uint64_t seed) {
+        key0 = (uint32_t) seed;
+        key1 = (uint32_t) (seed >> 32);
+    }
+    MQI_DI void init(uint32_t history, uint32_t spot, uint32_t scenario) {
+        uint32_t hi, lo;
+        mqi_rng::mulhilo32(0xCD9E8D57u, spot, &hi, &lo);
+        c1       = hi ^ history ^ key0;
+        c2       = lo;
+        c3       = scenario << 8;
+        step_blk = int_blk = pairs = 0;
+    }
+    static MQI_DI uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+        return (uint32_t) __builtin_amdgcn_bitop3_b32((int) a, (int) b, (int) c, 0x96);
+    }
+    // philox4x32_10 of {blk, history, spot, c3 | purpose}: round 0's products
+    // of the spot were formed at the history's start, three-way exclusive ors
+    // in one instruction, the key schedule formed anew (hoisted out of the
+    // history loop its 18 words would not fit the scalar registers)
+    MQI_DI mqi_rng::u32x4 block_of(uint32_t purpose, uint32_t blk) const {
+        const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
+        uint32_t       k0 = key0, k1 = key1;
+        asm volatile("" : "+s"(k0), "+s"(k1));
+        mqi_rng::u32x4 c;
+        uint32_t       hi, lo;
+        mqi_rng::mulhilo32(M0, blk, &hi, &lo);
+        c.v[0] = c1;
+        c.v[1] = c2;
+        c.v[2] = xor3(hi, c3 | purpose, k1);
+        c.v[3] = lo;
+#pragma unroll
+        for (int r = 1; r < 10; ++r) {
+            k0 += 0x9E3779B9u;
+            k1 += 0xBB67AE85u;
+            uint32_t hi0, lo0, hi1, lo1;
+            mqi_rng::mulhilo32(M0, c.v[0], &hi0, &lo0);
+            mqi_rng::mulhilo32(M1, c.v[2], &hi1, &lo1);
+            const uint32_t n0 = xor3(hi1, c.v[1], k0), n2 = xor3(hi0, c.v[3], k1);
+            c.v[0] = n0;
+            c.v[1] = lo1;
+            c.v[2] = n2;
+            c.v[3] = lo0;
+        }
+        return c;
+    }
+    // stream::to_uniform: (w >> 8) * 2^-24 + 2^-24, exact
+    static MQI_DI float to_uniform(uint32_t w) {
+        return __builtin_fmaf((float) (w >> 8), 0x1p-24f, 0x1p-24f);
+    }
+    // the draws of a step: st_u0 the mean free path, st_z0 the energy
+    // straggling, st_z1 the scattering angle, st_u1 the azimuth
+    MQI_DI void begin_step() {
+        const mqi_rng::u32x4 w = block_of(mqi_rng::STREAM_STEP, step_blk++);
+        st_u0                  = to_uniform(w.v[0]);
+        st_u1                  = to_uniform(w.v[3]);
+        // Box-Muller on the hardware log2, square root, sine and cosine (the
+        // last two take revolutions: sin(2 pi u))
+        const float u1 = to_uniform(w.v[1]);
+        const float u2 = to_uniform(w.v[2]);
+        const float r  = __builtin_amdgcn_sqrtf(-2.0f * 0.693147180559945309f * __builtin_amdgcn_logf(u1));
+        st_z0          = r * __builtin_amdgcn_cosf(u2);
+        st_z1          = r * __builtin_amdgcn_sinf(u2);
+    }
+    // the draws of an interaction: it_u0 the process, it_u1 and it_u2 the
+    // first delta-ray trial
+    MQI_DI void begin_interaction() {
+        const mqi_rng::u32x4 w = block_of(mqi_rng::STREAM_INTERACTION, int_blk++);
+        it_u0                  = to_uniform(w.v[0]);
+        it_u1                  = to_uniform(w.v[1]);
+        it_u2                  = to_uniform(w.v[2]);
+    }
+    // the next two numbers of the history's transport stream
+    MQI_DI void pair(float& a, float& b) {
+        const mqi_rng::u32x4 w = block_of(mqi_rng::STREAM_TRANSPORT, pairs >> 1);
+        const bool           h = pairs & 1u;
+        a                      = to_uniform(h ? w.v[2] : w.v[0]);
+        b                      = to_uniform(h ? w.v[3] : w.v[1]);
+        ++pairs;
+    }
+};
+#endif
+
+// The vertex's stream.  Standard normals: the verification build evaluates
+// Box-Muller as the CPU restatement does; the production build in float with
+// the device library.
+struct vertex_rng {
+    mqi_rng::stream s;
+    MQI_DI float    uniform() { return s.uniform(); }
+    MQI_DI float    gauss() {
 #if MQI_EXACT
         return (float) s.gauss();
 #else
@@ -549,63 +646,6 @@ struct rng_t {
         s.spare     = r * sn;
         s.has_spare = 1;
         return r * cs;
-#endif
-    }
-    MQI_DI float normal(float avg, float sig) {
-        float z = gauss();
-        return z * sig + avg;
-    }
-
-    // the draws of a step: step_uniform(0) the mean free path, step_normal(0)
-    // the energy straggling, step_normal(1) the scattering angle,
-    // step_uniform(1) the azimuth, in that order
-    MQI_DI void begin_step() {
-#if !MQI_EXACT
-        const mqi_rng::u32x4 w = s.block_of(mqi_rng::STREAM_STEP, step_blk++);
-        st_u0                  = mqi_rng::stream::to_uniform(w.v[0]);
-        st_u1                  = mqi_rng::stream::to_uniform(w.v[3]);
-        // Box-Muller on the hardware log2, square root, sine and cosine (the
-        // last two take revolutions: sin(2 pi u))
-        const float u1 = mqi_rng::stream::to_uniform(w.v[1]);
-        const float u2 = mqi_rng::stream::to_uniform(w.v[2]);
-        const float r  = __builtin_amdgcn_sqrtf(-2.0f * 0.693147180559945309f * __builtin_amdgcn_logf(u1));
-        st_z0          = r * __builtin_amdgcn_cosf(u2);
-        st_z1          = r * __builtin_amdgcn_sinf(u2);
-#endif
-    }
-    MQI_DI float step_uniform(int k) {
-#if MQI_EXACT
-        (void) k;
-        return uniform();
-#else
-        return k == 0 ? st_u0 : st_u1;
-#endif
-    }
-    MQI_DI float step_normal(int k, float avg, float sig) {
-#if MQI_EXACT
-        (void) k;
-        return normal(avg, sig);
-#else
-        return (k == 0 ? st_z0 : st_z1) * sig + avg;
-#endif
-    }
-    // the draws of an interaction: int_uniform(0) the process,
-    // int_uniform(1) and (2) the first delta-ray trial; later trials and the
-    // nuclear interactions draw uniform()
-    MQI_DI void begin_interaction() {
-#if !MQI_EXACT
-        const mqi_rng::u32x4 w = s.block_of(mqi_rng::STREAM_INTERACTION, int_blk++);
-        it_u0                  = mqi_rng::stream::to_uniform(w.v[0]);
-        it_u1                  = mqi_rng::stream::to_uniform(w.v[1]);
-        it_u2                  = mqi_rng::stream::to_uniform(w.v[2]);
-#endif
-    }
-    MQI_DI float int_uniform(int k) {
-#if MQI_EXACT
-        (void) k;
-        return uniform();
-#else
-        return k == 0 ? it_u0 : (k == 1 ? it_u1 : it_u2);
 #endif
     }
 };

@@ -123,7 +123,7 @@ MQI_DI float energy_loss(ctx& c, const rel_q& rel, float rho, float step_length,
     float Te      = (rel.Te_max >= 0.08511) ? 0.08511 : rel.Te_max;
     float O_sq    = units::two_pi_re2_mc2_h2o * rho / units::water_density * L_w;
     O_sq *= Te / rel.beta_sq * (1.0 - 0.5 * rel.beta_sq);
-    float ret = c.rng.step_normal(0, dE_mean, MQ_SQRTF(O_sq));
+    float ret = c.rng.normal(dE_mean, MQ_SQRTF(O_sq));
     if (ret < 0) ret *= -1.0;
     return ret;
 }
@@ -142,9 +142,9 @@ MQI_DI void along_step(ctx& c, trk& t, float len, float rho, float sp) {
     float X0    = radiation_length<DBG>(rho);
     float th_sq = ((13.9f / P) * (13.9f / P) / rel.beta_sq) * len / X0;
     float th    = MQ_SQRTF(th_sq);
-    th          = c.rng.step_normal(1, 0, MQ_SQRTF(2.0f) * th);
+    th          = c.rng.normal(0, MQ_SQRTF(2.0f) * th);
     if (th < 0) th *= -1.0;
-    float phi = 2.0 * 3.14159265358979323846 * c.rng.step_uniform(1);
+    float phi = 2.0 * 3.14159265358979323846 * c.rng.uniform();
     rotate_direction(t.d1, th, phi);
     t.dE += dE * r;
     update_pos(t, r * len);
@@ -318,10 +318,10 @@ MQI_DI void post_ion(ctx& c, trk& t) {
     // acceptance probability is above 1/2 for any finite energy; the bound
     // only ends the loop for non-finite input (which the reference would spin on)
     for (int it = 0; it < 4096; ++it) {
-        n  = it == 0 ? c.rng.int_uniform(1) : c.rng.uniform();
+        n  = c.rng.uniform();
         Te = T_cut * rel.Te_max;
         Te /= ((1.0 - n) * rel.Te_max + n * T_cut);
-        const float acc = it == 0 ? c.rng.int_uniform(2) : c.rng.uniform();
+        const float acc = c.rng.uniform();
         if (acc < 1.0 - rel.beta_sq * Te / rel.Te_max + Te * Te / (2.0 * rel.Et_sq)) break;
     }
     if (DBG) {
@@ -353,8 +353,7 @@ MQI_DI void post_ion(ctx& c, trk& t) {
         Te               = (float) d_quot(num, den, d_recip(den));
         const double a   = 1.0 - (double) (rel.beta_sq * Te * rte);
         if ((double) acc < a + d_quot((double) (Te * Te), e2, re2) || it == 4095) break;
-        n   = c.rng.uniform();
-        acc = c.rng.uniform();
+        c.rng.pair(n, acc);
     }
     if (DBG) {
         push_placed(c, 0.0f, t.p0, t.d0, 0.0f, Te);
@@ -369,7 +368,9 @@ MQI_DI void post_ion(ctx& c, trk& t) {
 MQI_DI void post_pp(ctx& c, trk& t) {
     rel_q rel       = relq(t.ke1);
     float min_value = 0.5f / rel.Ek;
-    float u         = c.rng.uniform() * (1.0 - 2.0 * min_value) + min_value;
+    float r0, r1;
+    c.rng.pair(r0, r1);
+    float u         = r0 * (1.0 - 2.0 * min_value) + min_value;
     float E1        = rel.Et;
     float dE        = rel.Ek * u;
     float E3        = (rel.Ek - dE) + units::Mp;
@@ -391,7 +392,7 @@ MQI_DI void post_pp(ctx& c, trk& t) {
         cos_th34 = -1.0;
     float th3 = MQ_ACOSF(cos_th3);
     float th4 = th3 - MQ_ACOSF(cos_th34);
-    float phi = 2.0 * 3.14159265358979323846 * c.rng.uniform();
+    float phi = 2.0 * 3.14159265358979323846 * r1;
     t.ke1 -= dE;
     rotate_direction(t.d1, th3, phi);
     v3 dd = t.d1;
@@ -418,7 +419,8 @@ MQI_DI void post_poe(ctx& c, trk& t) {
         Tp_max /= (1.0 + 2.0 * rel.gamma * units::MoMp + units::MoMp_sq);
         (void) Tp_max;
         float avg     = (float) (1.0 / Tp_avg);
-        float uu      = c.rng.uniform();
+        float uu, u1;
+        c.rng.pair(uu, u1);
         float dE      = -MQ_LOGF(uu) / avg;
         float E1      = rel.Ek * (rel.Ek + 2.0 * units::Mp);
         float E3      = (rel.Ek - dE) * (rel.Ek - dE + 2.0 * units::Mp);
@@ -426,7 +428,7 @@ MQI_DI void post_poe(ctx& c, trk& t) {
         if (cos_th3 > 1.0) cos_th3 = 1.0;
         if (cos_th3 < -1.0) cos_th3 = -1.0;
         float th3 = MQ_ACOSF(cos_th3);
-        float phi = 2.0 * 3.14159265358979323846 * c.rng.uniform();
+        float phi = 2.0 * 3.14159265358979323846 * u1;
         if (DBG)
             push_placed(c, dE, t.p0, t.d0, 0.0f, dE);
         else
@@ -463,18 +465,20 @@ MQI_DI void post_poi(ctx& c, trk& t) {
     }
     while ((Er - Eb) > E_mini) {
         Er -= Eb;
-        float u  = c.rng.uniform();
+        float u, zeta;
+        c.rng.pair(u, zeta);
         float dE = MQ_POWF(u, power) * (Er - E_mini) + E_mini;
         if (dE >= Er) dE = Er;
         Er -= dE;
         t.ke1 -= dE + Eb;
-        float zeta = c.rng.uniform();
         if (zeta < Prob_2nd) {
-            float cos_th = (2.0 * dE / Ek - 1.0) + 2.0 * (1 - dE / Ek) * c.rng.uniform();
+            float r0, r1;
+            c.rng.pair(r0, r1);
+            float cos_th = (2.0 * dE / Ek - 1.0) + 2.0 * (1 - dE / Ek) * r0;
             if (cos_th < -1) cos_th = -1;
             if (cos_th > 1) cos_th = 1;
             float th  = MQ_ACOSF(cos_th);
-            float phi = 2.0 * 3.14159265358979323846 * c.rng.uniform();
+            float phi = 2.0 * 3.14159265358979323846 * r1;
             v3    dd  = t.d1;
             rotate_direction(dd, th, phi);
             push_placed(c, dE, t.p1, dd, dE, 0.0f);
@@ -538,8 +542,7 @@ MQI_DI void stepping(ctx& c, trk& t, float rho, float d2b, float& sp) {
     float cs_sum  = first ? cs1_sum : cs2_sum;
     float cs0 = first ? cs1[0] : cs2[0], csa = first ? cs1[1] : cs2[1], csb = first ? cs1[2] : cs2[2],
           csc = first ? cs1[3] : cs2[3];
-    c.rng.begin_step();
-    float prob       = c.rng.step_uniform(0);
+    float prob       = c.rng.uniform();
     float mfp        = -1.0f * MQ_LOGF(prob) / cs_sum;
     float step_limit = cms * units::water_density / (sp * rho);
     int   br;
@@ -558,8 +561,7 @@ MQI_DI void stepping(ctx& c, trk& t, float rho, float d2b, float& sp) {
     along_step<DBG>(c, t, len, rho, sp);
     if (br != 1) return;
     if (t.ke1 <= 0.5f) return;
-    c.rng.begin_interaction();
-    float u = cs_sum * c.rng.int_uniform(0);
+    float u = cs_sum * c.rng.uniform();
     t.d1    = t.d0;
     if (u < cs0) {
         post_ion<DBG>(c, t);
@@ -1073,7 +1075,7 @@ MQI_DI void pop(ctx& c, trk& t) {
 // beamlet, then rotation/translation (mqi_beamlet.hpp:81-90, mqi_phsp6d.hpp:62-79).
 MQI_DI void sample_vertex(const transport_params& P, const mqi_spot& sp, uint32_t spot_id, uint32_t scenario,
                           uint64_t h, trk& t) {
-    rng_t r;
+    vertex_rng r;
     r.s.init(P.seed, (uint32_t) h, spot_id, scenario, mqi_rng::STREAM_VERTEX);
     float Ux, Vx, Uy, Vy, Uz;
     if (sp.phsp == MQI_PHSP_UNIFORM) {   // U(-1, 1) draws (phsp_6d_uniform)
@@ -1301,6 +1303,9 @@ k_transport(transport_params P) {
     c.child = 0;
     c.nbl   = P.n_bl;
     c.blxf  = P.bl_xf;
+#if !MQI_EXACT
+    c.rng.set_seed(P.seed);
+#endif
     const float* shb = c.g.ze + P.nz + 1;   // beamline edges in LDS
     // the lane's pending deposit sums (MQI_DEFER doubles, blockDim.x apart),
     // after the beamline edges at an 8-byte boundary
@@ -1433,7 +1438,11 @@ k_transport(transport_params P) {
             } else {
                 sample_vertex(P, P.spots[spot_id], spot_id, scen, L.hist + hoff, L.t);
             }
-            c.rng.init(P.seed, (uint32_t) (L.hist + hoff), spot_id, scen, mqi_rng::STREAM_TRANSPORT);
+#if MQI_EXACT
+            c.rng.init(P.seed, (uint32_t) (L.hist + hoff), spot_id, scen);
+#else
+            c.rng.init((uint32_t) (L.hist + hoff), spot_id, scen);
+#endif
             L.nsteps = 0;
             L.tsteps = 0;
             ++done;

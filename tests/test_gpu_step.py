@@ -127,6 +127,6 @@ def test_grouped_flush_equals_the_plain_launch(ctx, histories, mask):
             assert r.histories == 4 * histories
             out.append([ctx.scorer(k, s) for k in range(ctx.scorer_count()) for s in range(2 if per_scenario else 1)])
         for a, b in zip(*out):
-            assert b.sum() > 0
+            assert histories == 1 or b.sum() > 0   # a single proton may pass beside the box
             assert np.allclose(a, b, rtol=1e-12, atol=0)
     ctx.set_scenarios()
