@@ -609,13 +609,6 @@ fill_params(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg) {
         P.dij_vals     = c->d_dij_vals;
         P.dij_off      = c->d_dij_off;
     }
-    P.dij_slot = -1;
-    for (int k = 0; k < P.n_scorers; ++k) {
-        const int kd = P.kinds[k];
-        if (kd == MQI_KIND_DIJ) P.dij_slot = k;
-        if (kd == MQI_KIND_LETD_NUM || kd == MQI_KIND_LETD_DEN || kd == MQI_KIND_LETT_NUM || kd == MQI_KIND_LETT_DEN)
-            P.let_kinds = 1;
-    }
     P.out_scenario_stride = c->per_scen ? nvox(c) : 0;
     P.loops               = cfg.scoring_loops;
     P.stack               = c->d_stack;
@@ -633,6 +626,21 @@ bind_buffers(mqi_ctx* c, transport_params& P) {
     P.stack         = c->d_stack;
 }
 
+// the scorer words the kernels read, from the scorers and groups P names
+void
+pack_scoring(transport_params& P) {
+    int let = 0, dij = -1;
+    P.kind_word = 0;
+    for (int k = 0; k < P.n_scorers; ++k) {
+        const int kd = P.kinds[k];
+        P.kind_word |= (uint32_t) kd << 4 * k;
+        if (kd == MQI_KIND_DIJ) dij = k;
+        if (kd == MQI_KIND_LETD_NUM || kd == MQI_KIND_LETD_DEN || kd == MQI_KIND_LETT_NUM || kd == MQI_KIND_LETT_DEN)
+            let = 1;
+    }
+    P.mode_word = mqi_mode(P.n_scorers, let, P.loops, P.pair, P.group_ns, dij);
+}
+
 // A launch over the buffers P already names (work list, queue, counters,
 // stacks); stack_bytes is the size of the array P.stack points into.
 int
@@ -647,6 +655,7 @@ launch_bound(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int dyn
     if (trace && (!P.trace_cnb || !P.trace_rec || !P.trace_n)) return (int) hipErrorInvalidValue;
     if ((uint64_t) blocks * threads * (uint64_t) P.stack_cap * MQI_STACK_FLOATS * sizeof(float) > stack_bytes)
         return (int) hipErrorInvalidValue;
+    pack_scoring(P);
     const size_t sh = shmem_bytes(c, threads);
     if (dynamic) {
         const int e = mqi_aux::queue_init(P.queue, P.total, c->stream);
@@ -752,6 +761,7 @@ upload_plan(mqi_ctx* c, const run_plan& p) {
 int
 graph_pass(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int blocks, int threads, double* ms) {
     bind_buffers(c, P);
+    pack_scoring(P);
     const int variant[6] = {cfg.physics_debug, cfg.exact, cfg.exact ? 0 : cfg.waves_per_simd, blocks, threads,
                             (int) shmem_bytes(c, threads)};
     std::vector<unsigned char> key(sizeof P + sizeof variant);

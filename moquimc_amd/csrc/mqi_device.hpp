@@ -128,8 +128,8 @@ MQI_DI void normalize(v3& a) {
     a.y     = geo_div(a.y, n);
     a.z     = geo_div(a.z, n);
 }
-// the same in the physics (scattering rotations): hardware division and
-// square root in the production build
+#if MQI_EXACT
+// the same in the physics (scattering rotations; production: q_normalize)
 MQI_DI void normalize_fast(v3& a) {
     MQI_NO_CONTRACT
     float n = MQ_SQRTF(a.x * a.x + a.y * a.y + a.z * a.z);
@@ -137,7 +137,9 @@ MQI_DI void normalize_fast(v3& a) {
     a.y /= n;
     a.z /= n;
 }
+#endif
 
+#if MQI_EXACT   // the production build's are in mqi_prod.hpp
 // relativistic_quantities (mqi_relativistic_quantities.hpp:24-43)
 struct rel_q {
     float beta_sq, gamma_sq, gamma, Et, Et_sq, Ek, Te_max;
@@ -153,29 +155,15 @@ MQI_DI rel_q relq(float Ek) {
     const float   MeMp_sq = MeMp * MeMp;
     r.gamma               = r.Et / Mp;
     r.gamma_sq            = r.gamma * r.gamma;
-#if MQI_EXACT
     r.beta_sq = 1.0 - 1.0 / r.gamma_sq;
     r.Te_max  = (2.0 * Me * r.beta_sq * r.gamma_sq);
     r.Te_max /= (1.0 + 2.0 * r.gamma * MeMp + MeMp_sq);
-#else
-    // production: float, and beta^2 = Ek (Ek + 2 Mp) / Et^2, the same
-    // quantity without the cancellation of 1 - 1 / gamma^2 at low energy
-    r.beta_sq = Ek * (Ek + 2.0f * Mp) / r.Et_sq;
-    r.Te_max  = (2.0f * Me * r.beta_sq * r.gamma_sq) / (1.0f + 2.0f * r.gamma * MeMp + MeMp_sq);
-#endif
     return r;
 }
 MQI_DI float momentum(const rel_q& r) {
-#if MQI_EXACT
     return MQ_SQRTF(r.Et * r.Et - units::Mp * units::Mp);
-#else
-    // production: p^2 = Ek (Ek + 2 Mp), the same quantity without the
-    // cancellation of Et^2 - Mp^2 in float at low energy
-    return MQ_SQRTF(r.Ek * (r.Ek + 2.0f * units::Mp));
-#endif
 }
 
-#if MQI_EXACT   // the production build's are in mqi_prod.hpp
 MQI_DI float intpl(float x, float x0, float x1, float y0, float y1) {
     return (x1 == x0) ? y0 : y0 + (x - x0) * (y1 - y0) / (x1 - x0);
 }
@@ -398,17 +386,19 @@ MQI_DI float intersect_out(const grid_view& g, v3 p, v3& d, int& cx, int& cy, in
     return dist;
 }
 
-// index(vtx1, dir1, idx): +-1 cell update (mqi_grid3d.hpp:847-877)
-MQI_DI void step_axis(float v, float dir, const float* e, float sh, int& i) {
+// index(vtx1, dir1, idx): the +-1 cell update (mqi_grid3d.hpp:847-877) of a
+// position v in a cell [e0, e1]: -1 when dir < 0 and v is below e0 or within
+// the tolerance of it, +1 when dir > 0 and v is above e1 or within it.  Both
+// directions in one expression: v above the edge ahead or less than the
+// tolerance short of it is (v - e) sign(dir) > -tol (the float difference has
+// the sign of the comparison).
+MQI_DI int step_cell(float v, float dir, float e0, float e1) {
     MQI_NO_CONTRACT
     const float tol = 1e-3f;
-    if (dir < 0) {
-        const float e0 = e[i] + sh;
-        if (fabsf(v - e0) < tol || v < e0) i -= 1;
-    } else if (dir > 0) {
-        const float e1 = e[i + 1] + sh;
-        if (fabsf(v - e1) < tol || v > e1) i += 1;
-    }
+    const bool  up  = dir > 0;
+    const float a   = v - (up ? e1 : e0);
+    const bool  hit = (up ? a : -a) > -tol && dir != 0;
+    return hit ? (up ? 1 : -1) : 0;
 }
 
 // ------------------------------------------------------------------ track
@@ -435,6 +425,7 @@ MQI_DI void move(trk& t) {   // mqi_track.hpp:193-197
     t.ldE = 0;
 }
 
+#if MQI_EXACT   // production: q_align / q_turn (mqi_prod.hpp)
 // rotate_y / rotate_z on a matrix held as 9 floats (mqi_matrix.hpp:231-273)
 MQI_DI void rotate_y(float* m, float a) {
     float c1 = MQ_COSF(a), s1 = MQ_SINF(a);
@@ -505,6 +496,7 @@ MQI_DI void rotate_direction(v3& d, float theta, float phi) {
     d = mv(g, dl);
     normalize_fast(d);
 }
+#endif
 
 // ------------------------------------------------------------------ random numbers
 // The verification build draws every number from one lazily refilled stream

@@ -53,6 +53,8 @@ __host__ __device__ inline size_t mqi_shmem_bytes(int nx, int ny, int nz, int bl
 #define MQI_STATUS_TRACK_CAP 2u
 #define MQI_MAX_TRACK_STEPS 200000
 
+#define MQI_KDI __host__ __device__ inline
+
 // Work ranges of the dynamic form: one per XCD of the MI355X, counters a
 // 128-byte line apart.
 #define MQI_QUEUES 8
@@ -62,6 +64,14 @@ __host__ __device__ inline size_t mqi_shmem_bytes(int nx, int ny, int nz, int bl
 __host__ __device__ inline uint64_t mqi_range_begin(uint64_t total, int q) {
     const uint64_t base = total / MQI_QUEUES, rem = total % MQI_QUEUES;
     return base * (uint64_t) q + ((uint64_t) q < rem ? (uint64_t) q : rem);
+}
+
+// The scoring of a launch in one word: scorers (3 bits), a flag for any LETd
+// or LETt scorer, loops (2 bits), lanes per scoring group (0, 2 or 4; 3
+// bits), grouped scorers (3 bits), the Dij scorer's slot + 1 (4 bits).
+MQI_KDI uint32_t mqi_mode(int n, int let, int loops, int pair, int group_ns, int dij_slot) {
+    return (uint32_t) n | (uint32_t) let << 3 | (uint32_t) loops << 4 | (uint32_t) pair << 6 |
+           (uint32_t) group_ns << 9 | (uint32_t) (dij_slot + 1) << 12;
 }
 
 struct transport_params {
@@ -99,8 +109,8 @@ struct transport_params {
     double*  out[MQI_MAX_SCORERS];
     uint64_t out_scenario_stride;   // 0: scenarios share the arrays; else per-scenario offset (elements)
     int      loops;
-    int      let_kinds;   // any LETd / LETt scorer
-    int      dij_slot;    // the Dij scorer's slot, -1: none
+    uint32_t kind_word;   // kinds[], four bits each
+    uint32_t mode_word;   // MQI_MODE_*
     // Grouped scoring (production kernels, each-scorer-once, no Dij): the
     // leading group_ns scorers (2 .. 4) add into one interleaved array with
     // pair (2 or 4; 0: off) doubles per element, element i of scorer s at

@@ -107,49 +107,77 @@ MQI_DI void q_normalize(v3& a) {   // normalize_fast
     a.z           = a.z * r;
 }
 
-// rotate_direction with its matrices multiplied out: the local matrix
-// rotates about y and z from the identity and is applied to the z axis, and
-// the alignment takes the z axis to d
-MQI_DI void q_rotate(v3& d, float theta, float phi) {
+// rotate_direction in two parts.  q_align: the matrix g that takes the z axis
+// to d (Moller-Hughes) with the zeros of that axis multiplied out.  q_turn:
+// the local direction (theta, phi), the z axis rotated about y and z, taken
+// through it.  IEEE: divisions and square roots correctly rounded (post_poi,
+// whose matrix serves all its daughters); YX: the order |d|^2 is summed in
+// (x, y, z or y, x, z).
+struct q_mat {
+    float g0, g1, g2, g3, g4, g5, g6, g7, g8;
+};
+template<bool IEEE>
+MQI_DI float p_div(float a, float b) {
+    return IEEE ? r_div(a, b) : q_div(a, b);
+}
+template<bool IEEE>
+MQI_DI float p_sqrt(float a) {
+    return IEEE ? geo_sqrt(a) : q_sqrt(a);
+}
+template<bool IEEE, bool YX>
+MQI_DI q_mat q_align(v3 d) {
+    MQI_NO_CONTRACT
+    const float xy = YX ? __builtin_fmaf(d.x, d.x, d.y * d.y) : __builtin_fmaf(d.y, d.y, d.x * d.x);
+    const float c  = p_div<IEEE>(d.z, p_sqrt<IEEE>(__builtin_fmaf(d.z, d.z, xy)));
+    q_mat       m;
+    if (fminf(fabsf(c - 1.0f), fabsf(c + 1.0f)) < 1e-3f) {
+        // d close to the axis: two reflections, through the bisector of x
+        // and -z, U = (K, 0, -K), and through V = (1, 0, 0) - d normalised
+        const float K = 0x1.6a09e6p-1f;
+        v3          v = mk(1.0f - d.x, -d.y, -d.z);
+        const float n = p_sqrt<IEEE>(v.x * v.x + v.y * v.y + v.z * v.z);
+        v             = mk(p_div<IEEE>(v.x, n), p_div<IEEE>(v.y, n), p_div<IEEE>(v.z, n));
+        const float dot_v  = __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.x, v.x, v.y * v.y));
+        const float dot_uv = __builtin_fmaf(v.z, -K, K * v.x);
+        const float b      = p_div<IEEE>(2.0f, dot_v);
+        const float a      = p_div<IEEE>(4.0f * dot_uv, 0x1.fffffep-1f * dot_v);
+        const float b0 = v.x * b, b1 = v.y * b, b2 = v.z * b;
+        const float a0 = v.x * a, a1 = v.y * a, a2 = v.z * a;
+        m.g0 = __builtin_fmaf(K, a0, -(v.x * b0));
+        m.g1 = -(v.y * b0);
+        m.g2 = __builtin_fmaf(-K, a0, __builtin_fmaf(-v.z, b0, 1.0f));
+        m.g3 = __builtin_fmaf(K, a1, -(v.x * b1));
+        m.g4 = __builtin_fmaf(-v.y, b1, 1.0f);
+        m.g5 = __builtin_fmaf(-K, a1, -(v.z * b1));
+        m.g6 = __builtin_fmaf(K, a2, __builtin_fmaf(-v.x, b2, 1.0f));
+        m.g7 = -(v.y * b2);
+        m.g8 = __builtin_fmaf(-K, a2, -(v.z * b2));
+    } else {
+        const double dd = 1.0 - (double) (c * c);
+        const float  h  = (float) d_quot(1.0 - (double) c, dd, d_recip(dd));
+        const float  hx = d.x * h, hy = d.y * h;
+        m.g0 = __builtin_fmaf(d.y, hy, c);
+        m.g1 = m.g3 = -(d.x * hy);
+        m.g2 = d.x;
+        m.g4 = __builtin_fmaf(d.x, hx, c);
+        m.g5 = d.y;
+        m.g6 = -d.x;
+        m.g7 = -d.y;
+        m.g8 = c;
+    }
+    return m;
+}
+MQI_DI v3 q_turn(const q_mat& m, float theta, float phi) {
     MQI_NO_CONTRACT
     float st, ct, sp, cp;
     sincosf(theta, &st, &ct);
     sincosf(phi, &sp, &cp);
     v3 l = mk(cp * st, sp * st, ct);
     q_normalize(l);
-    const float tn = q_sqrt(__builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x)));
-    const float c  = q_div(d.z, tn);
-    v3          o;
-    if (fminf(fabsf(c - 1.0f), fabsf(c + 1.0f)) < 1e-3f) {
-        // d close to the axis: two reflections, through the bisector of x
-        // and -z, U = (K, 0, -K), and through V = (1, 0, 0) - d normalised
-        const float K = 0x1.6a09e6p-1f;
-        v3          v = mk(1.0f - d.x, -d.y, -d.z);
-        q_normalize(v);
-        const float dot_v  = __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.x, v.x, v.y * v.y));
-        const float dot_uv = __builtin_fmaf(v.z, -K, K * v.x);
-        const float b      = q_div(2.0f, dot_v);
-        const float a      = q_div(4.0f * dot_uv, 0x1.fffffep-1f * dot_v);
-        const float b0 = v.x * b, b1 = v.y * b, b2 = v.z * b;
-        const float a0 = v.x * a, a1 = v.y * a, a2 = v.z * a;
-        const float g0 = __builtin_fmaf(K, a0, -(v.x * b0)), g1 = -(v.y * b0),
-                    g2 = __builtin_fmaf(-K, a0, __builtin_fmaf(-v.z, b0, 1.0f));
-        const float g3 = __builtin_fmaf(K, a1, -(v.x * b1)), g4 = __builtin_fmaf(-v.y, b1, 1.0f),
-                    g5 = __builtin_fmaf(-K, a1, -(v.z * b1));
-        const float g6 = __builtin_fmaf(K, a2, __builtin_fmaf(-v.x, b2, 1.0f)), g7 = -(v.y * b2),
-                    g8 = __builtin_fmaf(-K, a2, -(v.z * b2));
-        o = mk(l.x * g0 + l.y * g1 + l.z * g2, l.x * g3 + l.y * g4 + l.z * g5, l.x * g6 + l.y * g7 + l.z * g8);
-    } else {
-        const double cc = (double) (c * c);
-        const double dd = 1.0 - cc;
-        const float  h  = (float) d_quot(1.0 - (double) c, dd, d_recip(dd));
-        const float  hx = d.x * h, hy = d.y * h;
-        const float  g0 = __builtin_fmaf(d.y, hy, c), g1 = -(d.x * hy), g4 = __builtin_fmaf(d.x, hx, c);
-        o = mk(l.x * g0 + l.y * g1 + l.z * d.x, l.x * g1 + l.y * g4 + l.z * d.y,
-               (-(l.x * d.x) - l.y * d.y) + l.z * c);
-    }
+    v3 o = mk(l.x * m.g0 + l.y * m.g1 + l.z * m.g2, l.x * m.g3 + l.y * m.g4 + l.z * m.g5,
+              l.x * m.g6 + l.y * m.g7 + l.z * m.g8);
     q_normalize(o);
-    d = o;
+    return o;
 }
 
 // distance along one axis to the exit of voxel i (axis_in with its two
@@ -178,7 +206,10 @@ MQI_DI float exit_distance(const grid_view& g, v3 p, v3& d, int& cx, int& cy, in
     return -1.0f;
 }
 
-// relq(Ek) as far as a step needs it
+// relativistic_quantities (mqi_relativistic_quantities.hpp:24-43) in float as
+// far as a step needs them: beta^2 = Ek (Ek + 2 Mp) / Et^2 and p^2 = Ek (Ek +
+// 2 Mp), without the cancellations of 1 - 1 / gamma^2 and Et^2 - Mp^2 at low
+// energy
 struct q_rel {
     float beta_sq, pp, Et_sq;   // pp = Ek (Ek + 2 Mp), the momentum squared
     float Et;

@@ -37,21 +37,31 @@ using namespace mqi_dev;
 namespace MQI_NS
 {
 
+// The launch's parameters as read where they are needed: loads through this
+// reference are not moved out of the history loop.  Parameters of the rare
+// paths (new histories, secondaries, beamline children) otherwise end up
+// loaded before the loop, spilled from the scalar registers into VGPR lanes
+// and read back by v_readlane wherever they are used.  With the scoring modes
+// of a step in two words and its cell's edges read once: 33 spilled scalars
+// for 171 and 138 VGPRs for 151; slab phantom 37.3 -> 33.5 ms, water spot 5.55
+// -> 5.31 ms.
+MQI_DI const transport_params& cold() {
+    uint64_t a = (uint64_t) __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    auto p = (const __attribute__((address_space(4))) transport_params*) a;
+    return *(const transport_params*) p;
+}
+
 // ------------------------------------------------------------------ physics
 // Per-lane context: LDS tables, grid view, RNG, the lane's secondary stack.
 struct ctx {
     const float* T;   // LDS tables
     grid_view    g;
     rng_t        rng;
-    float*       stack;   // HBM, stack_cap * MQI_STACK_FLOATS floats for this lane
     int          sp;
-    int          cap;
-    float        fwd[9];   // held by value: a pointer into the kernel
-    float        trans[3]; // arguments would force them into private memory
     unsigned     drops;
     int          child;    // world child the track is in: 0 .. nbl - 1 beamline, nbl the patient
     int          nbl;      // beamline children
-    const float* blxf;     // their transforms (fwd[9], inv[9], translation[3] each), HBM
 };
 
 #if MQI_EXACT
@@ -250,7 +260,7 @@ MQI_DI void q_along_step(ctx& c, trk& t, float len, float rho, float sp) {
     const float th_sq = q_div(q_div(q * q, rel.beta_sq) * len, q_radiation_length<DBG>(rho));
     const float th    = fabsf(c.rng.st_z1 * (0x1.6a09e6p+0f * q_sqrt(th_sq)));   // sqrt(2)
     const float phi   = (float) (2.0 * 3.14159265358979323846 * (double) c.rng.st_u1);
-    q_rotate(t.d1, th, phi);
+    t.d1 = q_turn(q_align<false, false>(t.d1), th, phi);
     t.dE = __builtin_fmaf(dE, r, t.dE);
     update_pos(t, r * len);
     t.ke1 = __builtin_fmaf(-dE, r, t.ke1);
@@ -260,17 +270,17 @@ MQI_DI void q_along_step(ctx& c, trk& t, float len, float rho, float sp) {
 
 // secondary placement: pos -> fwd (pos - T) + T, dir -> fwd dir (e.g.
 // mqi_pp_elastic.hpp:190-196), with the transform of the child the track is
-// in.  In the patient (c.fwd, c.trans) at the push; a secondary made in a
+// in.  In the patient (P.fwd, P.trans) at the push; a secondary made in a
 // beamline child is stored unplaced with the child's index and placed with
 // that child's transform when it is popped (the same operations, so the same
 // bits), which keeps the beamline transforms out of the physics.
-MQI_DI v3 place(const ctx& c, v3 p) {
+MQI_DI v3 place(const transport_params& P, v3 p) {
     MQI_NO_CONTRACT
-    v3 q = mk(p.x - c.trans[0], p.y - c.trans[1], p.z - c.trans[2]);
-    q    = mv(c.fwd, q);
-    return mk(q.x + c.trans[0], q.y + c.trans[1], q.z + c.trans[2]);
+    v3 q = mk(p.x - P.trans[0], p.y - P.trans[1], p.z - P.trans[2]);
+    q    = mv(P.fwd, q);
+    return mk(q.x + P.trans[0], q.y + P.trans[1], q.z + P.trans[2]);
 }
-MQI_DI v3 turn(const ctx& c, v3 d) { return mv(c.fwd, d); }
+MQI_DI v3 turn(const transport_params& P, v3 d) { return mv(P.fwd, d); }
 // the same with a child's transform (fwd[9], inv[9], translation[3]) in HBM
 MQI_DI v3 place_xf(const float* f, v3 p) {
     MQI_NO_CONTRACT
@@ -281,9 +291,15 @@ MQI_DI v3 place_xf(const float* f, v3 p) {
 // track_stack_t::push_secondary: dropped when the stack is full (mqi_track_stack.hpp:36-41).
 // A pushed track keeps vtx0, vtx1.ke and dE; vtx1 position/direction are
 // overwritten when it is popped, local_dE is always zero, status is CREATED.
-MQI_DI void push(ctx& c, float ke0, v3 p0, v3 d0, float ke1, float dE, float tag) {
-    if (c.sp < c.cap) {
-        float* s = c.stack + MQI_STACK_FLOATS * c.sp;
+// The lane's stack (P.stack_cap entries in HBM) is addressed from the launch
+// at the few pushes and pops, not from a pointer held through the loop.
+MQI_DI float* stack_entry(const transport_params& P, int k) {
+    const uint64_t tid = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    return P.stack + (tid * (uint32_t) P.stack_cap + (uint32_t) k) * MQI_STACK_FLOATS;
+}
+MQI_DI void push(const transport_params& P, ctx& c, float ke0, v3 p0, v3 d0, float ke1, float dE, float tag) {
+    if (c.sp < P.stack_cap) {
+        float* s = stack_entry(P, c.sp);
         s[0]     = ke0;
         s[1]     = p0.x;
         s[2]     = p0.y;
@@ -301,17 +317,17 @@ MQI_DI void push(ctx& c, float ke0, v3 p0, v3 d0, float ke1, float dE, float tag
 }
 
 // push a daughter made at (p, d) in the current child
-MQI_DI void push_placed(ctx& c, float ke0, v3 p, v3 d, float ke1, float dE) {
+MQI_DI void push_placed(const transport_params& P, ctx& c, float ke0, v3 p, v3 d, float ke1, float dE) {
     if (c.child < c.nbl)
-        push(c, ke0, p, d, ke1, dE, (float) c.child);
+        push(P, c, ke0, p, d, ke1, dE, (float) c.child);
     else
-        push(c, ke0, place(c, p), turn(c, d), ke1, dE, -1.0f);
+        push(P, c, ke0, place(P, p), turn(P, d), ke1, dE, -1.0f);
 }
 
 #if MQI_EXACT
 // p_ionization_tabulated::post_step: delta-ray (mqi_p_ionization.hpp:424-477)
 template<bool DBG>
-MQI_DI void post_ion(ctx& c, trk& t) {
+MQI_DI void post_ion(const transport_params& P, ctx& c, trk& t) {
     rel_q       rel   = relq(t.ke1);
     const float T_cut = DBG ? 0.08511 * 1.0 : 0.0815 * 1.0;
     float       Te, n;
@@ -325,7 +341,7 @@ MQI_DI void post_ion(ctx& c, trk& t) {
         if (acc < 1.0 - rel.beta_sq * Te / rel.Te_max + Te * Te / (2.0 * rel.Et_sq)) break;
     }
     if (DBG) {
-        push_placed(c, 0.0f, t.p0, t.d0, 0.0f, Te);
+        push_placed(P, c, 0.0f, t.p0, t.d0, 0.0f, Te);
     } else {
         t.dE += Te;
     }
@@ -336,7 +352,7 @@ MQI_DI void post_ion(ctx& c, trk& t) {
 // The first trial's numbers come from the interaction's block; the later
 // ones (acceptance is above 1/2) from the history's stream.
 template<bool DBG>
-MQI_DI void post_ion(ctx& c, trk& t) {
+MQI_DI void post_ion(const transport_params& P, ctx& c, trk& t) {
     MQI_NO_CONTRACT
     const q_rel  rel    = q_relq(t.ke1);
     const float  te_max = q_te_max(rel);
@@ -356,7 +372,7 @@ MQI_DI void post_ion(ctx& c, trk& t) {
         c.rng.pair(n, acc);
     }
     if (DBG) {
-        push_placed(c, 0.0f, t.p0, t.d0, 0.0f, Te);
+        push_placed(P, c, 0.0f, t.p0, t.d0, 0.0f, Te);
     } else {
         t.dE += Te;
     }
@@ -364,8 +380,10 @@ MQI_DI void post_ion(ctx& c, trk& t) {
 }
 #endif
 
+#if MQI_EXACT
 // pp_elastic_tabulated::post_step (mqi_pp_elastic.hpp:119-219)
-MQI_DI void post_pp(ctx& c, trk& t) {
+template<bool DBG>
+MQI_DI void post_pp(const transport_params& P, ctx& c, trk& t) {
     rel_q rel       = relq(t.ke1);
     float min_value = 0.5f / rel.Ek;
     float r0, r1;
@@ -397,17 +415,17 @@ MQI_DI void post_pp(ctx& c, trk& t) {
     rotate_direction(t.d1, th3, phi);
     v3 dd = t.d1;
     rotate_direction(dd, th4, phi);
-    push_placed(c, dE, t.p1, dd, dE, 0.0f);
+    push_placed(P, c, dE, t.p1, dd, dE, 0.0f);
 }
 
 // po_elastic::post_step (mqi_po_elastic.hpp:96-217); exponential not truncated (CPU semantics)
 template<bool DBG>
-MQI_DI void post_poe(ctx& c, trk& t) {
+MQI_DI void post_poe(const transport_params& P, ctx& c, trk& t) {
     rel_q rel = relq(t.ke1);
     if (rel.Ek <= 5.5f) {
         float dE = rel.Ek;
         if (DBG)
-            push_placed(c, dE, t.p1, t.d1, 0.0f, dE);
+            push_placed(P, c, dE, t.p1, t.d1, 0.0f, dE);
         else
             t.ldE += dE;
         t.ke1 -= dE;
@@ -430,7 +448,7 @@ MQI_DI void post_poe(ctx& c, trk& t) {
         float th3 = MQ_ACOSF(cos_th3);
         float phi = 2.0 * 3.14159265358979323846 * u1;
         if (DBG)
-            push_placed(c, dE, t.p0, t.d0, 0.0f, dE);
+            push_placed(P, c, dE, t.p0, t.d0, 0.0f, dE);
         else
             t.ldE += dE;
         t.ke1 -= dE;
@@ -440,7 +458,7 @@ MQI_DI void post_poe(ctx& c, trk& t) {
 
 // po_inelastic_tabulated::post_step (mqi_po_inelastic.hpp:158-288)
 template<bool DBG>
-MQI_DI void post_poi(ctx& c, trk& t) {
+MQI_DI void post_poi(const transport_params& P, ctx& c, trk& t) {
     const float Ek = t.ke1;
     float       Eb = 5.0f;
     float       Er = Ek;
@@ -481,11 +499,11 @@ MQI_DI void post_poi(ctx& c, trk& t) {
             float phi = 2.0 * 3.14159265358979323846 * r1;
             v3    dd  = t.d1;
             rotate_direction(dd, th, phi);
-            push_placed(c, dE, t.p1, dd, dE, 0.0f);
+            push_placed(P, c, dE, t.p1, dd, dE, 0.0f);
         } else if (zeta < Prob_long) {
             // long-range energy leaves the track
         } else if (DBG) {
-            push_placed(c, dE, t.p0, t.d0, 0.0f, dE);
+            push_placed(P, c, dE, t.p0, t.d0, 0.0f, dE);
         }
         Eb *= E_ratio;
     }
@@ -493,6 +511,144 @@ MQI_DI void post_poi(ctx& c, trk& t) {
     t.ke1 -= Er;
     t.stopped = true;
 }
+#else
+// pp_elastic_tabulated::post_step (mqi_pp_elastic.hpp:119-219)
+template<bool DBG>
+MQI_DI void post_pp(const transport_params& P, ctx& c, trk& t) {
+    MQI_NO_CONTRACT
+    const float Mp = units::Mp, Ek = t.ke1;
+    const q_rel rel = q_relq(Ek);
+    float       r0, r1;
+    c.rng.pair(r0, r1);
+    const double mv_ = (double) q_div(0.5f, Ek);
+    const float  u   = (float) __builtin_fma(__builtin_fma(mv_, -2.0, 1.0), (double) r0, mv_);
+    const float  E1 = rel.Et, dE = Ek * u, Ek1 = __builtin_fmaf(-Ek, u, Ek);
+    const float  E3 = Ek1 + Mp, E4 = dE + Mp;
+    const float  P1 = q_sqrt(rel.pp);
+    const float  P3 = q_sqrt(__builtin_fmaf(E3, E3, -units::Mp_sq));
+    const float  P4 = q_sqrt(__builtin_fmaf(E4, E4, -units::Mp_sq));
+    float cos_th3  = q_div(__builtin_fmaf(-Mp, E1 - E3, __builtin_fmaf(E1, E3, -units::Mp_sq)), P1 * P3);
+    float cos_th34 = q_div(__builtin_fmaf(E4, E3, -(Mp * E1)), P4 * P3);
+    if (cos_th3 > 1.0f)
+        cos_th3 = 1.0f;
+    else if (cos_th3 < -1.0f)
+        cos_th3 = -1.0f;
+    if (cos_th34 > 1.0f)
+        cos_th34 = 1.0f;
+    else if (cos_th34 < -1.0f)
+        cos_th34 = -1.0f;
+    const float th3 = MQ_ACOSF(cos_th3);
+    const float th4 = th3 - MQ_ACOSF(cos_th34);
+    const float phi = (float) (2.0 * 3.14159265358979323846 * (double) r1);
+    t.ke1           = Ek1;
+    t.d1            = q_turn(q_align<false, true>(t.d1), th3, phi);
+    const v3 dd     = q_turn(q_align<false, false>(t.d1), th4, phi);
+    push_placed(P, c, dE, t.p1, dd, dE, 0.0f);
+}
+
+// po_elastic::post_step (mqi_po_elastic.hpp:96-217); exponential not truncated (CPU semantics)
+template<bool DBG>
+MQI_DI void post_poe(const transport_params& P, ctx& c, trk& t) {
+    MQI_NO_CONTRACT
+    const float Ek = t.ke1;
+    if (Ek <= 5.5f) {
+        if (DBG)
+            push_placed(P, c, Ek, t.p1, t.d1, 0.0f, Ek);
+        else
+            t.ldE += Ek;
+        t.ke1 -= Ek;
+        t.stopped = true;
+    } else {
+        const double ek = (double) Ek;
+        float        Tp_avg = (float) (0.65 * MQ_EXPD(-0.0013 * ek));
+        Tp_avg              = (float) ((double) Tp_avg - 0.71 * MQ_EXPD(-0.0177 * ek));
+        float uu, u1;
+        c.rng.pair(uu, u1);
+        const float  dE  = q_div(-q_log(uu), r_div(1.0f, Tp_avg));
+        const float  Ek1 = Ek - dE;
+        const double ek1 = (double) Ek1, de = (double) dE;
+        const float  E1 = (float) ((ek + 2.0 * (double) units::Mp) * ek);
+        const float  E3 = (float) ((ek1 + 2.0 * (double) units::Mp) * ek1);
+        const double q  = (double) q_sqrt(E1 * E3);
+        const double n  = __builtin_fma(-(de + 2.0 * (double) units::Mo), de, (double) (E1 + E3)) * 0.5;
+        float        cos_th3 = (float) d_quot(n, q, d_recip(q));
+        if (cos_th3 > 1.0f) cos_th3 = 1.0f;
+        if (cos_th3 < -1.0f) cos_th3 = -1.0f;
+        const float th3 = MQ_ACOSF(cos_th3);
+        const float phi = (float) (2.0 * 3.14159265358979323846 * (double) u1);
+        if (DBG)
+            push_placed(P, c, dE, t.p0, t.d0, 0.0f, dE);
+        else
+            t.ldE += dE;
+        t.ke1 = Ek1;
+        t.d1  = q_turn(q_align<false, true>(t.d1), th3, phi);
+    }
+}
+
+// po_inelastic_tabulated::post_step (mqi_po_inelastic.hpp:158-288)
+template<bool DBG>
+MQI_DI void post_poi(const transport_params& P, ctx& c, trk& t) {
+    MQI_NO_CONTRACT
+    const float Ek = t.ke1;
+    float       Eb = 5.0f;
+    float       Er = Ek;
+    const float E_mini = 2.0f, E_ratio = 0.65f;
+    float       Prob_2nd, Prob_long, power;
+    if (Ek <= 215 && Ek > 200) {
+        Prob_2nd  = 0.78f;
+        Prob_long = Prob_2nd + (1 - Prob_2nd) * 0.9;
+        power     = 0.4f;
+    } else if (Ek > 215) {
+        Prob_2nd  = 0.78f;
+        Prob_long = Prob_2nd + (1 - Prob_2nd) * 1.0;
+        power     = 0.4f;
+    } else if (Ek <= 200 && Ek > 150) {
+        Prob_2nd  = 0.72f;
+        Prob_long = Prob_2nd + (1 - Prob_2nd) * 0.83;
+        power     = 0.45f;
+    } else {
+        Prob_2nd  = 0.7f;
+        Prob_long = Prob_2nd + (1 - Prob_2nd) * 0.83;
+        power     = 0.52f;
+    }
+    float rest = Er - Eb;   // the energy left, less the next binding energy
+    if (rest > E_mini) {
+        // every daughter leaves from the same direction
+        const q_mat  m  = q_align<true, true>(t.d1);
+        const double ek = (double) Ek, rk = d_recip(ek);
+        do {
+            Er = rest;
+            float u, zeta;
+            c.rng.pair(u, zeta);
+            float dE = __builtin_fmaf(Er - E_mini, MQ_POWF(u, power), E_mini);
+            if (dE >= Er) dE = Er;
+            Er -= dE;
+            t.ke1 -= dE + Eb;
+            if (zeta < Prob_2nd) {
+                float r0, r1;
+                c.rng.pair(r0, r1);
+                const double a  = d_quot((double) dE + (double) dE, ek, rk) - 1.0;
+                const double b  = (double) (1.0f - q_div(dE, Ek));
+                float        cos_th = (float) __builtin_fma(b + b, (double) r0, a);
+                if (cos_th < -1.0f) cos_th = -1.0f;
+                if (cos_th > 1.0f) cos_th = 1.0f;
+                const float th  = MQ_ACOSF(cos_th);
+                const float phi = (float) (2.0 * 3.14159265358979323846 * (double) r1);
+                push_placed(P, c, dE, t.p1, q_turn(m, th, phi), dE, 0.0f);
+            } else if (zeta < Prob_long) {
+                // long-range energy leaves the track
+            } else if (DBG) {
+                push_placed(P, c, dE, t.p0, t.d0, 0.0f, dE);
+            }
+            rest = __builtin_fmaf(-E_ratio, Eb, Er);
+            Eb *= E_ratio;
+        } while (rest > E_mini);
+    }
+    t.dE += Er;
+    t.ke1 -= Er;
+    t.stopped = true;
+}
+#endif
 
 #if MQI_EXACT
 // fippel_physics::stepping (mqi_fippel_physics.hpp:68-216).  The three
@@ -564,13 +720,13 @@ MQI_DI void stepping(ctx& c, trk& t, float rho, float d2b, float& sp) {
     float u = cs_sum * c.rng.uniform();
     t.d1    = t.d0;
     if (u < cs0) {
-        post_ion<DBG>(c, t);
+        post_ion<DBG>(cold(), c, t);
     } else if (u < (cs0 + csa)) {
-        post_pp(c, t);
+        post_pp<DBG>(cold(), c, t);
     } else if (u < (cs0 + csa + csb)) {
-        post_poe<DBG>(c, t);
+        post_poe<DBG>(cold(), c, t);
     } else if (u < (cs0 + csa + csb + csc)) {
-        post_poi<DBG>(c, t);
+        post_poi<DBG>(cold(), c, t);
     }
 }
 #else
@@ -635,13 +791,13 @@ MQI_DI void stepping(ctx& c, trk& t, float rho, float d2b, float& sp) {
     const float s0 = rho * ion, s1 = s0 + rho * pp, s2 = s1 + rho * poe, s3 = s2 + rho * poi;
     t.d1           = t.d0;
     if (u < s0) {
-        post_ion<DBG>(c, t);
+        post_ion<DBG>(cold(), c, t);
     } else if (u < s1) {
-        post_pp(c, t);
+        post_pp<DBG>(cold(), c, t);
     } else if (u < s2) {
-        post_poe<DBG>(c, t);
+        post_poe<DBG>(cold(), c, t);
     } else if (u < s3) {
-        post_poi<DBG>(c, t);
+        post_poi<DBG>(cold(), c, t);
     }
 }
 #endif
@@ -716,6 +872,27 @@ MQI_DI void dij_insert(const transport_params& P, uint64_t item, uint32_t voxel,
     atomicOr(P.status, MQI_STATUS_DIJ_FULL);
 }
 
+// The launch's scoring as the loop's code reads it: two words, taken apart
+// where a field is used (a compiler that sees the fields' comparisons before
+// the history loop keeps each one's lane mask in a pair of scalar registers).
+struct scoring {
+    uint32_t kinds, mode;
+    MQI_DI int  n() const { return mode & 7; }
+    MQI_DI int  kind(int s) const { return kinds >> 4 * s & 15; }
+    MQI_DI bool let() const { return mode & 8; }
+    MQI_DI int  loops() const { return mode >> 4 & 3; }
+    MQI_DI int  pair() const { return mode >> 6 & 7; }
+    MQI_DI int  grouped() const { return mode >> 9 & 7; }
+    MQI_DI int  dij_slot() const { return (int) (mode >> 12 & 15) - 1; }
+};
+MQI_DI scoring scoring_of(const transport_params& P) {
+    scoring S;
+    S.kinds = P.kind_word;
+    S.mode  = P.mode_word;
+    asm volatile("" : "+s"(S.kinds), "+s"(S.mode));
+    return S;
+}
+
 // Deposits of consecutive steps into the same voxel (and scenario, and Dij
 // table) are summed per lane and added to the scorer arrays, or inserted
 // into the Dij table, once, when the lane moves on (each-scorer-once scoring
@@ -735,20 +912,20 @@ MQI_DI uint64_t pend_element(const transport_params& P, const pending& A) {
 
 // accumulated slots are positive, +inf or NaN (every value that is not <= 0
 // is added, NaN included); untouched slots are 0
-MQI_DI void flush(const transport_params& P, pending& A, double* v) {
+MQI_DI void flush(const transport_params& P, const scoring& S, pending& A, double* v) {
     if (A.cnb >= 0) {
         const uint64_t k  = pend_element(P, A);
         double         dx = 0.0;   // the Dij slot's sum: inserted behind the loop, from one place
 #pragma unroll
         for (int s = 0; s < MQI_DEFER; ++s) {
-            if (s >= P.n_scorers) break;
+            if (s >= S.n()) break;
             const double x = v[s * blockDim.x];
-            if (s == P.dij_slot) {
+            if (s == S.dij_slot()) {
                 dx = x;
             } else if (x != 0.0) {
 #if !MQI_EXACT
-                if (P.pair && s < P.group_ns)
-                    atomicAdd(P.pair_out + (uint64_t) P.pair * k + s, x);
+                if (s < S.grouped())
+                    atomicAdd(P.pair_out + (uint64_t) S.pair() * k + s, x);
                 else
 #endif
                     atomicAdd(P.out[s] + k, x);
@@ -822,12 +999,12 @@ MQI_DI void quad_swap(bool up, double& x, double& y) {
 // a voxel's sums go out as one line request (the sums are transposed within
 // the group in two exchanges).  Lanes of a group with a lane that does not
 // step add their own sums.
-MQI_DI void flush_quad(const transport_params& P, pending& A, double* v, bool f) {
+MQI_DI void flush_quad(const transport_params& P, const scoring& S, pending& A, double* v, bool f) {
     const bool     has = f && A.cnb >= 0;
     double         x0  = has ? v[0] : 0.0;
     double         x1  = has ? v[blockDim.x] : 0.0;
     double         x2  = has ? v[2 * blockDim.x] : 0.0;
-    double         x3  = (has && P.group_ns > 3) ? v[3 * blockDim.x] : 0.0;
+    double         x3  = (has && S.grouped() > 3) ? v[3 * blockDim.x] : 0.0;
     const uint64_t k   = 4 * (has ? pend_element(P, A) : 0);
     const int      q   = __lane_id() & 3;
     const int      all = quad_get<QUAD_OF(0)>(0, 1) & quad_get<QUAD_OF(1)>(0, 1) & quad_get<QUAD_OF(2)>(0, 1) &
@@ -856,9 +1033,9 @@ MQI_DI void flush_quad(const transport_params& P, pending& A, double* v, bool f)
 #endif
 
 template<bool DBG>
-MQI_DI void score(const transport_params& P, const trk& t, uint32_t cnb, float density, float volume, float sp,
+MQI_DI void score(const transport_params& P, const scoring& S, const trk& t, uint32_t cnb, float density, float volume, float sp,
                   uint32_t dij_item, uint32_t scen, pending& A, double* pv) {
-    const int n = P.n_scorers;
+    const int n = S.n();
     // regular scorers score through roi_->idx(cnb) > 0, the statistics pair
     // through get_mask_idx(cnb) >= 0 (mqi_transport.hpp:342-364), under
     // roi_t DIRECT every voxel but 0 and every voxel; a CONTOUR ROI's answer
@@ -872,7 +1049,7 @@ MQI_DI void score(const transport_params& P, const trk& t, uint32_t cnb, float d
     const bool fresh = (int32_t) cnb != A.cnb;
     double     length = 0.0, let = 0.0;
     bool       has_let = false;
-    if (P.let_kinds) has_let = let_terms(t, density, length, let);
+    if (S.let()) has_let = let_terms(t, density, length, let);
     double dv = 0.0;   // the Dij scorer's value and repeats when it is not deferred
     int    dr = 0;
     // The loop runs over the fixed maximum with constant indices so that the
@@ -881,11 +1058,11 @@ MQI_DI void score(const transport_params& P, const trk& t, uint32_t cnb, float d
 #pragma unroll
     for (int s = 0; s < MQI_MAX_SCORERS; ++s) {
         if (s >= n) break;
-        const int kind = P.kinds[s];
+        const int kind = S.kind(s);
         double    v    = d;
         if (kind == MQI_KIND_STAT_DOSE2) {
             v = d * d;
-        } else if (P.let_kinds && kind != MQI_KIND_DOSE) {
+        } else if (S.let() && kind != MQI_KIND_DOSE) {
             if (kind == MQI_KIND_LETD_NUM)
                 v = (!has_let || let >= 25.0) ? 0.0 : t.dE * let;
             else if (kind == MQI_KIND_LETD_DEN)
@@ -900,16 +1077,16 @@ MQI_DI void score(const transport_params& P, const trk& t, uint32_t cnb, float d
         else if (kind == MQI_KIND_DM)
             v = dm_hit(t, density, volume);
         const bool stat = (kind == MQI_KIND_STAT_DOSE || kind == MQI_KIND_STAT_DOSE2);
-        if (P.loops == MQI_LOOPS_ONCE && s < MQI_DEFER) {
+        if (S.loops() == MQI_LOOPS_ONCE && s < MQI_DEFER) {
             double*      acc = pv + s * blockDim.x;
             const double o   = fresh ? 0.0 : *acc;
             *acc             = (!(stat ? in_stat : in_reg) || v <= 0) ? o : o + v;
             continue;
         }
         int reps = 0;
-        if (P.loops == MQI_LOOPS_ONCE) {
+        if (S.loops() == MQI_LOOPS_ONCE) {
             reps = (stat ? in_stat : in_reg) ? 1 : 0;
-        } else if (P.loops == MQI_LOOPS_PLAIN) {
+        } else if (S.loops() == MQI_LOOPS_PLAIN) {
             // mqi_transport.hpp:204-225: scorers 0..n-3 in both loops
             reps = in_reg ? ((s < n - 2) ? 2 : 1) : 0;
         } else {
@@ -929,7 +1106,7 @@ MQI_DI void score(const transport_params& P, const trk& t, uint32_t cnb, float d
     }
     // one insert site for every slot and loop
     for (int r = 0; r < dr; ++r) dij_insert(P, dij_item, cnb, dv);
-    if (P.loops == MQI_LOOPS_ONCE) {
+    if (S.loops() == MQI_LOOPS_ONCE) {
         A.cnb  = (int32_t) cnb;
         A.scen = scen;
         A.item = dij_item;
@@ -1053,14 +1230,14 @@ MQI_DI bool enter_chain(const transport_params& P, ctx& c, trk& t, const float* 
     return enter(P, c, t);
 }
 
-MQI_DI void pop(ctx& c, trk& t) {
+MQI_DI void pop(const transport_params& P, ctx& c, trk& t) {
     --c.sp;
-    const float* s = c.stack + MQI_STACK_FLOATS * c.sp;
+    const float* s = stack_entry(P, c.sp);
     t.ke0          = s[0];
     t.p0           = mk(s[1], s[2], s[3]);
     t.d0           = mk(s[4], s[5], s[6]);
     if (s[9] >= 0.0f) {   // made in beamline child s[9]: place it now
-        const float* f = c.blxf + 21 * (int) s[9];
+        const float* f = P.bl_xf + 21 * (int) s[9];
         t.p0           = place_xf(f, t.p0);
         t.d0           = mv(f, t.d0);
     }
@@ -1165,15 +1342,20 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
     const bool bl = c.child < c.nbl;
     uint64_t   cnb;
     float      rho;
+    // a track starts its step where it stands (said here so that the end point
+    // is not kept beside the start from one step to the next)
+    t.p1 = t.p0;
+    t.d1 = t.d0;
     if (bl) {
         // the beamline child's grid view is rebuilt after stepping rather
         // than kept live across it (register pressure of the patient path)
-        const grid_view gb = bl_view(P, shb, c.child);
-        const int*     m   = P.bl_meta + 8 * c.child;
+        const transport_params& B  = cold();
+        const grid_view         gb = bl_view(B, shb, c.child);
+        const int*              m  = B.bl_meta + 8 * c.child;
         const uint64_t off = (uint64_t) (uint32_t) m[4] | ((uint64_t) (uint32_t) m[5] << 32);
         cnb                = (uint64_t) (int32_t) (t.cz * gb.nx * gb.ny + t.cy * gb.nx + t.cx);
         t.its              = MQI_VOXEL_EXIT(gb, t.p0, t.d0, t.cx, t.cy, t.cz);
-        rho                = P.bl_density[off + cnb];
+        rho                = B.bl_density[off + cnb];
     } else {
         cnb              = (uint64_t) (int32_t) (t.cz * c.g.nx * c.g.ny + t.cy * c.g.nx + t.cx);
         const float dens = P.density[cnb];
@@ -1185,27 +1367,29 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
         // issued just before the next wait on a load would add their round
         // trip to every step.
         // (A history's deposits are its own scenario's and Dij table's.)
-        const bool leave = P.loops == MQI_LOOPS_ONCE && ((int32_t) cnb != L.acc.cnb || L.newhist);
+        const scoring S  = scoring_of(P);
+        const bool leave = S.loops() == MQI_LOOPS_ONCE && ((int32_t) cnb != L.acc.cnb || L.newhist);
         L.newhist        = false;
 #if !MQI_EXACT
-        if (P.pair == 2)
+        if (S.pair() == 2)
             flush_pair(P, L.acc, pv, leave);
-        else if (P.pair == 4)
-            flush_quad(P, L.acc, pv, leave);
+        else if (S.pair() == 4)
+            flush_quad(P, S, L.acc, pv, leave);
         else
 #endif
         if (leave)
-            flush(P, L.acc, pv);
+            flush(P, S, L.acc, pv);
     }
     float sp;   // stopping power ratio of the step
     stepping<DBG>(c, t, rho, t.its, sp);
     if (bl) {
-        const grid_view gb    = bl_view(P, shb, c.child);
-        bool            leave = t.its < 0;
+        const transport_params& B     = cold();
+        const grid_view         gb    = bl_view(B, shb, c.child);
+        bool                    leave = t.its < 0;
         if (!leave && !t.stopped) {
-            step_axis(t.p1.x, t.d1.x, gb.xe, 0.0f, t.cx);
-            step_axis(t.p1.y, t.d1.y, gb.ye, 0.0f, t.cy);
-            step_axis(t.p1.z, t.d1.z, gb.ze, 0.0f, t.cz);
+            t.cx += step_cell(t.p1.x, t.d1.x, gb.X(t.cx), gb.X(t.cx + 1));
+            t.cy += step_cell(t.p1.y, t.d1.y, gb.Y(t.cy), gb.Y(t.cy + 1));
+            t.cz += step_cell(t.p1.z, t.d1.z, gb.Z(t.cz), gb.Z(t.cz + 1));
             move(t);
             leave = !is_valid(gb, t.cx, t.cy, t.cz);
         }
@@ -1213,13 +1397,13 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
             // a stopped track does nothing in the children after this one
             L.active = false;
         } else if (leave) {
-            leave_bl(P, c.child, t);
+            leave_bl(B, c.child, t);
             ++c.child;
             L.reenter = true;
         }
         if (++L.tsteps > MQI_MAX_TRACK_STEPS && L.active) {
             L.active = false;
-            atomicOr(P.status, MQI_STATUS_TRACK_CAP);
+            atomicOr(cold().status, MQI_STATUS_TRACK_CAP);
         }
         return;
     }
@@ -1227,21 +1411,24 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
         L.active = false;
         return;
     }
+    // the voxel's edges: its volume and the cell after the step.
+    // get_volume(cnb) (mqi_grid3d.hpp:471-487) goes through cnb2ijk; the
+    // lane's cell indices are that (i, j, k) already
+    const float x0 = c.g.X(t.cx), x1 = c.g.X(t.cx + 1);
+    const float y0 = c.g.Y(t.cy), y1 = c.g.Y(t.cy + 1);
+    const float z0 = c.g.Z(t.cz), z1 = c.g.Z(t.cz + 1);
     if (TRACE) {
         trace_record(P, L, cnb);
     } else {
-        // get_volume(cnb) (mqi_grid3d.hpp:471-487) goes through cnb2ijk; the
-        // lane's cell indices are that (i, j, k) already
-        const int i = t.cx, j = t.cy, k = t.cz;
-        float     vol = c.g.X(i + 1) - c.g.X(i);
-        vol *= c.g.Y(j + 1) - c.g.Y(j);
-        vol *= c.g.Z(k + 1) - c.g.Z(k);
-        score<DBG>(P, t, (uint32_t) cnb, rho, vol, sp, L.dij_item, L.scen, L.acc, pv);
+        float vol = x1 - x0;
+        vol *= y1 - y0;
+        vol *= z1 - z0;
+        score<DBG>(P, scoring_of(P), t, (uint32_t) cnb, rho, vol, sp, L.dij_item, L.scen, L.acc, pv);
     }
     if (!t.stopped) {
-        step_axis(t.p1.x, t.d1.x, c.g.xe, c.g.sx, t.cx);
-        step_axis(t.p1.y, t.d1.y, c.g.ye, c.g.sy, t.cy);
-        step_axis(t.p1.z, t.d1.z, c.g.ze, c.g.sz, t.cz);
+        t.cx += step_cell(t.p1.x, t.d1.x, x0, x1);
+        t.cy += step_cell(t.p1.y, t.d1.y, y0, y1);
+        t.cz += step_cell(t.p1.z, t.d1.z, z0, z1);
         move(t);
     }
     L.active = is_valid(c.g, t.cx, t.cy, t.cz) && !t.stopped;
@@ -1249,7 +1436,7 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
     // tracks whose state went non-finite
     if (++L.tsteps > MQI_MAX_TRACK_STEPS && L.active) {
         L.active = false;
-        atomicOr(P.status, MQI_STATUS_TRACK_CAP);
+        atomicOr(cold().status, MQI_STATUS_TRACK_CAP);
     }
 }
 
@@ -1293,16 +1480,10 @@ k_transport(transport_params P) {
     c.g.xe  = sh + T_TABLES;
     c.g.ye  = c.g.xe + P.nx + 1;
     c.g.ze  = c.g.ye + P.ny + 1;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) c.fwd[i] = P.fwd[i];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) c.trans[i] = P.trans[i];
-    c.cap   = P.stack_cap;
     c.sp    = 0;
     c.drops = 0;
     c.child = 0;
     c.nbl   = P.n_bl;
-    c.blxf  = P.bl_xf;
 #if !MQI_EXACT
     c.rng.set_seed(P.seed);
 #endif
@@ -1314,7 +1495,6 @@ k_transport(transport_params P) {
     for (int s = 0; s < MQI_DEFER; ++s) pv[s * blockDim.x] = 0.0;
     const uint64_t tid      = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t nthreads = (uint64_t) gridDim.x * blockDim.x;
-    c.stack                 = P.stack + tid * (uint64_t) P.stack_cap * MQI_STACK_FLOATS;
 
     // plain: the thread's start_and_length slice; dynamic: the lane's current
     // chunk of P.fetch_chunk consecutive histories from the device counter
@@ -1363,13 +1543,14 @@ k_transport(transport_params P) {
         }
         if (need && !refill) continue;
         if (refill) {
-            uint64_t g;
+            const transport_params& C = cold();
+            uint64_t                g;
             if (DYNAMIC) {
                 if (s_next >= s_end) {
                     // Wave-aggregated fetch of fetch_chunk histories per dry
                     // lane from range qx (initially this XCD's own range; a
                     // range that runs dry sends the wave to the next one).
-                    const uint64_t chunk = (uint64_t) P.fetch_chunk;
+                    const uint64_t chunk = (uint64_t) C.fetch_chunk;
                     const int      me    = __lane_id();
                     bool           got   = false;
                     for (int r = 0; r < MQI_QUEUES; ++r) {
@@ -1382,9 +1563,9 @@ k_transport(transport_params P) {
                         const int          q    = __shfl(qx, lead);
                         unsigned long long base = 0;
                         if (me == lead)
-                            base = atomicAdd(P.queue + q * MQI_QUEUE_STRIDE, (unsigned long long) __popcll(m) * chunk);
+                            base = atomicAdd(C.queue + q * MQI_QUEUE_STRIDE, (unsigned long long) __popcll(m) * chunk);
                         base               = __shfl(base, lead);
-                        const uint64_t end = mqi_range_begin(P.total, q + 1);
+                        const uint64_t end = mqi_range_begin(C.total, q + 1);
                         if (!got) {
                             const uint64_t s0 = base + rank * chunk;
                             if (s0 < end) {
@@ -1405,26 +1586,26 @@ k_transport(transport_params P) {
             }
             L.g = g;
             uint32_t spot_id;
-            if (P.vertices) {
+            if (C.vertices) {
                 // caller-made vertex (upload_vertices path); scenario 0
-                spot_id  = P.vertex_spot ? P.vertex_spot[g] : 0;
+                spot_id  = C.vertex_spot ? C.vertex_spot[g] : 0;
                 L.item   = spot_id;
                 L.hist   = g;
                 scen     = 0;
             } else {
-                locate(P, g, L.item, L.hist);
-                spot_id = P.item_spot[L.item];
-                scen    = P.item_scenario[L.item];
+                locate(C, g, L.item, L.hist);
+                spot_id = C.item_spot[L.item];
+                scen    = C.item_scenario[L.item];
             }
-            c.g.sx                 = P.scen_shift ? P.scen_shift[3 * scen] : 0.0f;
-            c.g.sy                 = P.scen_shift ? P.scen_shift[3 * scen + 1] : 0.0f;
-            c.g.sz                 = P.scen_shift ? P.scen_shift[3 * scen + 2] : 0.0f;
-            L.scale                = P.scen_scale ? P.scen_scale[scen] : 1.0f;
+            c.g.sx                 = C.scen_shift ? C.scen_shift[3 * scen] : 0.0f;
+            c.g.sy                 = C.scen_shift ? C.scen_shift[3 * scen + 1] : 0.0f;
+            c.g.sz                 = C.scen_shift ? C.scen_shift[3 * scen + 2] : 0.0f;
+            L.scale                = C.scen_scale ? C.scen_scale[scen] : 1.0f;
             L.scen                 = scen;
-            L.dij_item             = scen * (uint32_t) P.n_spots + spot_id;
+            L.dij_item             = scen * (uint32_t) C.n_spots + spot_id;
             L.newhist              = true;
-            if (P.vertices) {
-                const float* v = P.vertices + 7 * g;
+            if (C.vertices) {
+                const float* v = C.vertices + 7 * g;
                 L.t.ke0        = v[0];
                 L.t.p0         = mk(v[1], v[2], v[3]);
                 L.t.d0         = mk(v[4], v[5], v[6]);
@@ -1436,10 +1617,10 @@ k_transport(transport_params P) {
                 L.t.stopped    = false;
                 L.t.primary    = true;
             } else {
-                sample_vertex(P, P.spots[spot_id], spot_id, scen, L.hist + hoff, L.t);
+                sample_vertex(C, C.spots[spot_id], spot_id, scen, L.hist + hoff, L.t);
             }
 #if MQI_EXACT
-            c.rng.init(P.seed, (uint32_t) (L.hist + hoff), spot_id, scen);
+            c.rng.init(C.seed, (uint32_t) (L.hist + hoff), spot_id, scen);
 #else
             c.rng.init((uint32_t) (L.hist + hoff), spot_id, scen);
 #endif
@@ -1449,7 +1630,7 @@ k_transport(transport_params P) {
             c.child   = 0;
             L.reenter = true;
         } else if (!L.active) {
-            pop(c, L.t);
+            pop(cold(), c, L.t);
             L.tsteps  = 0;
             c.child   = 0;
             L.reenter = true;
@@ -1458,16 +1639,16 @@ k_transport(transport_params P) {
         // the next child it reaches (one call site for all three)
         if (L.reenter) {
             L.reenter = false;
-            L.active  = enter_chain(P, c, L.t, shb);
+            L.active  = enter_chain(cold(), c, L.t, shb);
             if (!L.active) continue;
         }
         step<DBG, TRACE>(P, c, L, shb, pv);
         ++nstep;
     }
-    flush(P, L.acc, pv);
-    atomicAdd(P.tracked, (unsigned long long) done);
-    atomicAdd(P.steps, (unsigned long long) nstep);
-    if (c.drops) atomicAdd(P.drops, (unsigned long long) c.drops);
+    flush(P, scoring_of(P), L.acc, pv);
+    atomicAdd(cold().tracked, (unsigned long long) done);
+    atomicAdd(cold().steps, (unsigned long long) nstep);
+    if (c.drops) atomicAdd(cold().drops, (unsigned long long) c.drops);
 }
 
 namespace
