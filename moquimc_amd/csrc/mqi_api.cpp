@@ -298,39 +298,20 @@ free_dij(mqi_ctx* c) {
     c->dij.clear();
 }
 
-// CSR-Adaptive segmentation of a row pointer array: rows longer than
-// MQI_SEG_SHORT are cut into MQI_SEG_LONG pieces, shorter rows are packed
-// (MQI_SEG_SHORT entries, MQI_SEG_ROWS rows at most per segment).
+// CSR-Adaptive segmentation of a row pointer array (cut_segments)
+template<typename Idx>
 int
-build_plan(mqi_ctx* c, const std::vector<int64_t>& ip, csr_plan& P) {
+build_plan(mqi_ctx* c, const std::vector<Idx>& ip, csr_plan& P) {
     const int64_t         rows = (int64_t) ip.size() - 1;
     std::vector<int64_t>  sk;
     std::vector<uint32_t> si;
     std::vector<int32_t>  split;
     if (rows >= (1ll << 31)) return fail(c, MQI_E_ARG, "more than 2^31 - 1 rows");
-    int64_t r = 0;
-    while (r < rows) {
-        const int64_t len = ip[r + 1] - ip[r];
-        if (len > MQI_SEG_SHORT) {
-            split.push_back((int32_t) sk.size());
-            for (int64_t off = 0; off < len; off += MQI_SEG_LONG) {
-                sk.push_back(ip[r] + off);
-                si.push_back((uint32_t) r | 0x80000000u);
-            }
-            split.push_back((int32_t) sk.size());
-            ++r;
-        } else {
-            const int64_t r0 = r, kb = ip[r];
-            while (r < rows && r - r0 < MQI_SEG_ROWS && ip[r + 1] - kb <= MQI_SEG_SHORT) ++r;
-            sk.push_back(kb);
-            si.push_back((uint32_t) r0);
-        }
-        if (sk.size() >= (size_t) INT32_MAX) return fail(c, MQI_E_ARG, "too many CSR segments");
-    }
-    P.n_seg   = (int64_t) sk.size();
+    if (!cut_segments(ip.data(), rows, (int64_t) MQI_SEG_SHORT, (int64_t) MQI_SEG_LONG, (int64_t) MQI_SEG_ROWS, sk,
+                      si, split))
+        return fail(c, MQI_E_ARG, "too many CSR segments");
+    P.n_seg   = (int64_t) sk.size() - 1;
     P.n_split = (int64_t) split.size() / 2;
-    sk.push_back(ip[rows]);
-    si.push_back((uint32_t) rows);
     int e;
     if ((e = dalloc(c, &P.seg_k, sk.size())) || (e = dalloc(c, &P.seg_info, si.size())) ||
         (e = dalloc(c, &P.split_seg, std::max<size_t>(split.size(), 1))) ||
@@ -343,6 +324,57 @@ build_plan(mqi_ctx* c, const std::vector<int64_t>& ip, csr_plan& P) {
     return 0;
 }
 
+// Scratch of a matrix's build, one allocation: the list of nonzeros (voxel;
+// row, value) and the sort's second copy, 24 bytes per nonzero
+struct build_ws {
+    char*     base    = nullptr;
+    uint32_t *vox     = nullptr, *vox2    = nullptr;   // nnz
+    uint64_t *packed  = nullptr, *packed2 = nullptr;   // nnz
+    uint32_t *heads   = nullptr;                       // tiles + 1
+    uint32_t *tptr32  = nullptr;                       // min(nnz, cols) + 1
+    char*     sort    = nullptr;
+    size_t    sort_bytes = 0;
+    ~build_ws() { hipFree(base); }
+};
+
+int
+bits_for(int64_t n) {   // of the indices below n
+    int b = 1;
+    while (b < 32 && (1ll << b) < n) ++b;
+    return b;
+}
+
+// for a matrix of up to nnz nonzeros (nnz > 0)
+int
+build_scratch(mqi_ctx* c, build_ws& ws, int64_t rows, int64_t cols, int64_t nnz) {
+    size_t b1 = 0, b2 = 0;
+    KCHK(c, mqi_aux::sort_pairs(nullptr, nullptr, nullptr, nullptr, nnz, bits_for(cols), nullptr, &b1, nullptr,
+                                c->stream));
+    KCHK(c, mqi_aux::sort_pairs(nullptr, nullptr, nullptr, nullptr, nnz, bits_for(rows), nullptr, &b2, nullptr,
+                                c->stream));
+    size_t at   = 0;
+    auto   take = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) & ~(size_t) 255;
+        return o;
+    };
+    const size_t n = (size_t) nnz, tiles = (n + MQI_TILE - 1) / MQI_TILE;
+    const size_t o_v = take(4 * n), o_v2 = take(4 * n), o_p = take(8 * n), o_p2 = take(8 * n);
+    const size_t o_h = take(4 * (tiles + 1) + 8), o_t = take(4 * ((size_t) std::min(nnz, cols) + 1));
+    ws.sort_bytes    = std::max<size_t>(std::max(b1, b2), 1);
+    const size_t o_s = take(ws.sort_bytes);
+    const int    r   = dalloc(c, &ws.base, at);
+    if (r) return r;
+    ws.vox     = (uint32_t*) (ws.base + o_v);
+    ws.vox2    = (uint32_t*) (ws.base + o_v2);
+    ws.packed  = (uint64_t*) (ws.base + o_p);
+    ws.packed2 = (uint64_t*) (ws.base + o_p2);
+    ws.heads   = (uint32_t*) (ws.base + o_h);
+    ws.tptr32  = (uint32_t*) (ws.base + o_t);
+    ws.sort    = ws.base + o_s;
+    return 0;
+}
+
 // The pieces of D^T g over column deltas (mqi_aux::pieces_staged): the
 // 16-bit deltas of the compacted columns, and the positions where a row
 // skips more than 65535 columns, come from the device; each row is cut there
@@ -350,97 +382,82 @@ build_plan(mqi_ctx* c, const std::vector<int64_t>& ip, csr_plan& P) {
 // whole lane-major batches with one byte per delta (the deltas of 255 and
 // more in per-piece escape lists) and ordered by their first columns.
 int
-build_pieces(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& ip) {
+build_pieces(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& ip, const build_ws& ws) {
+    // the sorts are done: the columns are in vox, the deltas go to packed and
+    // the gaps to packed2 (as many as there are nonzeros fit)
     const int64_t       rows   = m.rows;
-    unsigned long long* d_ngap = nullptr;
-    int64_t *           d_gaps = nullptr, *d_pk = nullptr;
-    uint16_t*           d_dcol = nullptr;
+    const int32_t*      d_ccol = (const int32_t*) ws.vox;
+    uint16_t*           d_dcol = (uint16_t*) ws.packed;
+    unsigned long long* d_ngap = (unsigned long long*) ws.heads;
     int                 r      = 0;
-    struct guard {
-        unsigned long long*& n;
-        int64_t *&           g, *&k;
-        uint16_t*&           d;
-        ~guard() {
-            hipFree(n);
-            hipFree(g);
-            hipFree(k);
-            hipFree(d);
-        }
-    } g{ d_ngap, d_gaps, d_pk, d_dcol };
-    int64_t cap = 1 << 16;
-    if ((r = dalloc(c, &d_dcol, m.nnz)) || (r = dalloc(c, &d_ngap, 1)) || (r = dalloc(c, &d_gaps, cap))) return r;
-    unsigned long long n_gaps = 0;
-    for (int pass = 0; pass < 2; ++pass) {
-        KCHK(c, mqi_aux::deltas16(m.indptr, m.ccol, rows, m.nnz, d_dcol, d_ngap, d_gaps, cap, c->stream));
-        HIPCHK(c, hipMemcpy(&n_gaps, d_ngap, sizeof n_gaps, hipMemcpyDeviceToHost));
-        if ((int64_t) n_gaps <= cap) break;
-        hipFree(d_gaps);
-        d_gaps = nullptr;
-        cap    = (int64_t) n_gaps;
-        if ((r = dalloc(c, &d_gaps, cap))) return r;
-    }
+    unsigned long long  n_gaps = 0;
+    KCHK(c, mqi_aux::deltas16(m.indptr, d_ccol, rows, m.nnz, d_dcol, d_ngap, (int64_t*) ws.packed2, m.nnz, c->stream));
+    HIPCHK(c, hipMemcpy(&n_gaps, d_ngap, sizeof n_gaps, hipMemcpyDeviceToHost));
     std::vector<int64_t> gaps(n_gaps);
-    if (n_gaps) HIPCHK(c, hipMemcpy(gaps.data(), d_gaps, sizeof(int64_t) * n_gaps, hipMemcpyDeviceToHost));
+    if (n_gaps) HIPCHK(c, hipMemcpy(gaps.data(), ws.packed2, sizeof(int64_t) * n_gaps, hipMemcpyDeviceToHost));
     std::sort(gaps.begin(), gaps.end());
     std::vector<int64_t> pk;
     std::vector<int32_t> row_piece;
     if (!cut_pieces(ip, gaps, MQI_PIECE, pk, row_piece)) return fail(c, MQI_E_ARG, "too many Dij pieces");
-    m.n_piece = (int64_t) pk.size() - 1;
-    std::vector<int64_t> pb(m.n_piece + 1, 0);
-    for (int64_t i = 0; i < m.n_piece; ++i) pb[i + 1] = pb[i] + ((pk[i + 1] - pk[i] + 255) & ~(int64_t) 255);
-    if ((pb.back() >> 8) > (int64_t) UINT32_MAX) return fail(c, MQI_E_CAPACITY, "too many Dij batches");
-    int32_t*  d_base = nullptr;
-    int64_t*  d_pb   = nullptr;
-    uint32_t* d_ecnt = nullptr;
-    struct guard2 {
-        int32_t*&  b;
-        int64_t*&  p;
-        uint32_t*& e;
-        ~guard2() {
-            hipFree(b);
-            hipFree(p);
-            hipFree(e);
-        }
-    } g2{ d_base, d_pb, d_ecnt };
-    const int64_t np1 = std::max<int64_t>(m.n_piece, 1);
-    if ((r = dalloc(c, &d_pk, pk.size())) || (r = dalloc(c, &d_base, np1)) || (r = dalloc(c, &d_ecnt, np1)) ||
-        (r = dalloc(c, &m.row_piece, rows + 1)) || (r = dalloc(c, &m.ppart, np1)) ||
-        (r = dalloc(c, &d_pb, pb.size())) || (r = dalloc(c, &m.sval, std::max<int64_t>(pb.back(), 1))) ||
-        (r = dalloc(c, &m.sd8, std::max<int64_t>(pb.back(), 1))) || (r = dalloc(c, &m.phdr, np1)))
+    m.n_piece         = (int64_t) pk.size() - 1;
+    const size_t np   = (size_t) m.n_piece;
+    // the pieces' tables go to the device in one copy: first nonzeros (np +
+    // 1), staged starts (np + 1), then first columns and escapes per piece
+    pk.resize(2 * (np + 1), 0);
+    int64_t* pb = pk.data() + np + 1;
+    for (size_t i = 0; i < np; ++i) pb[i + 1] = pb[i] + ((pk[i + 1] - pk[i] + 255) & ~(int64_t) 255);
+    const int64_t staged = pb[np];
+    if ((staged >> 8) > (int64_t) UINT32_MAX) return fail(c, MQI_E_CAPACITY, "too many Dij batches");
+    struct guard {
+        int64_t* p = nullptr;
+        ~guard() { hipFree(p); }
+    } own;
+    int64_t* d_pk = (int64_t*) ws.packed2;
+    if (3 * (np + 1) > (size_t) m.nnz) {
+        if ((r = dalloc(c, &own.p, 3 * (np + 1)))) return r;
+        d_pk = own.p;
+    }
+    int64_t*     d_pb   = d_pk + np + 1;
+    int32_t*     d_base = (int32_t*) (d_pb + np + 1);
+    uint32_t*    d_ecnt = (uint32_t*) d_base + np;
+    const size_t np1    = std::max<size_t>(np, 1);
+    if ((r = dalloc(c, &m.row_piece, rows + 1)) || (r = dalloc(c, &m.ppart, np1)) ||
+        (r = dalloc(c, &m.sval, std::max<int64_t>(staged, 1))) ||
+        (r = dalloc(c, &m.sd8, std::max<int64_t>(staged, 1))) || (r = dalloc(c, &m.phdr, np1)))
         return r;
     HIPCHK(c, hipMemcpy(d_pk, pk.data(), sizeof(int64_t) * pk.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(m.row_piece, row_piece.data(), sizeof(int32_t) * (rows + 1), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(d_pb, pb.data(), sizeof(int64_t) * pb.size(), hipMemcpyHostToDevice));
-    KCHK(c, mqi_aux::piece_base(m.ccol, d_dcol, d_pk, m.n_piece, d_base, c->stream));
-    // escapes (deltas of 255 and more): counted per piece, their lists placed
-    // by the exclusive prefix sum, padded by the 64 entries the product may
-    // read past the last one
-    std::vector<uint32_t> ecnt(m.n_piece), ebase(np1, 0);
-    if (m.n_piece) {
+    // first columns, and the escapes (deltas of 255 and more) counted per
+    // piece; their lists are placed by the exclusive prefix sum and padded by
+    // the 64 entries the product may read past the last one
+    std::vector<int32_t>  table(2 * np1, 0);   // first columns, escapes
+    std::vector<uint32_t> ebase(np1, 0);
+    if (np) {
+        KCHK(c, mqi_aux::piece_base(d_ccol, d_dcol, d_pk, m.n_piece, d_base, c->stream));
         KCHK(c, mqi_aux::piece_escapes(d_dcol, d_pk, m.n_piece, d_ecnt, c->stream));
-        HIPCHK(c, hipMemcpy(ecnt.data(), d_ecnt, sizeof(uint32_t) * m.n_piece, hipMemcpyDeviceToHost));
+        HIPCHK(c, hipMemcpy(table.data(), d_base, sizeof(int32_t) * 2 * np, hipMemcpyDeviceToHost));
     }
-    uint64_t n_esc = 0;
-    for (int64_t i = 0; i < m.n_piece; ++i) {
+    const int32_t* first = table.data();
+    uint64_t       n_esc = 0;
+    for (size_t i = 0; i < np; ++i) {
         ebase[i] = (uint32_t) n_esc;
-        n_esc += ecnt[i];
+        n_esc += (uint32_t) table[np + i];
     }
     if (n_esc + 64 > (uint64_t) UINT32_MAX) return fail(c, MQI_E_CAPACITY, "too many Dij escapes");
     const uint64_t n_esc_alloc = (n_esc + 64 + 1) & ~(uint64_t) 1;
     if ((r = dalloc(c, &m.pesc, n_esc_alloc))) return r;
     KCHK(c, mqi_aux::fill_u32(m.pesc, 0u, n_esc_alloc / 2, c->stream));
-    if (m.n_piece) HIPCHK(c, hipMemcpy(d_ecnt, ebase.data(), sizeof(uint32_t) * m.n_piece, hipMemcpyHostToDevice));
+    if (np) HIPCHK(c, hipMemcpy(d_ecnt, ebase.data(), sizeof(uint32_t) * np, hipMemcpyHostToDevice));
     KCHK(c, mqi_aux::stage_pieces(m.val, d_dcol, d_pk, d_pb, d_ecnt, m.n_piece, m.sval, m.sd8, m.pesc, c->stream));
     // processed in the order of their first columns: the pieces that run at
     // the same time gather from the same stretch of x (7 % faster on the
     // 5000-spot Dij than row order); one 32-byte header per piece in that
     // order, so a wave starts a piece after one round trip
-    std::vector<int32_t> first(m.n_piece), order(m.n_piece);
-    if (m.n_piece) HIPCHK(c, hipMemcpy(first.data(), d_base, sizeof(int32_t) * m.n_piece, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < m.n_piece; ++i) order[i] = (int32_t) i;
+    std::vector<int32_t> order(np);
+    for (size_t i = 0; i < np; ++i) order[i] = (int32_t) i;
     std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return first[a] < first[b]; });
-    std::vector<mqi_aux::piece_hdr> hdr(m.n_piece);
-    for (int64_t i = 0; i < m.n_piece; ++i) {
+    std::vector<mqi_aux::piece_hdr> hdr(np);
+    for (size_t i = 0; i < np; ++i) {
         const int32_t q = order[i];
         hdr[i].batch0   = (uint32_t) (pb[q] >> 8);
         hdr[i].batches  = (uint32_t) ((pb[q + 1] - pb[q]) >> 8);
@@ -449,8 +466,7 @@ build_pieces(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& ip) {
         hdr[i].esc0     = ebase[q];
         hdr[i].pad[0] = hdr[i].pad[1] = hdr[i].pad[2] = 0;
     }
-    if (m.n_piece)
-        HIPCHK(c, hipMemcpy(m.phdr, hdr.data(), sizeof(mqi_aux::piece_hdr) * m.n_piece, hipMemcpyHostToDevice));
+    if (np) HIPCHK(c, hipMemcpy(m.phdr, hdr.data(), sizeof(mqi_aux::piece_hdr) * np, hipMemcpyHostToDevice));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -1640,106 +1656,53 @@ mqi_stat(mqi_ctx* c, int scenario, uint64_t n, float thr, double* out) {
     return stat_value(c, scenario, n, thr, out);
 }
 
-// The product structures of a CSR on the device (m.indptr, m.col, m.val set;
-// indptr its row pointers on the host): rows sorted by column (unless they
-// are already), the voxel-major copy and plan of D w, the compacted columns
-// of D^T g and, for long rows, its pieces.
+// The product structures of a matrix (m.indptr set, its row pointers indptr
+// also on the host, m.col and m.val allocated) from its nonzeros in ws.vox /
+// ws.packed, rows ascending: the voxel-major copy and plan of D w, the rows
+// sorted by voxel, and for D^T g their compacted columns and plan or, for
+// long rows, their pieces.
 int
-prepare_products(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& indptr, bool sort_rows) {
+prepare_products(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& indptr, build_ws& ws) {
     int r = 0;
-    if ((r = build_plan(c, indptr, m.plan))) return r;
-    if (m.nnz > 0) {
-        // sort every row by voxel (rows handed in by the caller are checked
-        // sorted instead)
-        if (sort_rows) {
-            // the segmented radix sort counts items in 32 bits
-            if (m.nnz > (int64_t) INT32_MAX)
-                return fail(c, MQI_E_CAPACITY, "%lld nonzeros in one Dij exceed the row sort's 2^31 - 1",
-                            (long long) m.nnz);
-            int32_t* tk = nullptr;
-            float*   tv = nullptr;
-            if ((r = dalloc(c, &tk, m.nnz)) || (r = dalloc(c, &tv, m.nnz))) return r;
-            size_t bytes = 0;
-            KCHK(c, mqi_aux::segmented_sort(m.col, m.val, tk, tv, m.nnz, (int) m.rows, m.indptr, m.indptr + 1,
-                                            nullptr, &bytes, c->stream));
-            char* scratch = nullptr;
-            if ((r = dalloc(c, &scratch, std::max<size_t>(bytes, 1)))) return r;
-            KCHK(c, mqi_aux::segmented_sort(m.col, m.val, tk, tv, m.nnz, (int) m.rows, m.indptr, m.indptr + 1,
-                                            scratch, &bytes, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-            hipFree(scratch);
-            hipFree(tk);
-            hipFree(tv);
-        }
-        // voxel-major copy for D w: row lengths by counting, entries by a
-        // stable sort on the voxel (each voxel's spots ascending); its rows
-        // are the voxels with a nonzero only (D w zeroes the others)
-        uint32_t* d_cc = nullptr;
-        if ((r = dalloc(c, &d_cc, m.cols)) || (r = dalloc(c, &m.tcol, m.nnz)) || (r = dalloc(c, &m.tval, m.nnz)))
-            return r;
-        KCHK(c, mqi_aux::fill_u32(d_cc, 0u, m.cols, c->stream));
-        KCHK(c, mqi_aux::csr_transpose_count(m.col, m.nnz, d_cc, c->stream));
-        std::vector<uint32_t> cc(m.cols);
-        HIPCHK(c, hipMemcpy(cc.data(), d_cc, sizeof(uint32_t) * m.cols, hipMemcpyDeviceToHost));
-        // voxels with a nonzero (the rows of the voxel-major copy and the
-        // compacted gather of D^T g), each one's rank, and their bitmask
-        std::vector<int32_t>  nz, rank(m.cols, 0);
-        std::vector<int64_t>  tptr(1, 0);
-        std::vector<uint32_t> bits((m.cols + 31) / 32, 0u);
-        for (int64_t v = 0; v < m.cols; ++v)
-            if (cc[v]) {
-                rank[v] = (int32_t) nz.size();
-                nz.push_back((int32_t) v);
-                tptr.push_back(tptr.back() + cc[v]);
-                bits[v >> 5] |= 1u << (v & 31);
-            }
-        m.n_nz = (int64_t) nz.size();
-        if ((r = dalloc(c, &m.tindptr, m.n_nz + 1)) || (r = dalloc(c, &m.tnonempty, bits.size()))) return r;
-        HIPCHK(c, hipMemcpy(m.tindptr, tptr.data(), sizeof(int64_t) * (m.n_nz + 1), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(m.tnonempty, bits.data(), sizeof(uint32_t) * bits.size(), hipMemcpyHostToDevice));
-        if ((r = build_plan(c, tptr, m.tplan))) return r;
-        int32_t* d_rank = nullptr;
-        if ((r = dalloc(c, &m.nzvox, m.n_nz)) || (r = dalloc(c, &m.ccol, m.nnz)) || (r = dalloc(c, &m.xc, m.n_nz)) ||
-            (r = dalloc(c, &d_rank, m.cols)))
-            return r;
-        HIPCHK(c, hipMemcpy(m.nzvox, nz.data(), sizeof(int32_t) * m.n_nz, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(d_rank, rank.data(), sizeof(int32_t) * m.cols, hipMemcpyHostToDevice));
-        KCHK(c, mqi_aux::renumber(m.col, m.nnz, d_rank, m.ccol, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        hipFree(d_rank);
-        // long rows (the Dij of pencil beams): D^T g over byte column deltas
-        if (m.nnz >= (int64_t) MQI_SEG_SHORT * m.rows) {
-            if ((r = build_pieces(c, m, indptr))) return r;
-            dfree(m.ccol);
-        }
-        int key_bits = 1;
-        while (key_bits < 32 && (1ll << key_bits) < m.cols) ++key_bits;
-        int32_t*  d_keys = nullptr;
-        uint64_t *d_pk = nullptr, *d_pk2 = nullptr;
-        char*     d_tmp = nullptr;
-        size_t    tbytes = 0;
-        KCHK(c, mqi_aux::csr_transpose_sorted(m.indptr, m.col, m.val, m.rows, m.nnz, key_bits, nullptr, nullptr,
-                                              nullptr, nullptr, nullptr, nullptr, &tbytes, c->stream));
-        if ((r = dalloc(c, &d_keys, m.nnz)) || (r = dalloc(c, &d_pk, m.nnz)) || (r = dalloc(c, &d_pk2, m.nnz)) ||
-            (r = dalloc(c, &d_tmp, std::max<size_t>(tbytes, 1))))
-            return r;
-        KCHK(c, mqi_aux::csr_transpose_sorted(m.indptr, m.col, m.val, m.rows, m.nnz, key_bits, d_keys, d_pk, d_pk2,
-                                              m.tcol, m.tval, d_tmp, &tbytes, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        hipFree(d_keys);
-        hipFree(d_pk);
-        hipFree(d_pk2);
-        hipFree(d_tmp);
-        hipFree(d_cc);
-        // D w over 16-bit spot columns
-        if (m.rows <= 65536) {
-            if ((r = dalloc(c, &m.tcol16, m.nnz))) return r;
-            KCHK(c, mqi_aux::low16(m.tcol, m.nnz, m.tcol16, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-            dfree(m.tcol);
-        }
+    if (m.nnz == 0) return build_plan(c, indptr, m.plan);
+    int tmp = 0;
+    KCHK(c, mqi_aux::sort_pairs(ws.vox, ws.vox2, ws.packed, ws.packed2, m.nnz, bits_for(m.cols), ws.sort,
+                                &ws.sort_bytes, &tmp, c->stream));
+    if (tmp) {
+        std::swap(ws.vox, ws.vox2);
+        std::swap(ws.packed, ws.packed2);
     }
-    return 0;
+    // the voxels with a nonzero (the rows of the voxel-major copy and the
+    // compacted gather of D^T g)
+    KCHK(c, mqi_aux::tile_heads(ws.vox, m.nnz, ws.heads, c->stream));
+    uint32_t n_nz = 0;
+    HIPCHK(c, hipMemcpy(&n_nz, ws.heads + (m.nnz + MQI_TILE - 1) / MQI_TILE, sizeof n_nz, hipMemcpyDeviceToHost));
+    m.n_nz = (int64_t) n_nz;
+    // D w over 16-bit spot columns where they fit
+    if ((r = m.rows <= 65536 ? dalloc(c, &m.tcol16, m.nnz) : dalloc(c, &m.tcol, m.nnz)) ||
+        (r = dalloc(c, &m.tval, m.nnz)) || (r = dalloc(c, &m.tindptr, m.n_nz + 1)) ||
+        (r = dalloc(c, &m.tnonempty, (m.cols + 31) / 32)) || (r = dalloc(c, &m.nzvox, m.n_nz)) ||
+        (r = dalloc(c, &m.xc, m.n_nz)))
+        return r;
+    KCHK(c, mqi_aux::voxel_rows(ws.vox, ws.packed, m.nnz, ws.heads, m.nzvox, m.tindptr, ws.tptr32, m.tnonempty,
+                                m.cols, m.tcol16, m.tcol, m.tval, ws.vox2, ws.packed2, c->stream));
+    // back to the rows, now in voxel order
+    KCHK(c, mqi_aux::sort_pairs(ws.vox2, ws.vox, ws.packed2, ws.packed, m.nnz, bits_for(m.rows), ws.sort,
+                                &ws.sort_bytes, &tmp, c->stream));
+    if (!tmp) {
+        std::swap(ws.vox, ws.vox2);
+        std::swap(ws.packed, ws.packed2);
+    }
+    // long rows (the Dij of pencil beams): D^T g over byte column deltas
+    const bool pieces = m.nnz >= (int64_t) MQI_SEG_SHORT * m.rows;
+    if (!pieces && (r = dalloc(c, &m.ccol, m.nnz))) return r;
+    KCHK(c, mqi_aux::spot_rows(ws.packed, m.nzvox, m.nnz, m.col, pieces ? (int32_t*) ws.vox : m.ccol, m.val,
+                               c->stream));
+    std::vector<uint32_t> tptr(m.n_nz + 1);
+    HIPCHK(c, hipMemcpy(tptr.data(), ws.tptr32, sizeof(uint32_t) * (m.n_nz + 1), hipMemcpyDeviceToHost));
+    if ((r = build_plan(c, tptr, m.tplan))) return r;
+    if (pieces) return build_pieces(c, m, indptr, ws);
+    return build_plan(c, indptr, m.plan);
 }
 
 int
@@ -1751,38 +1714,70 @@ mqi_dij_build(mqi_ctx* c, double rel_thr) {
         return fail(c, MQI_E_STATE, "the spots or scenarios changed since the run that scored the Dij tables");
     hipSetDevice(c->device);
     free_dij(c);
-    const uint32_t n_items = (uint32_t) c->dij_items;
-    const int      n_spots = (int) c->spots.size();
-    double*        d_max   = nullptr;
-    uint32_t*      d_cnt   = nullptr;
-    if ((r = dalloc(c, &d_max, n_items)) || (r = dalloc(c, &d_cnt, n_items))) return r;
-    KCHK(c, mqi_aux::dij_compact(c->d_dij_keys, c->d_dij_vals, c->d_dij_off, n_items, rel_thr, d_max, d_cnt,
-                                 c->stream));
-    std::vector<uint32_t> cnt(n_items);
-    HIPCHK(c, hipMemcpy(cnt.data(), d_cnt, sizeof(uint32_t) * n_items, hipMemcpyDeviceToHost));
+    const uint32_t n_items = (uint32_t) c->dij_items, n_spots = (uint32_t) c->spots.size();
+    // workgroups per table: a few per CU in all, of 2048 slots at least
+    const uint64_t slots  = c->dij_off[n_items];
+    const uint32_t chunks = (uint32_t) std::max<uint64_t>(
+      1, std::min<uint64_t>((8192 + n_items - 1) / n_items, slots / n_items / 2048));
+    struct tables {
+        double*   max   = nullptr;   // per item
+        uint32_t* count = nullptr;   // per chunk: entries, then the first place
+        ~tables() {
+            hipFree(max);
+            hipFree(count);
+        }
+    } d;
+    const size_t n_chunks = (size_t) n_items * chunks;
+    if ((r = dalloc(c, &d.max, n_items)) || (r = dalloc(c, &d.count, n_chunks))) return r;
+    KCHK(c, mqi_aux::dij_count(c->d_dij_vals, c->d_dij_off, n_items, chunks, rel_thr, d.max, d.count, c->stream));
+    std::vector<uint32_t> cnt(n_chunks);
+    HIPCHK(c, hipMemcpy(cnt.data(), d.count, sizeof(uint32_t) * n_chunks, hipMemcpyDeviceToHost));
+    // row pointers and the chunks' first places, per scenario
+    std::vector<std::vector<int64_t>> indptr(c->n_scen, std::vector<int64_t>(n_spots + 1, 0));
+    int64_t                           most = 0;
+    size_t                            at   = 0;
+    for (int s = 0; s < c->n_scen; ++s) {
+        int64_t nnz = 0;
+        for (uint32_t j = 0; j < n_spots; ++j) {
+            for (uint32_t k = 0; k < chunks; ++k, ++at) {
+                const uint32_t n = cnt[at];
+                cnt[at]          = (uint32_t) nnz;
+                nnz += n;
+            }
+            indptr[s][j + 1] = nnz;
+        }
+        if ((r = dij_size_check(nnz)))
+            return fail(c, r, "scenario %d's Dij has %lld nonzeros: its rows are sorted with 32-bit counts "
+                              "(at most %lld); raise the threshold or split the plan", s, (long long) nnz,
+                        (long long) MQI_MAX_SORT_NNZ);
+        most = std::max(most, nnz);
+    }
+    HIPCHK(c, hipMemcpy(d.count, cnt.data(), sizeof(uint32_t) * n_chunks, hipMemcpyHostToDevice));
+    build_ws ws;
+    if (most && (r = build_scratch(c, ws, n_spots, (int64_t) nvox(c), most))) return r;
     c->dij.resize(c->n_scen);
     for (int s = 0; s < c->n_scen; ++s) {
         csr_dev& m = c->dij[s];
         m.rows     = n_spots;
         m.cols     = (int64_t) nvox(c);
-        std::vector<int64_t> indptr(n_spots + 1, 0);
-        for (int j = 0; j < n_spots; ++j) indptr[j + 1] = indptr[j] + cnt[(size_t) s * n_spots + j];
-        m.nnz = indptr[n_spots];
-        if ((r = dij_size_check(m.nnz)))
-            return fail(c, r, "scenario %d's Dij has %lld nonzeros: its rows are sorted with 32-bit counts "
-                              "(at most %lld); raise the threshold or split the plan", s, (long long) m.nnz,
-                        (long long) MQI_MAX_SORT_NNZ);
+        m.nnz      = indptr[s][n_spots];
         if ((r = dalloc(c, &m.indptr, n_spots + 1)) || (r = dalloc(c, &m.col, std::max<int64_t>(1, m.nnz))) ||
             (r = dalloc(c, &m.val, std::max<int64_t>(1, m.nnz))))
-            return r;
-        HIPCHK(c, hipMemcpy(m.indptr, indptr.data(), sizeof(int64_t) * (n_spots + 1), hipMemcpyHostToDevice));
-        KCHK(c, mqi_aux::dij_write(c->d_dij_keys, c->d_dij_vals, c->d_dij_off + (size_t) s * n_spots, n_spots, rel_thr,
-                                   d_max + (size_t) s * n_spots, m.indptr, m.col, m.val, c->stream));
-        if ((r = prepare_products(c, m, indptr, true))) return r;
+            break;
+        hipError_t e = hipMemcpy(m.indptr, indptr[s].data(), sizeof(int64_t) * (n_spots + 1), hipMemcpyHostToDevice);
+        if (e == hipSuccess && m.nnz)
+            e = (hipError_t) mqi_aux::dij_write(c->d_dij_keys, c->d_dij_vals, c->d_dij_off, (uint32_t) s * n_spots,
+                                                n_spots, chunks, d.max, rel_thr, d.count, ws.vox, ws.packed,
+                                                c->stream);
+        if (e != hipSuccess) {
+            r = fail(c, MQI_E_HIP, "Dij build: %s", hipGetErrorString(e));
+            break;
+        }
+        if ((r = prepare_products(c, m, indptr[s], ws))) break;
     }
-    hipFree(d_max);
-    hipFree(d_cnt);
-    return 0;
+    // a matrix without all its product structures is no matrix
+    if (r) free_dij(c);
+    return r;
 }
 
 int
@@ -1815,11 +1810,17 @@ mqi_dij_set_csr(mqi_ctx* c, int s, int64_t rows, int64_t cols, const int64_t* in
         return r;
     std::vector<int64_t> ip(indptr, indptr + rows + 1);
     HIPCHK(c, hipMemcpy(m.indptr, ip.data(), sizeof(int64_t) * (rows + 1), hipMemcpyHostToDevice));
+    build_ws ws;
     if (nnz) {
-        HIPCHK(c, hipMemcpy(m.col, indices, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
+        if ((r = build_scratch(c, ws, rows, cols, nnz))) {
+            free_csr(m);
+            return r;
+        }
+        HIPCHK(c, hipMemcpy(ws.vox, indices, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(m.val, values, sizeof(float) * nnz, hipMemcpyHostToDevice));
+        KCHK(c, mqi_aux::pack_rows(m.indptr, m.val, rows, ws.packed, c->stream));
     }
-    if ((r = prepare_products(c, m, ip, false))) {
+    if ((r = prepare_products(c, m, ip, ws))) {
         free_csr(m);
         return r;
     }

@@ -23,13 +23,32 @@ int scale(double* p, uint64_t n, double w, hipStream_t s);
 // dose += w * (stat - snap) outside voxel 0 of each block of nvox
 int dose_from_stat(double* dose, const double* stat, const double* snap, uint64_t n, uint64_t nvox, double w,
                    hipStream_t s);
-int dij_compact(const uint32_t* keys, const double* vals, const uint64_t* off, uint32_t n_items, double rel_thr,
-                double* item_max, uint32_t* counts, hipStream_t s);
-int dij_write(const uint32_t* keys, const double* vals, const uint64_t* off, uint32_t n_items, double rel_thr,
-              const double* item_max, const int64_t* row_start, int32_t* cols, float* out_vals, hipStream_t s);
-int segmented_sort(int32_t* keys, float* vals, int32_t* keys_tmp, float* vals_tmp, int64_t nnz, int n_seg,
-                   const int64_t* seg_begin, const int64_t* seg_end, void* scratch, size_t* scratch_bytes,
-                   hipStream_t s);
+// Dij tables into (voxel; spot, value) lists (mqi_aux.hip): each item's
+// maximum and the entries >= rel_thr * max of each of its chunks, then a
+// scenario's entries from each chunk's place (start)
+int dij_count(const double* vals, const uint64_t* off, uint32_t n_items, uint32_t chunks, double rel_thr,
+              double* item_max, uint32_t* counts, hipStream_t s);
+int dij_write(const uint32_t* keys, const double* vals, const uint64_t* off, uint32_t item0, uint32_t n_spots,
+              uint32_t chunks, const double* item_max, double rel_thr, const uint32_t* start, uint32_t* vox,
+              uint64_t* packed, hipStream_t s);
+// a CSR's values with their rows: packed[k] = (row, value) of nonzero k
+int pack_rows(const int64_t* indptr, const float* val, int64_t n_rows, uint64_t* packed, hipStream_t s);
+// stable radix sort of n (key; 64-bit value) pairs by the low `bits` of the
+// key; the result is in the tmp arrays if *in_tmp.  With scratch NULL only
+// *scratch_bytes is set.
+int sort_pairs(uint32_t* keys, uint32_t* keys_tmp, uint64_t* vals, uint64_t* vals_tmp, int64_t n, int bits,
+               void* scratch, size_t* scratch_bytes, int* in_tmp, hipStream_t s);
+// keys sorted by voxel: the voxels that begin before each tile of MQI_TILE
+// keys, and (heads[tiles]) in all
+#define MQI_TILE 4096
+int tile_heads(const uint32_t* key, int64_t n, uint32_t* heads, hipStream_t s);
+// the voxel-major copy of (voxel; spot, value) sorted by voxel, and (spot;
+// rank, value) for the sort back; tcol16 or tcol is written
+int voxel_rows(const uint32_t* key, const uint64_t* packed, int64_t n, const uint32_t* heads, int32_t* nzvox,
+               int64_t* tptr, uint32_t* tptr32, uint32_t* bits, int64_t cols, uint16_t* tcol16, int32_t* tcol,
+               float* tval, uint32_t* spot, uint64_t* ranked, hipStream_t s);
+int spot_rows(const uint64_t* ranked, const int32_t* nzvox, int64_t n, int32_t* col, int32_t* ccol, float* val,
+              hipStream_t s);
 // CSR-Adaptive segment sizes (entries of one long-row piece; entries and rows
 // of one packed segment)
 #define MQI_SEG_LONG 16384
@@ -110,19 +129,8 @@ struct alignas(16) piece_hdr {
 int pieces_staged(const float* sval, const uint8_t* sd8, const uint16_t* esc, const float* x, const piece_hdr* hdr,
                   int64_t n_p, const int32_t* row_piece, int64_t rows, double* part, void* y, int y_is_double,
                   double alpha, int accumulate, hipStream_t s);
-// low 16 bits of int32 columns (D w over at most 65536 spots)
-int low16(const int32_t* col, int64_t nnz, uint16_t* out, hipStream_t s);
-// D^T g on compacted x: xc = x[nzvox]; ccol = rank[col]
+// D^T g on compacted x: xc = x[nzvox]
 int gather_x(const float* x, const int32_t* nzvox, int64_t n, float* xc, hipStream_t s);
-int renumber(const int32_t* col, int64_t nnz, const int32_t* rank, int32_t* ccol, hipStream_t s);
-int csr_transpose_count(const int32_t* col, int64_t nnz, uint32_t* cnt, hipStream_t s);
-// voxel-major copy (tcol = spot, tval) with each voxel's spots ascending:
-// stable radix sort of the nonzeros by voxel (key_bits bits); with scratch
-// NULL only *scratch_bytes is set.  keys_tmp: nnz ints, packed / packed_tmp:
-// nnz 64-bit words.
-int csr_transpose_sorted(const int64_t* indptr, const int32_t* col, const float* val, int64_t n_rows, int64_t nnz,
-                         int key_bits, int32_t* keys_tmp, uint64_t* packed, uint64_t* packed_tmp, int32_t* tcol,
-                         float* tval, void* scratch, size_t* scratch_bytes, hipStream_t s);
 // grouped scoring: out[s][i] += pair[stride i + s] for s < ns, i < n (stride
 // 2 or 4), pair cleared
 int pair_fold(double* const* out, int ns, int stride, double* pair, uint64_t n, hipStream_t s);

@@ -44,6 +44,42 @@ cut_pieces(const std::vector<int64_t>& ip, const std::vector<int64_t>& gaps, int
     return true;
 }
 
+// CSR-Adaptive segments of the row pointers ip[0..rows] (Idx: 32 or 64 bits):
+// a row of more than `shrt` nonzeros is cut into `lng`-nonzero pieces (their
+// segments in split: first, one past the last), shorter rows are packed, at
+// most `shrt` nonzeros and `max_rows` rows a segment.  sk: first nonzero of
+// each segment plus ip[rows]; si: its first row (bit 31: a piece of a long
+// row) plus rows.  A packed segment ends at the last row that fits: found by
+// bisection, not row by row (540 k rows of a field's voxel-major matrix: 0.4
+// ms).  Returns false when the segments would not fit int32.
+template<typename Idx>
+static inline bool
+cut_segments(const Idx* ip, int64_t rows, int64_t shrt, int64_t lng, int64_t max_rows, std::vector<int64_t>& sk,
+             std::vector<uint32_t>& si, std::vector<int32_t>& split) {
+    int64_t r = 0;
+    while (r < rows) {
+        const int64_t kb = (int64_t) ip[r], len = (int64_t) ip[r + 1] - kb;
+        if (len > shrt) {
+            split.push_back((int32_t) sk.size());
+            for (int64_t off = 0; off < len; off += lng) {
+                sk.push_back(kb + off);
+                si.push_back((uint32_t) r | 0x80000000u);
+            }
+            split.push_back((int32_t) sk.size());
+            ++r;
+        } else {
+            sk.push_back(kb);
+            si.push_back((uint32_t) r);
+            const Idx* e = ip + std::min(rows, r + max_rows) + 1;
+            r = (std::upper_bound(ip + r + 1, e, (Idx) (kb + shrt)) - ip) - 1;
+        }
+        if (sk.size() >= (size_t) INT32_MAX) return false;
+    }
+    sk.push_back((int64_t) ip[rows]);
+    si.push_back((uint32_t) rows);
+    return true;
+}
+
 // A CSR handed in by a caller (rows x cols, row pointers ip[0..rows], column
 // indices idx[0 .. ip[rows])): 0 when ip starts at 0 and does not decrease
 // and every row's columns lie in [0, cols) and ascend strictly; else 1 (ip,
