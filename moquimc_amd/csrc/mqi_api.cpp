@@ -111,6 +111,9 @@ struct mqi_ctx {
     // Dose derived from Dose_stat (mqi_run with each scorer once): the kernel
     // scores Dose_stat only; d_snap holds Dose_stat before the run
     bool    alias_dose = false;
+    // Dose derived from the Dij tables (mqi_run, production kernels): the
+    // kernel scores the tables only
+    bool    dij_dose   = false;
     double* d_snap     = nullptr;
     size_t  snap_n     = 0;
     unsigned int*       d_status   = nullptr;
@@ -519,9 +522,14 @@ upload_grid_common(mqi_ctx* c, int nx, int ny, int nz, const float* xe, const fl
     return dalloc(c, &c->d_density, nvox(c));
 }
 
+// dynamic LDS of a transport launch; the waves' Dij queues are left out of a
+// production launch with the Dij scorer where they would not fit 64 KB
 size_t
-shmem_bytes(const mqi_ctx* c, int threads) {
-    return mqi_shmem_bytes(c->nx, c->ny, c->nz, c->bl_n_edges, threads);
+shmem_bytes(const mqi_ctx* c, const mqi_run_config& cfg, int threads, int* queued = nullptr) {
+    const size_t sh = mqi_shmem_bytes(c->nx, c->ny, c->nz, c->bl_n_edges, threads), q = mqi_dij_queue_bytes(threads);
+    const bool   with = cfg.dij && !cfg.exact && cfg.scoring_loops == MQI_LOOPS_ONCE && sh + q <= 65536;
+    if (queued) *queued = with ? 1 : 0;
+    return sh + (with ? q : 0);
 }
 
 int
@@ -612,7 +620,7 @@ fill_params(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg) {
     // (the kernel then does one atomic less per step)
     P.n_scorers = 0;
     for (size_t k = 0; k < c->kinds.size(); ++k) {
-        if (c->alias_dose && k == 0) continue;
+        if ((c->alias_dose || c->dij_dose) && k == 0) continue;
         P.kinds[P.n_scorers] = c->kinds[k];
         P.out[P.n_scorers]   = c->d_out[k];
         P.n_scorers++;
@@ -624,6 +632,7 @@ fill_params(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg) {
         P.dij_keys     = c->d_dij_keys;
         P.dij_vals     = c->d_dij_vals;
         P.dij_off      = c->d_dij_off;
+        P.dij_dose     = c->dij_dose ? c->d_out[0] : nullptr;
     }
     P.out_scenario_stride = c->per_scen ? nvox(c) : 0;
     P.loops               = cfg.scoring_loops;
@@ -672,7 +681,7 @@ launch_bound(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int dyn
     if ((uint64_t) blocks * threads * (uint64_t) P.stack_cap * MQI_STACK_FLOATS * sizeof(float) > stack_bytes)
         return (int) hipErrorInvalidValue;
     pack_scoring(P);
-    const size_t sh = shmem_bytes(c, threads);
+    const size_t sh = shmem_bytes(c, cfg, threads, &P.dij_queued);
     if (dynamic) {
         const int e = mqi_aux::queue_init(P.queue, P.total, c->stream);
         if (e) return e;
@@ -749,7 +758,7 @@ check_tuning(mqi_ctx* c, const mqi_run_config& cfg) {
 int
 persistent_blocks(mqi_ctx* c, const mqi_run_config& cfg, int threads, int trace) {
     if (cfg.blocks > 0) return cfg.blocks;
-    const size_t sh  = shmem_bytes(c, threads);
+    const size_t sh  = shmem_bytes(c, cfg, threads);
     int          occ = cfg.exact ? mqi_exact::occupancy(cfg.physics_debug, 1, trace, 0, threads, sh)
                                  : mqi_fast::occupancy(cfg.physics_debug, 1, trace, cfg.waves_per_simd, threads, sh);
     return c->n_cu * occ;
@@ -779,7 +788,7 @@ graph_pass(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int block
     bind_buffers(c, P);
     pack_scoring(P);
     const int variant[6] = {cfg.physics_debug, cfg.exact, cfg.exact ? 0 : cfg.waves_per_simd, blocks, threads,
-                            (int) shmem_bytes(c, threads)};
+                            (int) shmem_bytes(c, cfg, threads)};
     std::vector<unsigned char> key(sizeof P + sizeof variant);
     std::memcpy(key.data(), &P, sizeof P);
     std::memcpy(key.data() + sizeof P, variant, sizeof variant);
@@ -946,6 +955,14 @@ alloc_dij(mqi_ctx* c, const mqi_run_config& cfg) {
     KCHK(c, mqi_aux::fill_u32(c->d_dij_keys, 0xffffffffu, total, c->stream));
     KCHK(c, mqi_aux::fill_u64(c->d_dij_vals, 0ull, total, c->stream));
     return 0;
+}
+
+// workgroups per table of the scans over the Dij tables: a few per CU in
+// all, of 2048 slots at least
+uint32_t
+dij_chunks(const mqi_ctx* c) {
+    const uint64_t n = std::max<uint64_t>(c->dij_items, 1), slots = c->dij_off[c->dij_items];
+    return (uint32_t) std::max<uint64_t>(1, std::min<uint64_t>((8192 + n - 1) / n, slots / n / 2048));
 }
 
 // message of the last failed mqi_create on this thread (there is no context
@@ -1269,9 +1286,15 @@ mqi_run(mqi_ctx* c, const mqi_run_config* cfg_in, mqi_run_result* res) {
     }
     struct alias_guard {
         mqi_ctx* c;
-        ~alias_guard() { c->alias_dose = false; }
+        ~alias_guard() { c->alias_dose = c->dij_dose = false; }
     } ag{c};
     c->alias_dose = alias;
+    // Dose and the Dij receive the same per-step value under the same ROI
+    // (unless Dose comes from Dose_stat already): score the tables only and
+    // add their entries to Dose at the end of the run.  A step leaves one
+    // FP64 atomic instead of two: MEASURED
+    c->dij_dose = !alias && cfg.dij && !cfg.exact && cfg.scoring_loops == MQI_LOOPS_ONCE && !c->kinds.empty() &&
+                  c->kinds[0] == MQI_KIND_DOSE;
     uint64_t  round_len  = p.max_item;
     double    ms         = 0;
     int       rounds     = 0;
@@ -1293,6 +1316,10 @@ mqi_run(mqi_ctx* c, const mqi_run_config* cfg_in, mqi_run_result* res) {
     // (mqi_tps_env.hpp:1430-1476, mqi_variables.hpp:51-66)
     const bool   rescale = cfg.stat_criterion > 0 && rounds > 1;
     const double w       = rescale ? (double) (float) (double) (p.total * 1.0 / (double) cnt[1]) : 1.0;
+    if (c->dij_dose)
+        KCHK(c, mqi_aux::dose_from_dij(c->d_dij_keys, c->d_dij_vals, c->d_dij_off, (uint32_t) c->dij_items,
+                                       dij_chunks(c), (uint32_t) c->spots.size(), c->per_scen ? nvox(c) : 0,
+                                       c->d_out[0], c->stream));
     if (alias) {
         KCHK(c, mqi_aux::dose_from_stat(c->d_out[0], c->d_out[s1], c->d_snap, n_all, nvox(c), w, c->stream));
     }
@@ -1715,10 +1742,7 @@ mqi_dij_build(mqi_ctx* c, double rel_thr) {
     hipSetDevice(c->device);
     free_dij(c);
     const uint32_t n_items = (uint32_t) c->dij_items, n_spots = (uint32_t) c->spots.size();
-    // workgroups per table: a few per CU in all, of 2048 slots at least
-    const uint64_t slots  = c->dij_off[n_items];
-    const uint32_t chunks = (uint32_t) std::max<uint64_t>(
-      1, std::min<uint64_t>((8192 + n_items - 1) / n_items, slots / n_items / 2048));
+    const uint32_t chunks  = dij_chunks(c);
     struct tables {
         double*   max   = nullptr;   // per item
         uint32_t* count = nullptr;   // per chunk: entries, then the first place

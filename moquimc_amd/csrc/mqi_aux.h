@@ -31,6 +31,9 @@ int dij_count(const double* vals, const uint64_t* off, uint32_t n_items, uint32_
 int dij_write(const uint32_t* keys, const double* vals, const uint64_t* off, uint32_t item0, uint32_t n_spots,
               uint32_t chunks, const double* item_max, double rel_thr, const uint32_t* start, uint32_t* vox,
               uint64_t* packed, hipStream_t s);
+// the tables' entries added to Dose (scenario s at dose + s * stride)
+int dose_from_dij(const uint32_t* keys, const double* vals, const uint64_t* off, uint32_t n_items, uint32_t chunks,
+                  uint32_t n_spots, uint64_t stride, double* dose, hipStream_t s);
 // a CSR's values with their rows: packed[k] = (row, value) of nonzero k
 int pack_rows(const int64_t* indptr, const float* val, int64_t n_rows, uint64_t* packed, hipStream_t s);
 // stable radix sort of n (key; 64-bit value) pairs by the low `bits` of the

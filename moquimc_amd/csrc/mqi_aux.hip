@@ -325,6 +325,32 @@ k_dij_write(const uint32_t* __restrict__ keys, const double* __restrict__ vals, 
     }
 }
 
+// every entry of every table added to its scenario's Dose
+__global__ void __launch_bounds__(256)
+k_dij_dose(const uint32_t* __restrict__ keys, const double* __restrict__ vals, const uint64_t* __restrict__ off,
+           uint32_t chunks, uint32_t n_spots, uint64_t stride, double* __restrict__ dose) {
+    const uint32_t item = blockIdx.x / chunks, chunk = blockIdx.x % chunks;
+    const uint64_t o = off[item], cap = off[item + 1] - o;
+    const uint64_t e   = o + chunk_begin(cap, chunk + 1, chunks);
+    double*        out = dose + stride * (item / n_spots);
+    for (uint64_t i = o + chunk_begin(cap, chunk, chunks) + threadIdx.x; i < e; i += 256 * MQI_SCAN) {
+        double v[MQI_SCAN];
+#pragma unroll
+        for (int j = 0; j < MQI_SCAN; ++j) v[j] = i + 256 * j < e ? vals[i + 256 * j] : 0.0;
+#pragma unroll
+        for (int j = 0; j < MQI_SCAN; ++j)
+            if (v[j] != 0.0) atomicAdd(out + keys[i + 256 * j], v[j]);
+    }
+}
+int
+dose_from_dij(const uint32_t* keys, const double* vals, const uint64_t* off, uint32_t n_items, uint32_t chunks,
+              uint32_t n_spots, uint64_t stride, double* dose, hipStream_t s) {
+    if (n_items == 0) return 0;
+    hipLaunchKernelGGL(k_dij_dose, dim3(n_items * chunks), dim3(256), 0, s, keys, vals, off, chunks, n_spots, stride,
+                       dose);
+    return (int) hipGetLastError();
+}
+
 int
 dij_count(const double* vals, const uint64_t* off, uint32_t n_items, uint32_t chunks, double rel_thr,
           double* item_max, uint32_t* counts, hipStream_t s) {

@@ -45,6 +45,21 @@ __host__ __device__ inline size_t mqi_shmem_bytes(int nx, int ny, int nz, int bl
     return sizeof(float) * (size_t) mqi_pend_offset(nx, ny, nz, bl_edges) + sizeof(double) * MQI_DEFER * (size_t) threads;
 }
 
+// Production launches with the Dij scorer: behind the pending sums, a queue
+// per wave of the deposits whose slot is not known yet
+#define MQI_DIJ_QUEUE 128
+struct mqi_dij_entry {
+    uint32_t voxel, item;
+    double   value;
+};
+struct mqi_dij_queue {
+    uint32_t      n, pad[3];
+    mqi_dij_entry e[MQI_DIJ_QUEUE];
+};
+__host__ __device__ inline size_t mqi_dij_queue_bytes(int threads) {
+    return sizeof(mqi_dij_queue) * (size_t) ((threads + 63) / 64);
+}
+
 // floats per secondary-stack entry: ke0, pos[3], dir[3], ke1, dE, and the
 // beamline child whose transform still has to place it (-1: placed)
 #define MQI_STACK_FLOATS 10
@@ -121,6 +136,8 @@ struct transport_params {
     uint32_t* dij_keys;
     double*   dij_vals;
     const uint64_t* dij_off;  // item i owns slots [dij_off[i], dij_off[i + 1]) of dij_keys/dij_vals
+    double*   dij_dose;       // Dose, when it is derived from the tables: takes what a full table cannot
+    int       dij_queued;     // the launch's LDS holds the waves' Dij queues
     // secondary stack
     float* stack;
     int    stack_cap;

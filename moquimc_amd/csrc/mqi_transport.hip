@@ -847,30 +847,103 @@ MQI_DI bool let_terms(const trk& t, float density, double& length, double& let) 
 // probing stops after MQI_DIJ_MAX_PROBE slots (a table that full is an
 // overflow: the run reports it instead of crawling through a full table).
 #define MQI_DIJ_MAX_PROBE 4096
-MQI_DI void dij_insert(const transport_params& P, uint64_t item, uint32_t voxel, double value) {
+// A table's slots in groups of 32 for the 4 x 4 x 2 voxels of a block, so the
+// keys of a block share a 128-byte line and its values two: the lanes of a
+// spot work in the same few blocks.  A voxel's home is its place in the group
+// that its block's number hashes to; on a conflict it tries its place in the
+// next groups, then the slots behind its home one by one (a table smaller
+// than a group has no groups).
+#define MQI_DIJ_GROUP_PROBES 16
+MQI_DI uint32_t dij_home(const transport_params& P, int cx, int cy, int cz, uint32_t groups) {
+    const uint32_t nbx = (uint32_t) (P.nx + 3) >> 2, nby = (uint32_t) (P.ny + 3) >> 2;
+    const uint32_t id  = ((uint32_t) (cz >> 1) * nby + (uint32_t) (cy >> 2)) * nbx + (uint32_t) (cx >> 2);
+    const uint32_t g   = __umulhi(id * 2654435761u, groups);
+    return g << 5 | (uint32_t) (cx & 3) | (uint32_t) (cy & 3) << 2 | (uint32_t) (cz & 1) << 4;
+}
+// A key changes once, from empty to its voxel, so a plain load that shows a
+// voxel is final: the slot is ours, or taken by another voxel.  Only a load
+// that shows it empty (possibly a stale cached line) needs the
+// compare-and-swap, which is performed beyond the caches.
+MQI_DI bool dij_claim(uint32_t* key, uint32_t voxel) {
+    uint32_t k = *key;
+    if (k == 0xffffffffu) k = atomicCAS(key, 0xffffffffu, voxel);
+    return k == 0xffffffffu || k == voxel;
+}
+MQI_DI void dij_insert(const transport_params& P, uint32_t item, uint32_t voxel, double value) {
     if (value <= 0) return;
-    const uint64_t base = P.dij_off[item];
-    const uint64_t cap  = P.dij_off[item + 1] - base;
-    uint32_t*      keys = P.dij_keys + base;
-    double*        vals = P.dij_vals + base;
-    uint32_t       h    = voxel * 2654435761u;
-    uint64_t       slot = ((uint64_t) h * cap) >> 32;
-    const uint64_t n_probe = cap < MQI_DIJ_MAX_PROBE ? cap : MQI_DIJ_MAX_PROBE;
-    // A key changes once, from empty to its voxel, so a plain load that
-    // shows a voxel is final: the slot is ours, or taken by another voxel.
-    // Only a load that shows it empty (possibly a stale cached line) needs
-    // the compare-and-swap, which is performed beyond the caches.
-    for (uint64_t probe = 0; probe < n_probe; ++probe) {
-        uint32_t k = keys[slot];
-        if (k == 0xffffffffu) k = atomicCAS(keys + slot, 0xffffffffu, voxel);
-        if (k == 0xffffffffu || k == voxel) {
+    const uint64_t base   = P.dij_off[item];
+    const uint64_t cap    = P.dij_off[item + 1] - base;
+    uint32_t*      keys   = P.dij_keys + base;
+    double*        vals   = P.dij_vals + base;
+    const uint32_t groups = (uint32_t) (cap >> 5), tries = groups ? MQI_DIJ_GROUP_PROBES : 0;
+    const uint32_t last   = tries + (uint32_t) (cap < MQI_DIJ_MAX_PROBE ? cap : MQI_DIJ_MAX_PROBE);
+    uint32_t       home   = 0;
+    if (groups) {
+        const uint32_t yz = voxel / (uint32_t) P.nx, cz = yz / (uint32_t) P.ny;
+        home = dij_home(P, (int) (voxel - yz * (uint32_t) P.nx), (int) (yz - cz * (uint32_t) P.ny), (int) cz, groups);
+    }
+    uint32_t slot = home;
+    for (uint32_t probe = 1; probe <= last; ++probe) {
+        if (dij_claim(keys + slot, voxel)) {
             atomicAdd(vals + slot, value);
             return;
         }
-        slot = (slot + 1 == cap) ? 0 : slot + 1;
+        if (probe < tries)
+            slot = slot >> 5 < groups - 1 ? slot + 32 : slot & 31;
+        else if (probe == tries)
+            slot = home;
+        else
+            slot = (uint64_t) slot + 1 < cap ? slot + 1 : 0;
     }
     atomicOr(P.status, MQI_STATUS_DIJ_FULL);
+    if (P.dij_dose) atomicAdd(P.dij_dose + P.out_scenario_stride * (item / (uint32_t) P.n_spots) + voxel, value);
 }
+
+#if !MQI_EXACT
+// Deposits whose slot the key loaded with the voxel's density did not show
+// wait in their wave's queue in LDS until half of it may be in use, and then
+// go into the tables side by side: a first touch, a conflict or a probe by
+// one lane costs the other 63 nothing.  The lanes of a wave share the queue
+// without barriers (LDS accesses of one wave are performed in order).
+MQI_DI void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+MQI_DI uint32_t lane_rank(unsigned long long m) {   // lanes of m below this one
+    return __builtin_amdgcn_mbcnt_hi((uint32_t) (m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) m, 0u));
+}
+MQI_DI void dij_defer(mqi_dij_queue* q, const mqi_dij_entry& e) {
+    const unsigned long long m    = __ballot(1);
+    const uint32_t           rank = lane_rank(m), at = q->n;
+    wave_fence();
+    q->e[at + rank] = e;
+    if (rank == 0) q->n = at + (uint32_t) __popcll(m);
+    wave_fence();
+}
+// The queue if it holds more than `keep` entries, by the lanes that are here;
+// without a queue each lane's own deposit (voxel 0xffffffff: none).
+MQI_DI void dij_drain(const transport_params& P, mqi_dij_queue* q, const mqi_dij_entry& own, uint32_t keep) {
+    uint32_t i = 0, n = own.voxel != 0xffffffffu ? 1 : 0, step = 1;
+    if (q) {
+        const unsigned long long m = __ballot(1);
+        n    = q->n;
+        i    = lane_rank(m);
+        step = (uint32_t) __popcll(m);
+        if (n <= keep) return;
+        wave_fence();
+    }
+    const bool first = i == 0;
+    for (; i < n; i += step) {
+        const mqi_dij_entry x = q ? q->e[i] : own;
+        dij_insert(P, x.item, x.voxel, x.value);
+    }
+    if (q) {
+        wave_fence();
+        if (first) q->n = 0;
+        wave_fence();
+    }
+}
+#endif
 
 // The launch's scoring as the loop's code reads it: two words, taken apart
 // where a field is used (a compiler that sees the fields' comparisons before
@@ -884,6 +957,7 @@ struct scoring {
     MQI_DI int  pair() const { return mode >> 6 & 7; }
     MQI_DI int  grouped() const { return mode >> 9 & 7; }
     MQI_DI int  dij_slot() const { return (int) (mode >> 12 & 15) - 1; }
+    MQI_DI bool dij_deferred() const { return loops() == MQI_LOOPS_ONCE && (uint32_t) dij_slot() < MQI_DEFER; }
 };
 MQI_DI scoring scoring_of(const transport_params& P) {
     scoring S;
@@ -905,6 +979,10 @@ struct pending {
     int32_t  cnb;    // voxel of the pending sums, -1: none
     uint32_t scen;   // their scenario
     uint32_t item;   // their Dij table (scenario, spot)
+#if !MQI_EXACT
+    uint32_t key;    // what the voxel's home slot in that table showed, and
+    uint64_t slot;   // that slot
+#endif
 };
 MQI_DI uint64_t pend_element(const transport_params& P, const pending& A) {
     return P.out_scenario_stride * A.scen + (uint32_t) A.cnb;
@@ -912,7 +990,8 @@ MQI_DI uint64_t pend_element(const transport_params& P, const pending& A) {
 
 // accumulated slots are positive, +inf or NaN (every value that is not <= 0
 // is added, NaN included); untouched slots are 0
-MQI_DI void flush(const transport_params& P, const scoring& S, pending& A, double* v) {
+MQI_DI void flush(const transport_params& P, const scoring& S, pending& A, double* v, mqi_dij_entry& own,
+                  mqi_dij_queue* q) {
     if (A.cnb >= 0) {
         const uint64_t k  = pend_element(P, A);
         double         dx = 0.0;   // the Dij slot's sum: inserted behind the loop, from one place
@@ -931,7 +1010,21 @@ MQI_DI void flush(const transport_params& P, const scoring& S, pending& A, doubl
                     atomicAdd(P.out[s] + k, x);
             }
         }
-        if (dx != 0.0) dij_insert(P, A.item, (uint32_t) A.cnb, dx);
+        if (dx != 0.0) {
+#if MQI_EXACT
+            dij_insert(P, A.item, (uint32_t) A.cnb, dx);
+#else
+            if (A.key == (uint32_t) A.cnb) {
+                atomicAdd(P.dij_vals + A.slot, dx);
+            } else {
+                const mqi_dij_entry e = { (uint32_t) A.cnb, A.item, dx };
+                if (q)
+                    dij_defer(q, e);
+                else
+                    own = e;
+            }
+#endif
+        }
     }
     A.cnb = -1;
 }
@@ -1124,6 +1217,10 @@ struct lane {
     float    scale;      // scenario density scale
     uint32_t scen;       // scenario
     uint32_t dij_item;   // Dij table of (scenario, spot): scenario * n_spots + spot
+#if !MQI_EXACT
+    uint64_t dij_base;   // its first slot and groups of slots
+    uint32_t dij_groups;
+#endif
     int      tsteps;     // steps of the current track
     pending  acc;        // deferred deposits of the current voxel
     bool     newhist;    // the first step of a history: the pending deposits are another one's
@@ -1337,7 +1434,7 @@ MQI_DI void trace_record(const transport_params& P, lane& L, uint64_t cnb) {
 // in a beamline child (no scoring there; leaving it hands the track to the
 // next child).  One stepping call site serves both.
 template<bool DBG, bool TRACE>
-MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, double* pv) {
+MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, double* pv, mqi_dij_queue* q) {
     trk&       t  = L.t;
     const bool bl = c.child < c.nbl;
     uint64_t   cnb;
@@ -1359,6 +1456,17 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
     } else {
         cnb              = (uint64_t) (int32_t) (t.cz * c.g.nx * c.g.ny + t.cy * c.g.nx + t.cx);
         const float dens = P.density[cnb];
+        const scoring S  = scoring_of(P);
+#if !MQI_EXACT
+        // the voxel's home in the spot's Dij table: its key, read now, is
+        // looked at when the lane leaves the voxel
+        uint64_t home = 0;
+        uint32_t key  = 0xffffffffu;
+        if (S.dij_deferred() && L.dij_groups) {
+            home = L.dij_base + dij_home(P, t.cx, t.cy, t.cz, L.dij_groups);
+            key  = P.dij_keys[home];
+        }
+#endif
         t.its            = MQI_VOXEL_EXIT(c.g, t.p0, t.d0, t.cx, t.cy, t.cz);
         rho              = dens * L.scale;
         // The deposits gathered in the voxel the lane has left go out here,
@@ -1367,7 +1475,6 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
         // issued just before the next wait on a load would add their round
         // trip to every step.
         // (A history's deposits are its own scenario's and Dij table's.)
-        const scoring S  = scoring_of(P);
         const bool leave = S.loops() == MQI_LOOPS_ONCE && ((int32_t) cnb != L.acc.cnb || L.newhist);
         L.newhist        = false;
 #if !MQI_EXACT
@@ -1377,8 +1484,17 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
             flush_quad(P, S, L.acc, pv, leave);
         else
 #endif
-        if (leave)
-            flush(P, S, L.acc, pv);
+        {
+            mqi_dij_entry own = { 0xffffffffu, 0, 0.0 };
+            if (leave) flush(P, S, L.acc, pv, own, q);
+#if !MQI_EXACT
+            if (S.dij_deferred()) dij_drain(cold(), q, own, MQI_DIJ_QUEUE - 64);
+#endif
+        }
+#if !MQI_EXACT
+        L.acc.key  = key;
+        L.acc.slot = home;
+#endif
     }
     float sp;   // stopping power ratio of the step
     stepping<DBG>(c, t, rho, t.its, sp);
@@ -1493,6 +1609,13 @@ k_transport(transport_params P) {
     double* pv = reinterpret_cast<double*>(sh + mqi_pend_offset(P.nx, P.ny, P.nz, P.bl_n_edges)) + threadIdx.x;
 #pragma unroll
     for (int s = 0; s < MQI_DEFER; ++s) pv[s * blockDim.x] = 0.0;
+    mqi_dij_queue* q = nullptr;   // the wave's, if the launch has room for them
+#if !MQI_EXACT
+    if (P.dij_queued) {
+        q = reinterpret_cast<mqi_dij_queue*>(pv - threadIdx.x + MQI_DEFER * blockDim.x) + (threadIdx.x >> 6);
+        q->n = 0;
+    }
+#endif
     const uint64_t tid      = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t nthreads = (uint64_t) gridDim.x * blockDim.x;
 
@@ -1515,6 +1638,12 @@ k_transport(transport_params P) {
     L.acc.cnb  = -1;
     L.acc.scen = 0;
     L.acc.item = 0;
+#if !MQI_EXACT
+    L.acc.key    = 0xffffffffu;
+    L.acc.slot   = 0;
+    L.dij_base   = 0;
+    L.dij_groups = 0;
+#endif
     L.newhist  = false;
     L.reenter  = false;
     c.g.sx = c.g.sy = c.g.sz = 0.0f;
@@ -1604,6 +1733,12 @@ k_transport(transport_params P) {
             L.scen                 = scen;
             L.dij_item             = scen * (uint32_t) C.n_spots + spot_id;
             L.newhist              = true;
+#if !MQI_EXACT
+            if (C.dij_off) {
+                L.dij_base   = C.dij_off[L.dij_item];
+                L.dij_groups = (uint32_t) ((C.dij_off[L.dij_item + 1] - L.dij_base) >> 5);
+            }
+#endif
             if (C.vertices) {
                 const float* v = C.vertices + 7 * g;
                 L.t.ke0        = v[0];
@@ -1642,10 +1777,14 @@ k_transport(transport_params P) {
             L.active  = enter_chain(cold(), c, L.t, shb);
             if (!L.active) continue;
         }
-        step<DBG, TRACE>(P, c, L, shb, pv);
+        step<DBG, TRACE>(P, c, L, shb, pv, q);
         ++nstep;
     }
-    flush(P, scoring_of(P), L.acc, pv);
+    mqi_dij_entry own = { 0xffffffffu, 0, 0.0 };
+    flush(P, scoring_of(P), L.acc, pv, own, q);
+#if !MQI_EXACT
+    if (scoring_of(P).dij_deferred()) dij_drain(cold(), q, own, 0);
+#endif
     atomicAdd(cold().tracked, (unsigned long long) done);
     atomicAdd(cold().steps, (unsigned long long) nstep);
     if (c.drops) atomicAdd(cold().drops, (unsigned long long) c.drops);
