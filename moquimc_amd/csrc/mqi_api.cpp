@@ -755,6 +755,18 @@ check_tuning(mqi_ctx* c, const mqi_run_config& cfg) {
     return 0;
 }
 
+// waves_per_simd 0: 4 for a launch of more histories than the lanes of 3 hold,
+// 3 for a smaller one, which the longest track bounds: its wave runs alone on
+// a SIMD at the end, and the register budget of 3 spills nothing.  Slab
+// phantom (2.5e6 histories) 28.9 ms with 4 against 30.5 with 3, 2000-spot CT
+// 355 / 360, nine Dij scenarios (1.2e6) 8.9 / 9.8, Dij field (2e6) 14.6 /
+// 15.7; water spot (1e5) 5.20 / 5.12, small CT field (1.3e5) 2.83 / 2.84.
+int
+waves_for(const mqi_ctx* c, const mqi_run_config& cfg, uint64_t histories) {
+    if (cfg.exact || cfg.waves_per_simd) return cfg.waves_per_simd;
+    return histories > (uint64_t) c->n_cu * 4 * 3 * 64 ? 4 : 3;
+}
+
 int
 persistent_blocks(mqi_ctx* c, const mqi_run_config& cfg, int threads, int trace) {
     if (cfg.blocks > 0) return cfg.blocks;
@@ -828,7 +840,8 @@ graph_pass(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int block
 // launch per spot of the plan.  Adds the device time of the transport
 // kernels to *ms.
 int
-transport_pass(mqi_ctx* c, const mqi_run_config& cfg, uint64_t hoff, double* ms) {
+transport_pass(mqi_ctx* c, const mqi_run_config& cfg_in, uint64_t hoff, double* ms) {
+    mqi_run_config cfg = cfg_in;
     const int threads = cfg.block_size > 0 ? cfg.block_size : 256;
     if (threads % 64 != 0 || threads > 256) return fail(c, MQI_E_ARG, "block_size must be 64, 128, 192 or 256");
     transport_params P;
@@ -843,6 +856,7 @@ transport_pass(mqi_ctx* c, const mqi_run_config& cfg, uint64_t hoff, double* ms)
         if (p.total == 0) return 0;
         P.n_items      = (int) p.item_end.size();
         P.total        = p.total;
+        cfg.waves_per_simd = waves_for(c, cfg, p.total);
         const int blocks = persistent_blocks(c, cfg, threads, 0);
         if ((r = ensure_stack(c, lane_bytes * (size_t) blocks * threads))) return r;
         P.stack = c->d_stack;
@@ -869,6 +883,7 @@ transport_pass(mqi_ctx* c, const mqi_run_config& cfg, uint64_t hoff, double* ms)
         if ((r = upload_plan(c, p))) return r;
         P.n_items    = (int) p.item_end.size();
         P.total      = p.total;
+        cfg.waves_per_simd = waves_for(c, cfg_in, p.total);
         uint64_t lanes = std::min<uint64_t>(p.total, max_lanes);
         int      blocks = (int) ((lanes + threads - 1) / threads);   // <= max_blocks
         HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1465,6 +1480,7 @@ mqi_run_vertices(mqi_ctx* c, const float* vtx, uint64_t n, const uint32_t* spot_
     mqi_run_config cfg = *cfg_in;
     if ((r = check_tuning(c, cfg))) return r;
     if (cfg.dij) return fail(c, MQI_E_ARG, "Dij scoring needs a spot table (mqi_run)");
+    cfg.waves_per_simd = waves_for(c, cfg, n);
     float*    d_v = nullptr;
     uint32_t* d_s = nullptr;
     if ((r = dalloc(c, &d_v, 7 * n))) return r;

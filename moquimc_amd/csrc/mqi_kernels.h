@@ -46,7 +46,9 @@ __host__ __device__ inline size_t mqi_shmem_bytes(int nx, int ny, int nz, int bl
 }
 
 // Production launches with the Dij scorer: behind the pending sums, a queue
-// per wave of the deposits whose slot is not known yet
+// per wave of the deposits whose slot is not known yet, with the lanes' view
+// of their Dij table: its first slot and groups of 32 slots, and the home
+// slot (from the first table's first slot) of the pending voxel
 #define MQI_DIJ_QUEUE 128
 struct mqi_dij_entry {
     uint32_t voxel, item;
@@ -55,6 +57,8 @@ struct mqi_dij_entry {
 struct mqi_dij_queue {
     uint32_t      n, pad[3];
     mqi_dij_entry e[MQI_DIJ_QUEUE];
+    uint64_t      base[64], slot[64];
+    uint32_t      groups[64];
 };
 __host__ __device__ inline size_t mqi_dij_queue_bytes(int threads) {
     return sizeof(mqi_dij_queue) * (size_t) ((threads + 63) / 64);

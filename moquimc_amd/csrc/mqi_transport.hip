@@ -980,8 +980,7 @@ struct pending {
     uint32_t scen;   // their scenario
     uint32_t item;   // their Dij table (scenario, spot)
 #if !MQI_EXACT
-    uint32_t key;    // what the voxel's home slot in that table showed, and
-    uint64_t slot;   // that slot
+    uint32_t key;    // what the voxel's home slot in that table showed
 #endif
 };
 MQI_DI uint64_t pend_element(const transport_params& P, const pending& A) {
@@ -1014,8 +1013,8 @@ MQI_DI void flush(const transport_params& P, const scoring& S, pending& A, doubl
 #if MQI_EXACT
             dij_insert(P, A.item, (uint32_t) A.cnb, dx);
 #else
-            if (A.key == (uint32_t) A.cnb) {
-                atomicAdd(P.dij_vals + A.slot, dx);
+            if (q && A.key == (uint32_t) A.cnb) {
+                atomicAdd(P.dij_vals + q->slot[__lane_id()], dx);
             } else {
                 const mqi_dij_entry e = { (uint32_t) A.cnb, A.item, dx };
                 if (q)
@@ -1217,10 +1216,6 @@ struct lane {
     float    scale;      // scenario density scale
     uint32_t scen;       // scenario
     uint32_t dij_item;   // Dij table of (scenario, spot): scenario * n_spots + spot
-#if !MQI_EXACT
-    uint64_t dij_base;   // its first slot and groups of slots
-    uint32_t dij_groups;
-#endif
     int      tsteps;     // steps of the current track
     pending  acc;        // deferred deposits of the current voxel
     bool     newhist;    // the first step of a history: the pending deposits are another one's
@@ -1462,9 +1457,12 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
         // looked at when the lane leaves the voxel
         uint64_t home = 0;
         uint32_t key  = 0xffffffffu;
-        if (S.dij_deferred() && L.dij_groups) {
-            home = L.dij_base + dij_home(P, t.cx, t.cy, t.cz, L.dij_groups);
-            key  = P.dij_keys[home];
+        if (q) {
+            const uint32_t groups = q->groups[__lane_id()];
+            if (groups) {
+                home = q->base[__lane_id()] + dij_home(P, t.cx, t.cy, t.cz, groups);
+                key  = P.dij_keys[home];
+            }
         }
 #endif
         t.its            = MQI_VOXEL_EXIT(c.g, t.p0, t.d0, t.cx, t.cy, t.cz);
@@ -1492,8 +1490,10 @@ MQI_DI void step(const transport_params& P, ctx& c, lane& L, const float* shb, d
 #endif
         }
 #if !MQI_EXACT
-        L.acc.key  = key;
-        L.acc.slot = home;
+        if (q) {
+            q->slot[__lane_id()] = home;
+            L.acc.key            = key;
+        }
 #endif
     }
     float sp;   // stopping power ratio of the step
@@ -1639,10 +1639,7 @@ k_transport(transport_params P) {
     L.acc.scen = 0;
     L.acc.item = 0;
 #if !MQI_EXACT
-    L.acc.key    = 0xffffffffu;
-    L.acc.slot   = 0;
-    L.dij_base   = 0;
-    L.dij_groups = 0;
+    L.acc.key = 0xffffffffu;
 #endif
     L.newhist  = false;
     L.reenter  = false;
@@ -1734,9 +1731,10 @@ k_transport(transport_params P) {
             L.dij_item             = scen * (uint32_t) C.n_spots + spot_id;
             L.newhist              = true;
 #if !MQI_EXACT
-            if (C.dij_off) {
-                L.dij_base   = C.dij_off[L.dij_item];
-                L.dij_groups = (uint32_t) ((C.dij_off[L.dij_item + 1] - L.dij_base) >> 5);
+            if (q) {
+                const uint64_t b        = C.dij_off[L.dij_item];
+                q->base[__lane_id()]    = b;
+                q->groups[__lane_id()]  = (uint32_t) ((C.dij_off[L.dij_item + 1] - b) >> 5);
             }
 #endif
             if (C.vertices) {
@@ -1816,10 +1814,8 @@ variant pick_waves(int waves) {
     return make<D, Y, T, 0>();
 #else
     if (T) return make<D, Y, T, 0>();
-    // 0: 3 waves/SIMD, the measured optimum of the production kernels with
-    // deferred scoring on every plan measured (CT, Dij, robust, slab and
-    // water phantoms: 4-16% faster than 4, whose extra waves add atomics in
-    // flight and spills); 2: the compiler's own register budget
+    // the callers choose between 3 and 4 (the budgets without spills in the
+    // step; 5 spills and is slower everywhere); 2: the compiler's own budget
     switch (waves) {
     case 2: return make<D, Y, T, 0>();
     case 4: return make<D, Y, T, 4>();
