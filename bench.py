@@ -1,5 +1,5 @@
 """Benchmark: proton transport histories/s on one MI355X, batched persistent
-launch vs plain per-spot launches, on the 2000-spot synthetic CT plan; plus
+launch vs plain launches, on the 2000-spot synthetic CT plan; plus
 the Dij adjoint (D^T g) bandwidth on the 5000-spot Dij workload, the
 9-scenario robust Dij leg, and the water and slab phantom workloads.
 
@@ -503,7 +503,7 @@ def main():
     ctx.run(cfg)
     dose_batched = ctx.scorer(0)
 
-    # plain per-spot launches (one launch and host sync per spot, as run_by_spot), same criterion
+    # plain launches (a lane per history, host sync per launch, spots sharing one), same criterion
     plain_ms, plain_hist, plain_wall, agree = 0.0, 0, 0.0, None
     for i in range(args.plain_passes):
         ctx.zero_scorers()

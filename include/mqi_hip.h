@@ -54,7 +54,8 @@ typedef struct mqi_run_config {
     uint64_t seed;             /* master seed of the per-history Philox streams */
     int32_t  physics_debug;    /* 1: the __PHYSICS_DEBUG__ physics of the phantom build, 0: release */
     int32_t  exact;            /* 1: verification kernels (portable math, no FMA), 0: production */
-    int32_t  batched;          /* 1: one persistent launch over all items; 0: one plain launch per spot */
+    int32_t  batched;          /* 1: one persistent launch over all items; 0: plain launches, a lane per history,
+                                  consecutive spots sharing one up to 2^18 histories */
     int32_t  scoring_loops;    /* MQI_LOOPS_* */
     int32_t  stack_depth;      /* secondary stack per lane; 0: the reference's (200 debug, 10 release) */
     int32_t  block_size;       /* threads per workgroup; 0: 256 */

@@ -526,7 +526,8 @@ upload_grid_common(mqi_ctx* c, int nx, int ny, int nz, const float* xe, const fl
 // production launch with the Dij scorer where they would not fit 64 KB
 size_t
 shmem_bytes(const mqi_ctx* c, const mqi_run_config& cfg, int threads, int* queued = nullptr) {
-    const size_t sh = mqi_shmem_bytes(c->nx, c->ny, c->nz, c->bl_n_edges, threads), q = mqi_dij_queue_bytes(threads);
+    const size_t sh = mqi_shmem_bytes(c->nx, c->ny, c->nz, c->bl_n_edges, threads);
+    const size_t q    = mqi_dij_queue_bytes(threads);
     const bool   with = cfg.dij && !cfg.exact && cfg.scoring_loops == MQI_LOOPS_ONCE && sh + q <= 65536;
     if (queued) *queued = with ? 1 : 0;
     return sh + (with ? q : 0);
@@ -559,15 +560,20 @@ struct run_plan {
     uint64_t              max_item = 0;
 };
 
-// items are (scenario, spot), scenario-major; empty spots are skipped
+uint64_t
+item_histories(const mqi_ctx* c, int scenario, size_t spot) {
+    const uint64_t h = c->spots[spot].histories;
+    return c->scen_budget.empty() ? h : (uint64_t) std::llround((double) h * c->scen_budget[scenario]);
+}
+
+// items are (scenario, spot) of the spots [first, end), scenario-major; empty
+// spots are skipped
 run_plan
-make_plan(const mqi_ctx* c, int only_spot) {
+make_plan(const mqi_ctx* c, size_t first, size_t end) {
     run_plan p;
     for (int s = 0; s < c->n_scen; ++s)
-        for (size_t j = 0; j < c->spots.size(); ++j) {
-            if (only_spot >= 0 && (int) j != only_spot) continue;
-            uint64_t h = c->spots[j].histories;
-            if (!c->scen_budget.empty()) h = (uint64_t) std::llround((double) h * c->scen_budget[s]);
+        for (size_t j = first; j < end; ++j) {
+            const uint64_t h = item_histories(c, s, j);
             if (h == 0) continue;
             p.total += h;
             p.max_item = std::max(p.max_item, h);
@@ -697,9 +703,13 @@ launch_bound(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int dyn
 // scorers (two: pairs of lanes; three or four: groups of four lanes) add
 // into one interleaved array, all sums of a voxel in one line and added by
 // one atomic instruction from the group, folded into their arrays after the
-// pass.
+// pass.  The fold reads the whole array (4 to 8 ps per voxel), the groups save
+// some 5 to 10 ns per history, so a pass of less than a history per
+// MQI_PAIR_VOXELS voxels scores ungrouped, as does (optional) one whose array
+// the device has no memory for.
+#define MQI_PAIR_VOXELS 1024
 int
-pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg) {
+pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, uint64_t histories, bool optional) {
     c->pair_n = 0;
     if (cfg.exact || cfg.dij || cfg.scoring_loops != MQI_LOOPS_ONCE) return 0;
     int ns = 0;
@@ -707,10 +717,15 @@ pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg) {
     if (ns < 2) return 0;
     const int    stride = ns == 2 ? 2 : 4;
     const size_t n      = (size_t) nvox(c) * (c->per_scen ? (size_t) c->n_scen : 1u);
+    if (histories * MQI_PAIR_VOXELS < n) return 0;
     if (stride * n > c->pair_cap) {
         dfree(c->d_pair);
         c->pair_cap = 0;
         int r = dalloc(c, &c->d_pair, stride * n);
+        if (r && optional) {
+            (void) hipGetLastError();
+            return 0;
+        }
         if (r) return r;
         KCHK(c, mqi_aux::fill_u64(c->d_pair, 0ull, stride * n, c->stream));
         c->pair_cap = stride * n;
@@ -729,6 +744,17 @@ int
 pair_fold(mqi_ctx* c) {
     if (c->pair_n)
         KCHK(c, mqi_aux::pair_fold(c->pair_real, c->pair_ns, c->pair_stride, c->d_pair, c->pair_n, c->stream));
+    return 0;
+}
+
+// waits for the stream and adds its time since ev0 to *ms
+int
+add_elapsed(mqi_ctx* c, double* ms) {
+    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
+    HIPCHK(c, hipEventSynchronize(c->ev1));
+    float t = 0;
+    HIPCHK(c, hipEventElapsedTime(&t, c->ev0, c->ev1));
+    *ms += t;
     return 0;
 }
 
@@ -828,17 +854,15 @@ graph_pass(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int block
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     HIPCHK(c, hipGraphLaunch(c->graph_exec, c->stream));
     if (int e = pair_fold(c)) return e;
-    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-    HIPCHK(c, hipEventSynchronize(c->ev1));
-    float t = 0;
-    HIPCHK(c, hipEventElapsedTime(&t, c->ev0, c->ev1));
-    *ms += t;
-    return 0;
+    return add_elapsed(c, ms);
 }
 
-// One pass over a plan: the persistent dynamic launch, or (plain) one static
-// launch per spot of the plan.  Adds the device time of the transport
-// kernels to *ms.
+// One pass over a plan: the persistent dynamic launch, or (plain) static
+// launches in the order of the spots, a lane per history.  Consecutive spots
+// share a plain launch while its lanes hold their histories: a launch of one
+// spot (2e3 .. 2e4 histories, 110 waves for 1024 SIMDs) lasts as long as its
+// longest track, and 40 of them took 82 ms where two shared ones take
+// 7.3.  Adds the device time of the transport kernels to *ms.
 int
 transport_pass(mqi_ctx* c, const mqi_run_config& cfg_in, uint64_t hoff, double* ms) {
     mqi_run_config cfg = cfg_in;
@@ -851,7 +875,7 @@ transport_pass(mqi_ctx* c, const mqi_run_config& cfg_in, uint64_t hoff, double* 
     const size_t lane_bytes = (size_t) P.stack_cap * MQI_STACK_FLOATS * sizeof(float);
     int          r;
     if (cfg.batched) {
-        run_plan p = make_plan(c, -1);
+        run_plan p = make_plan(c, 0, c->spots.size());
         if ((r = upload_plan(c, p))) return r;
         if (p.total == 0) return 0;
         P.n_items      = (int) p.item_end.size();
@@ -860,25 +884,28 @@ transport_pass(mqi_ctx* c, const mqi_run_config& cfg_in, uint64_t hoff, double* 
         const int blocks = persistent_blocks(c, cfg, threads, 0);
         if ((r = ensure_stack(c, lane_bytes * (size_t) blocks * threads))) return r;
         P.stack = c->d_stack;
-        if ((r = pair_setup(c, P, cfg))) return r;
+        if ((r = pair_setup(c, P, cfg, p.total, false))) return r;
         if (cfg.use_graph) return graph_pass(c, P, cfg, blocks, threads, ms);
         HIPCHK(c, hipEventRecord(c->ev0, c->stream));
         KCHK(c, launch(c, P, cfg, 1, 0, blocks, threads));
         if ((r = pair_fold(c))) return r;
-        HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-        HIPCHK(c, hipEventSynchronize(c->ev1));
-        float t = 0;
-        HIPCHK(c, hipEventElapsedTime(&t, c->ev0, c->ev1));
-        *ms += t;
-        return 0;
+        return add_elapsed(c, ms);
     }
-    // plain: per scenario, per spot
     const uint64_t max_lanes = 1ull << 18;
     const int      max_blocks = (int) ((max_lanes + threads - 1) / threads);
     if ((r = ensure_stack(c, lane_bytes * (size_t) max_blocks * threads))) return r;
     P.stack = c->d_stack;
-    for (size_t j = 0; j < c->spots.size(); ++j) {
-        run_plan p = make_plan(c, (int) j);
+    std::vector<uint64_t> hist(c->spots.size(), 0);
+    uint64_t              total = 0;
+    for (size_t j = 0; j < hist.size(); ++j) {
+        for (int s = 0; s < c->n_scen; ++s) hist[j] += item_histories(c, s, j);
+        total += hist[j];
+    }
+    if ((r = pair_setup(c, P, cfg, total, true))) return r;
+    for (size_t j = 0, end = 0; j < hist.size(); j = end) {
+        uint64_t n = hist[j];
+        for (end = j + 1; end < hist.size() && n + hist[end] <= max_lanes; ++end) n += hist[end];
+        run_plan p = make_plan(c, j, end);
         if (p.total == 0) continue;
         if ((r = upload_plan(c, p))) return r;
         P.n_items    = (int) p.item_end.size();
@@ -888,11 +915,11 @@ transport_pass(mqi_ctx* c, const mqi_run_config& cfg_in, uint64_t hoff, double* 
         int      blocks = (int) ((lanes + threads - 1) / threads);   // <= max_blocks
         HIPCHK(c, hipEventRecord(c->ev0, c->stream));
         KCHK(c, launch(c, P, cfg, 0, 0, blocks, threads));
-        HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-        HIPCHK(c, hipEventSynchronize(c->ev1));
-        float t = 0;
-        HIPCHK(c, hipEventElapsedTime(&t, c->ev0, c->ev1));
-        *ms += t;
+        if ((r = add_elapsed(c, ms))) return r;
+    }
+    if (c->pair_n) {
+        HIPCHK(c, hipEventRecord(c->ev0, c->stream));
+        if ((r = pair_fold(c)) || (r = add_elapsed(c, ms))) return r;
     }
     return 0;
 }
@@ -1284,7 +1311,7 @@ mqi_run(mqi_ctx* c, const mqi_run_config* cfg_in, mqi_run_result* res) {
     std::memset(&out, 0, sizeof out);
     out.stat          = -1.0;
     const int max_rounds = cfg.max_rounds > 0 ? cfg.max_rounds : 64;
-    run_plan  p          = make_plan(c, -1);
+    run_plan  p          = make_plan(c, 0, c->spots.size());
     // Dose and Dose_stat receive the same per-step value except in voxel 0
     // (excluded from Dose, mqi_roi.hpp): with each scorer scored once, score
     // Dose_stat only and derive Dose at the end of the run
@@ -1632,7 +1659,7 @@ mqi_trace(mqi_ctx* c, const mqi_run_config* cfg_in, const float* vertices, uint6
         HIPCHK(c, hipMemcpyAsync(d_v, vertices, sizeof(float) * 7 * n_hist, hipMemcpyHostToDevice, c->stream));
     } else {
         if (c->spots.empty()) return fail(c, MQI_E_STATE, "no spots");
-        p = make_plan(c, -1);
+        p = make_plan(c, 0, c->spots.size());
         if (p.total != n_hist) return fail(c, MQI_E_ARG, "trace: plan has %llu histories, caller expects %llu",
                                            (unsigned long long) p.total, (unsigned long long) n_hist);
     }

@@ -7,9 +7,10 @@
 //            atomic per wavefront refill (ballot + popcount), so a lane whose
 //            track ends takes the next secondary or history on the next
 //            iteration while its neighbours keep stepping.
-//   plain    one launch per spot, histories split statically over threads
-//            (the reference's mc::transport_particles_patient launch,
-//            mqi_transport.hpp:113-250, mqi_tps_env.hpp:1058-1129).
+//   plain    histories split statically over threads (the reference's
+//            mc::transport_particles_patient launch, mqi_transport.hpp:
+//            113-250, mqi_tps_env.hpp:1058-1129), consecutive spots sharing
+//            a launch while a lane per history holds them.
 //
 // Compiled twice: MQI_EXACT=1 (namespace mqi_exact, -ffp-contract=off,
 // portable math: bit-identical to the CPU restatement) and MQI_EXACT=0
