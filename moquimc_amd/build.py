@@ -3,8 +3,9 @@
     python -m moquimc_amd.build            # or: python moquimc_amd/build.py
 
 Translation units:
-  mqi_transport.hip  -> twice: MQI_EXACT=1 (-ffp-contract=off, portable math;
-                        the verification kernels) and MQI_EXACT=0 (production)
+  mqi_transport.hip  -> three times: MQI_EXACT=1 (-ffp-contract=off, portable
+                        math; the verification kernels), MQI_EXACT=0
+                        (production), and the same for five or six scorers
   mqi_aux.hip        -> fills, calibration, statistics, Dij CSR, sparse products
   mqi_api.cpp        -> the C ABI of include/mqi_hip.h
 """
@@ -51,10 +52,13 @@ def build(verbose=True):
             (os.path.join(CSRC, "mqi_transport.hip"), os.path.join(tmp, "transport_fast.o"),
              ["-DMQI_EXACT=0", "-ffp-contract=fast-honor-pragmas",
               "-fno-hip-fp32-correctly-rounded-divide-sqrt"]),
+            (os.path.join(CSRC, "mqi_transport.hip"), os.path.join(tmp, "transport_fast6.o"),
+             ["-DMQI_EXACT=0", "-DMQI_DEFER=6", "-ffp-contract=fast-honor-pragmas",
+              "-fno-hip-fp32-correctly-rounded-divide-sqrt"]),
             (os.path.join(CSRC, "mqi_aux.hip"), os.path.join(tmp, "aux.o"), ["-ffp-contract=off"]),
             (os.path.join(CSRC, "mqi_api.cpp"), os.path.join(tmp, "api.o"), ["-x", "hip", "-ffp-contract=off"]),
         ]
-        with ThreadPoolExecutor(max_workers=4) as ex:
+        with ThreadPoolExecutor(max_workers=5) as ex:
             objs = list(ex.map(_compile, jobs))
         out_tmp = LIB + ".tmp"
         cmd = [hipcc(), "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", out_tmp] + objs

@@ -522,11 +522,23 @@ upload_grid_common(mqi_ctx* c, int nx, int ny, int nz, const float* xe, const fl
     return dalloc(c, &c->d_density, nvox(c));
 }
 
+// Scorer slots summed per voxel by the kernels a launch runs: MQI_MAX_SCORERS
+// (mqi_fast6) for more than MQI_GROUP scorers, each scored once, if the LDS
+// holds their sums (and the waves' Dij queues) in 64 KB; else MQI_DEFER
+int
+deferred_slots(const mqi_ctx* c, const mqi_run_config& cfg, int threads) {
+    const int n = (int) c->kinds.size() - (c->alias_dose || c->dij_dose ? 1 : 0) + (cfg.dij ? 1 : 0);
+    if (n <= MQI_GROUP || cfg.exact || cfg.scoring_loops != MQI_LOOPS_ONCE) return MQI_DEFER;
+    const size_t q = cfg.dij ? mqi_dij_queue_bytes(threads) : 0;
+    return mqi_shmem_bytes(c->nx, c->ny, c->nz, c->bl_n_edges, threads, MQI_MAX_SCORERS) + q <= 65536 ? MQI_MAX_SCORERS
+                                                                                                      : MQI_DEFER;
+}
+
 // dynamic LDS of a transport launch; the waves' Dij queues are left out of a
 // production launch with the Dij scorer where they would not fit 64 KB
 size_t
 shmem_bytes(const mqi_ctx* c, const mqi_run_config& cfg, int threads, int* queued = nullptr) {
-    const size_t sh = mqi_shmem_bytes(c->nx, c->ny, c->nz, c->bl_n_edges, threads);
+    const size_t sh = mqi_shmem_bytes(c->nx, c->ny, c->nz, c->bl_n_edges, threads, deferred_slots(c, cfg, threads));
     const size_t q    = mqi_dij_queue_bytes(threads);
     const bool   with = cfg.dij && !cfg.exact && cfg.scoring_loops == MQI_LOOPS_ONCE && sh + q <= 65536;
     if (queued) *queued = with ? 1 : 0;
@@ -694,6 +706,9 @@ launch_bound(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int dyn
     }
     if (cfg.exact)
         return mqi_exact::launch_transport(P, cfg.physics_debug, dynamic, trace, 0, blocks, threads, sh, c->stream);
+    if (deferred_slots(c, cfg, threads) > MQI_DEFER)
+        return mqi_fast6::launch_transport(P, cfg.physics_debug, dynamic, trace, cfg.waves_per_simd, blocks, threads,
+                                           sh, c->stream);
     return mqi_fast::launch_transport(P, cfg.physics_debug, dynamic, trace, cfg.waves_per_simd, blocks, threads, sh,
                                       c->stream);
 }
@@ -713,7 +728,7 @@ pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, uint64_t 
     c->pair_n = 0;
     if (cfg.exact || cfg.dij || cfg.scoring_loops != MQI_LOOPS_ONCE) return 0;
     int ns = 0;
-    while (ns < P.n_scorers && ns < MQI_DEFER && P.kinds[ns] != MQI_KIND_DIJ) ++ns;
+    while (ns < P.n_scorers && ns < MQI_GROUP && P.kinds[ns] != MQI_KIND_DIJ) ++ns;
     if (ns < 2) return 0;
     const int    stride = ns == 2 ? 2 : 4;
     const size_t n      = (size_t) nvox(c) * (c->per_scen ? (size_t) c->n_scen : 1u);
@@ -797,8 +812,10 @@ int
 persistent_blocks(mqi_ctx* c, const mqi_run_config& cfg, int threads, int trace) {
     if (cfg.blocks > 0) return cfg.blocks;
     const size_t sh  = shmem_bytes(c, cfg, threads);
-    int          occ = cfg.exact ? mqi_exact::occupancy(cfg.physics_debug, 1, trace, 0, threads, sh)
-                                 : mqi_fast::occupancy(cfg.physics_debug, 1, trace, cfg.waves_per_simd, threads, sh);
+    const auto   of  = cfg.exact                                         ? mqi_exact::occupancy
+                       : deferred_slots(c, cfg, threads) > MQI_DEFER ? mqi_fast6::occupancy
+                                                                     : mqi_fast::occupancy;
+    const int    occ = of(cfg.physics_debug, 1, trace, cfg.exact ? 0 : cfg.waves_per_simd, threads, sh);
     return c->n_cu * occ;
 }
 
@@ -1541,8 +1558,10 @@ mqi_run_vertices(mqi_ctx* c, const float* vtx, uint64_t n, const uint32_t* spot_
     }
     if ((r = ensure_stack(c, (size_t) P.stack_cap * MQI_STACK_FLOATS * sizeof(float) * (size_t) blocks * threads))) return r;
     P.stack = c->d_stack;
+    if ((r = pair_setup(c, P, cfg, n, true))) return r;
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     KCHK(c, launch(c, P, cfg, cfg.batched ? 1 : 0, 0, blocks, threads));
+    if ((r = pair_fold(c))) return r;
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, hipEventSynchronize(c->ev1));
     float t = 0;

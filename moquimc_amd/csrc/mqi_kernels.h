@@ -31,18 +31,22 @@ enum {
 };
 
 // Scorer slots whose deposits a lane sums per voxel before one atomic add
-// (the rest are added per step), and where those sums sit in the dynamic LDS
-// of the transport kernel: after the six 600-entry tables, the three edge
-// arrays and the beamline edges, at an 8-byte boundary, MQI_DEFER doubles
-// per thread.
-#define MQI_DEFER 4
+// (the rest are added per step): MQI_DEFER, or all of them in the kernels
+// built for more scorers (mqi_fast6).  At most MQI_GROUP are added by groups
+// of lanes.  The sums sit in the dynamic LDS of the transport kernel: after
+// the six 600-entry tables, the three edge arrays and the beamline edges, at
+// an 8-byte boundary, one double per slot and thread.
+#define MQI_GROUP 4
+#ifndef MQI_DEFER
+#define MQI_DEFER MQI_GROUP
+#endif
 #define MQI_LDS_TABLE_FLOATS 3600
 __host__ __device__ inline uint32_t mqi_pend_offset(int nx, int ny, int nz, int bl_edges) {
     const uint32_t f = MQI_LDS_TABLE_FLOATS + (uint32_t) (nx + 1 + ny + 1 + nz + 1 + bl_edges);
     return (f + 1u) & ~1u;
 }
-__host__ __device__ inline size_t mqi_shmem_bytes(int nx, int ny, int nz, int bl_edges, int threads) {
-    return sizeof(float) * (size_t) mqi_pend_offset(nx, ny, nz, bl_edges) + sizeof(double) * MQI_DEFER * (size_t) threads;
+__host__ __device__ inline size_t mqi_shmem_bytes(int nx, int ny, int nz, int bl_edges, int threads, int slots) {
+    return sizeof(float) * (size_t) mqi_pend_offset(nx, ny, nz, bl_edges) + sizeof(double) * (size_t) slots * threads;
 }
 
 // Production launches with the Dij scorer: behind the pending sums, a queue
@@ -179,6 +183,12 @@ int launch_transport(const transport_params& P, int debug, int dynamic, int trac
                      int threads, size_t shmem, hipStream_t stream);
 int occupancy(int debug, int dynamic, int trace, int waves, int threads, size_t shmem);
 int physics_probe(int debug, int fn, const float* rho, const float* ek, int64_t n, float* out, hipStream_t stream);
+}
+namespace mqi_fast6   // the production kernels with every scorer slot summed per voxel
+{
+int launch_transport(const transport_params& P, int debug, int dynamic, int trace, int waves, int blocks,
+                     int threads, size_t shmem, hipStream_t stream);
+int occupancy(int debug, int dynamic, int trace, int waves, int threads, size_t shmem);
 }
 namespace mqi_exact
 {

@@ -12,9 +12,14 @@
 //            113-250, mqi_tps_env.hpp:1058-1129), consecutive spots sharing
 //            a launch while a lane per history holds them.
 //
-// Compiled twice: MQI_EXACT=1 (namespace mqi_exact, -ffp-contract=off,
-// portable math: bit-identical to the CPU restatement) and MQI_EXACT=0
-// (namespace mqi_fast, device math library, FMA contraction).
+// Compiled three times: MQI_EXACT=1 (namespace mqi_exact, -ffp-contract=off,
+// portable math: bit-identical to the CPU restatement), MQI_EXACT=0
+// (namespace mqi_fast, device math library, FMA contraction), and the latter
+// again with MQI_DEFER=6 (namespace mqi_fast6) for launches of five or six
+// scorers.  A fifth scorer added on every step cost 2.5 ms of the 11.9 of 3e5
+// histories with dose and four LET scorers (9.4 with its sum in LDS too);
+// built into mqi_fast the two slots cost every launch registers (143 -> 153
+// VGPRs, Dij field 18.9 -> 20.1 ms).
 #include "mqi_device.hpp"
 #include "mqi_kernels.h"
 #if MQI_EXACT
@@ -29,6 +34,8 @@
 
 #if MQI_EXACT
 #define MQI_NS mqi_exact
+#elif MQI_DEFER > MQI_GROUP
+#define MQI_NS mqi_fast6
 #else
 #define MQI_NS mqi_fast
 #endif
@@ -1121,6 +1128,17 @@ MQI_DI void flush_quad(const transport_params& P, const scoring& S, pending& A, 
         if (x2 != 0.0) atomicAdd(P.pair_out + k + 2, x2);
         if (x3 != 0.0) atomicAdd(P.pair_out + k + 3, x3);
     }
+#if MQI_DEFER > MQI_GROUP
+    // the scorers behind the group, each into its own array
+    if (has) {
+#pragma unroll
+        for (int s = MQI_GROUP; s < MQI_DEFER; ++s) {
+            if (s >= S.n()) break;
+            const double x = v[s * blockDim.x];
+            if (x != 0.0) atomicAdd(P.out[s] + (k >> 2), x);
+        }
+    }
+#endif
     if (has) A.cnb = -1;
 }
 #endif
@@ -1845,6 +1863,7 @@ launch_transport(const transport_params& P, int debug, int dynamic, int trace, i
     return (int) hipGetLastError();
 }
 
+#if MQI_DEFER == MQI_GROUP
 // Verification probes of the material and physics functions as the
 // transport kernels evaluate them: fn 0 spr (rho, ek), fn 1 radiation length
 // (rho), fn 2 per (rho, ek) the four cross sections at rho, dEdx and the
@@ -1919,6 +1938,8 @@ physics_probe(int debug, int fn, const float* rho, const float* ek, int64_t n, f
         hipLaunchKernelGGL(k_physics_probe<false>, grid, dim3(256), 0, stream, fn, rho, ek, n, out);
     return (int) hipGetLastError();
 }
+
+#endif
 
 // resident workgroups per CU of one instantiation
 int
