@@ -220,6 +220,20 @@ int mqi_dij_matvec(mqi_ctx* ctx, int scenario, int transpose, const float* x, vo
 int mqi_dij_quadratic(mqi_ctx* ctx, int scenario, const float* w, const double* p, const float* c, double alpha,
                       float* g, double* f, void* stream);
 
+/* The objective's values of several scenarios' dose of one w: f[i] (device
+ * doubles) is mqi_dij_quadratic's *f of scenario scenarios[i] with alpha[i]
+ * (host arrays), to the bit, from one pass of launches over all of them.  The
+ * scenarios are distinct and their matrices of one size. */
+int mqi_dij_quadratics(mqi_ctx* ctx, int n, const int32_t* scenarios, const double* alpha, const float* w,
+                       const double* p, const float* c, double* f, void* stream);
+
+/* y = alpha * D^T x, times *up (a device double) when up is set: the product
+ * of mqi_dij_matvec with transpose = 1 for the backward pass.  x: device
+ * float32, or float64 (x_double; rounded to float32 as it is read); y: device
+ * float64 (y_double) or float32. */
+int mqi_dij_adjoint(mqi_ctx* ctx, int scenario, const void* x, int x_double, const double* up, double alpha, void* y,
+                    int y_double, void* stream);
+
 /* Region of interest of the scorers (target 0: Dose, LETd, LETt, Edep, Dm
  * and Dij) or of the statistics pair (target 1), from a voxel mask (x
  * fastest, the grid's size; the reference's mask_total, the sum of the

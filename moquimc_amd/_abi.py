@@ -85,6 +85,8 @@ def lib():
             "mqi_dij_copy": (i, [vp, i, vp, vp, vp]),
             "mqi_dij_set_csr": (i, [vp, i, ctypes.c_int64, ctypes.c_int64, vp, vp, vp]),
             "mqi_dij_quadratic": (i, [vp, i, vp, vp, vp, d, vp, vp, vp]),
+            "mqi_dij_quadratics": (i, [vp, i, vp, vp, vp, vp, vp, vp, vp]),
+            "mqi_dij_adjoint": (i, [vp, i, vp, i, vp, d, vp, i, vp]),
             "mqi_dij_device_ptrs": (i, [vp, i, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(vp)]),
             "mqi_dij_matvec": (i, [vp, i, i, vp, vp, i, d, i, vp]),
             "mqi_last_matvec_ms": (i, [vp, ctypes.POINTER(d)]),
@@ -110,6 +112,7 @@ EXPORTED = ["mqi_create", "mqi_destroy", "mqi_last_error", "mqi_device_info", "m
             "mqi_get_density", "mqi_set_spots", "mqi_set_scenarios", "mqi_set_scorers", "mqi_zero_scorers",
             "mqi_scorer_count", "mqi_run", "mqi_run_vertices", "mqi_trace", "mqi_get_scorer",
             "mqi_scorer_device_ptr", "mqi_stat", "mqi_dij_build", "mqi_dij_info", "mqi_dij_copy", "mqi_dij_set_csr", "mqi_dij_quadratic",
+            "mqi_dij_quadratics", "mqi_dij_adjoint",
             "mqi_dij_device_ptrs", "mqi_dij_matvec", "mqi_last_matvec_ms", "mqi_math_probe", "mqi_autotune",
             "mqi_dij_save_npz", "mqi_save_scorer", "mqi_set_grid_ct_mha", "mqi_set_beamline", "mqi_set_roi", "mqi_set_roi_mha",
             "mqi_physics_probe", "mqi_run_vertices_noalloc", "mqi_atomic_probe"]
@@ -433,6 +436,25 @@ class Context:
                                             ctypes.c_void_p(g_ptr or None), ctypes.c_void_p(f_ptr),
                                             None if stream is None else ctypes.c_void_p(stream)),
                   "mqi_dij_quadratic")
+
+    def dij_quadratics(self, scenarios, alphas, w_ptr, p_ptr, c_ptr, f_ptr, stream=None):
+        """dij_quadratic's f of several scenarios into f_ptr[i]
+        (mqi_dij_quadratics)."""
+        n = len(scenarios)
+        self._chk(self._L.mqi_dij_quadratics(self.h, n, (ctypes.c_int32 * n)(*scenarios),
+                                             (ctypes.c_double * n)(*alphas), ctypes.c_void_p(w_ptr),
+                                             ctypes.c_void_p(p_ptr), ctypes.c_void_p(c_ptr or None),
+                                             ctypes.c_void_p(f_ptr),
+                                             None if stream is None else ctypes.c_void_p(stream)),
+                  "mqi_dij_quadratics")
+
+    def dij_adjoint(self, scenario, x_ptr, x_double, up_ptr, alpha, y_ptr, y_double, stream=None):
+        """y = alpha D^T x (times the device double at up_ptr, unless 0)
+        (mqi_dij_adjoint)."""
+        self._chk(self._L.mqi_dij_adjoint(self.h, scenario, ctypes.c_void_p(x_ptr), int(x_double),
+                                          ctypes.c_void_p(up_ptr or None), ctypes.c_double(alpha),
+                                          ctypes.c_void_p(y_ptr), int(y_double),
+                                          None if stream is None else ctypes.c_void_p(stream)), "mqi_dij_adjoint")
 
     def last_matvec_ms(self):
         ms = ctypes.c_double()

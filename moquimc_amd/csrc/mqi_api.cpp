@@ -2096,6 +2096,45 @@ mqi_dij_device_ptrs(mqi_ctx* c, int s, const int64_t** indptr, const int32_t** i
     return 0;
 }
 
+namespace
+{
+// D^T x of a scenario's Dij: y = alpha * D^T x (* *up) (+ y); x float, or
+// double rounded to float
+int
+adjoint(mqi_ctx* c, const csr_dev& m, const void* x, int x_double, const double* up, double alpha, void* y,
+        int y_double, int accumulate, hipStream_t st) {
+    const csr_plan& p = m.plan;
+    // the x of the voxels with a nonzero (12 MB instead of 33.5 MB on the
+    // 5000-spot plan)
+    const bool compact = m.sval || m.ccol;
+    if (compact) KCHK(c, mqi_aux::gather_x(x, x_double, m.nzvox, m.n_nz, m.xc, st));
+    if (m.sval)   // pieces over byte column deltas
+        KCHK(c, mqi_aux::pieces_staged(m.sval, m.sd8, m.pesc, m.xc, m.phdr, m.n_piece, m.row_piece, m.rows, m.ppart,
+                                       y, y_double, alpha, up, accumulate, st));
+    else
+        KCHK(c, mqi_aux::csr_adaptive(m.indptr, compact ? m.ccol : m.col, m.val, compact ? m.xc : (const float*) x,
+                                      p.seg_k, p.seg_info, p.n_seg, p.split_seg, p.n_split, p.part, y, y_double,
+                                      alpha, up, accumulate, nullptr, nullptr, 0, st));
+    return 0;
+}
+
+// the D w matrix of a scenario as the objective's kernels read it
+int
+quad_matrix(mqi_ctx* c, int s, double alpha, mqi_aux::quad_mat& q) {
+    if (s < 0 || s >= (int) c->dij.size()) return fail(c, MQI_E_STATE, "no Dij for scenario %d", s);
+    csr_dev& m = c->dij[s];
+    if (m.nnz == 0) return fail(c, MQI_E_STATE, "scenario %d's Dij has no nonzeros", s);
+    csr_plan& P = m.tplan;
+    int       r = 0;
+    if (!P.qpart &&
+        (r = dalloc(c, &P.qpart, P.n_seg + P.n_split + MQI_QUAD_EMPTY_BLOCKS + MQI_QUAD_SUM_BLOCKS)))
+        return r;
+    q = { m.tindptr, m.tcol16 ? (const void*) m.tcol16 : (const void*) m.tcol, m.tval, P.seg_k, P.seg_info,
+          P.split_seg, m.nzvox, m.tnonempty, P.part, P.qpart, P.n_seg, P.n_split, alpha, 0 };
+    return 0;
+}
+}   // namespace
+
 int
 mqi_dij_matvec(mqi_ctx* c, int s, int transpose, const float* x, void* y, int y_double, double alpha, int accumulate,
                void* stream) {
@@ -2106,24 +2145,7 @@ mqi_dij_matvec(mqi_ctx* c, int s, int transpose, const float* x, void* y, int y_
     hipStream_t    st = stream ? (hipStream_t) stream : c->stream;
     HIPCHK(c, hipEventRecord(c->ev_mv0, st));
     if (transpose) {
-        // D^T g: rows of the spot-major matrix
-        const csr_plan& p = m.plan;
-        if (m.sval) {   // pieces over byte column deltas of the compacted x
-            KCHK(c, mqi_aux::gather_x(x, m.nzvox, m.n_nz, m.xc, st));
-            KCHK(c, mqi_aux::pieces_staged(m.sval, m.sd8, m.pesc, m.xc, m.phdr, m.n_piece, m.row_piece, m.rows,
-                                           m.ppart, y, y_double, alpha, accumulate, st));
-        } else {
-            const int32_t* colp = m.col;
-            const float*   xp   = x;
-            if (m.ccol) {   // gather from the compacted x (12 MB instead of 33.5 MB on the 5000-spot plan)
-                KCHK(c, mqi_aux::gather_x(x, m.nzvox, m.n_nz, m.xc, st));
-                colp = m.ccol;
-                xp   = m.xc;
-            }
-            KCHK(c, mqi_aux::csr_adaptive(m.indptr, colp, m.val, xp, p.seg_k, p.seg_info, p.n_seg, p.split_seg,
-                                          p.n_split, p.part, y, y_double, alpha, accumulate, nullptr, nullptr, 0,
-                                          st));
-        }
+        if (int r = adjoint(c, m, x, 0, nullptr, alpha, y, y_double, accumulate, st)) return r;
     } else if (m.nnz == 0) {
         // D w of an empty matrix: zeros (or y unchanged)
         if (!accumulate) {
@@ -2138,13 +2160,29 @@ mqi_dij_matvec(mqi_ctx* c, int s, int transpose, const float* x, void* y, int y_
         const csr_plan& p = m.tplan;
         if (m.tcol16)
             KCHK(c, mqi_aux::csr_adaptive16(m.tindptr, m.tcol16, m.tval, x, p.seg_k, p.seg_info, p.n_seg,
-                                            p.split_seg, p.n_split, p.part, y, y_double, alpha, accumulate, m.nzvox,
-                                            m.tnonempty, m.cols, st));
+                                            p.split_seg, p.n_split, p.part, y, y_double, alpha, nullptr, accumulate,
+                                            m.nzvox, m.tnonempty, m.cols, st));
         else
             KCHK(c, mqi_aux::csr_adaptive(m.tindptr, m.tcol, m.tval, x, p.seg_k, p.seg_info, p.n_seg, p.split_seg,
-                                          p.n_split, p.part, y, y_double, alpha, accumulate, m.nzvox, m.tnonempty,
-                                          m.cols, st));
+                                          p.n_split, p.part, y, y_double, alpha, nullptr, accumulate, m.nzvox,
+                                          m.tnonempty, m.cols, st));
     }
+    HIPCHK(c, hipEventRecord(c->ev_mv1, st));
+    c->matvec_pending = true;
+    return 0;
+}
+
+int
+mqi_dij_adjoint(mqi_ctx* c, int s, const void* x, int x_double, const double* up, double alpha, void* y, int y_double,
+                void* stream) {
+    if (!c || !x || !y) return MQI_E_ARG;
+    if (s < 0 || s >= (int) c->dij.size()) return fail(c, MQI_E_STATE, "no Dij for scenario %d", s);
+    hipSetDevice(c->device);
+    const csr_dev& m = c->dij[s];
+    if (x_double && !m.sval && !m.ccol && m.nnz) return fail(c, MQI_E_STATE, "scenario %d's Dij takes float vectors", s);
+    hipStream_t st = stream ? (hipStream_t) stream : c->stream;
+    HIPCHK(c, hipEventRecord(c->ev_mv0, st));
+    if (int r = adjoint(c, m, x, x_double, up, alpha, y, y_double, 0, st)) return r;
     HIPCHK(c, hipEventRecord(c->ev_mv1, st));
     c->matvec_pending = true;
     return 0;
@@ -2154,31 +2192,38 @@ int
 mqi_dij_quadratic(mqi_ctx* c, int s, const float* w, const double* p, const float* cw, double alpha, float* g,
                   double* f, void* stream) {
     if (!c || !w || !p || !f) return MQI_E_ARG;
-    if (s < 0 || s >= (int) c->dij.size()) return fail(c, MQI_E_STATE, "no Dij for scenario %d", s);
     hipSetDevice(c->device);
-    csr_dev& m = c->dij[s];
-    if (m.nnz == 0) return fail(c, MQI_E_STATE, "scenario %d's Dij has no nonzeros", s);
-    csr_plan& P = m.tplan;
-    int       r = 0;
-    if (!P.qpart &&
-        (r = dalloc(c, &P.qpart, P.n_seg + P.n_split + MQI_QUAD_EMPTY_BLOCKS + MQI_QUAD_SUM_BLOCKS)))
-        return r;
-    hipStream_t       st = stream ? (hipStream_t) stream : c->stream;
-    mqi_aux::quad_obj o;
-    o.p         = p;
-    o.c         = cw;
-    o.g         = g;
-    o.part      = P.qpart;
-    o.two_inv_n = 2.0 / (double) m.cols;
-    o.n_seg     = P.n_seg;
-    const double inv_n = 1.0 / (double) m.cols;
+    mqi_aux::quad_mat q;
+    if (int r = quad_matrix(c, s, alpha, q)) return r;
+    const csr_dev& m  = c->dij[s];
+    hipStream_t    st = stream ? (hipStream_t) stream : c->stream;
     HIPCHK(c, hipEventRecord(c->ev_mv0, st));
-    if (m.tcol16)
-        KCHK(c, mqi_aux::csr_quadratic16(m.tindptr, m.tcol16, m.tval, w, P.seg_k, P.seg_info, P.n_seg, P.split_seg,
-                                         P.n_split, P.part, alpha, o, inv_n, f, m.nzvox, m.tnonempty, m.cols, st));
-    else
-        KCHK(c, mqi_aux::csr_quadratic(m.tindptr, m.tcol, m.tval, w, P.seg_k, P.seg_info, P.n_seg, P.split_seg,
-                                       P.n_split, P.part, alpha, o, inv_n, f, m.nzvox, m.tnonempty, m.cols, st));
+    KCHK(c, mqi_aux::csr_quadratic(&q, 1, m.tcol16 != nullptr, w, p, cw, g, m.cols, f, st));
+    HIPCHK(c, hipEventRecord(c->ev_mv1, st));
+    c->matvec_pending = true;
+    return 0;
+}
+
+int
+mqi_dij_quadratics(mqi_ctx* c, int n, const int32_t* scenarios, const double* alpha, const float* w, const double* p,
+                   const float* cw, double* f, void* stream) {
+    if (!c || n < 1 || !scenarios || !alpha || !w || !p || !f) return MQI_E_ARG;
+    hipSetDevice(c->device);
+    std::vector<mqi_aux::quad_mat> q((size_t) n);
+    for (int i = 0; i < n; ++i) {
+        if (int r = quad_matrix(c, scenarios[i], alpha[i], q[i])) return r;
+        const csr_dev &a = c->dij[scenarios[0]], &b = c->dij[scenarios[i]];
+        if (a.rows != b.rows || a.cols != b.cols)
+            return fail(c, MQI_E_ARG, "scenarios %d and %d differ in size", scenarios[0], scenarios[i]);
+        for (int j = 0; j < i; ++j)   // its terms' place is one
+            if (scenarios[j] == scenarios[i]) return fail(c, MQI_E_ARG, "scenario %d is listed twice", scenarios[i]);
+    }
+    const csr_dev& m  = c->dij[scenarios[0]];
+    hipStream_t    st = stream ? (hipStream_t) stream : c->stream;
+    HIPCHK(c, hipEventRecord(c->ev_mv0, st));
+    for (int i = 0; i < n; i += MQI_QUAD_MATS)
+        KCHK(c, mqi_aux::csr_quadratic(q.data() + i, std::min(n - i, MQI_QUAD_MATS), m.tcol16 != nullptr, w, p, cw,
+                                       nullptr, m.cols, f + i, st));
     HIPCHK(c, hipEventRecord(c->ev_mv1, st));
     c->matvec_pending = true;
     return 0;

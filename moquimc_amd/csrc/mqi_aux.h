@@ -63,44 +63,53 @@ int spot_rows(const uint64_t* ranked, const int32_t* nzvox, int64_t n, int32_t* 
 // matrix stored without its empty rows (rowmap set) writes y = 0 at the n_y
 // elements whose bit in nonempty is clear, from MQI_ZERO_BLOCKS workgroups of
 // the same launch (with accumulate it leaves them alone).
+// up (device, may be NULL): y = alpha * A x * *up.
 #define MQI_ZERO_BLOCKS 1024
 int csr_adaptive(const int64_t* indptr, const int32_t* col, const float* val, const float* x, const int64_t* seg_k,
                  const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-                 void* y, int y_is_double, double alpha, int accumulate, const int32_t* rowmap,
+                 void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
                  const uint32_t* nonempty, int64_t n_y, hipStream_t s);
 // the same over 16-bit columns (D w of a Dij with at most 65536 spots)
 int csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, const int64_t* seg_k,
                    const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-                   void* y, int y_is_double, double alpha, int accumulate, const int32_t* rowmap,
+                   void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
                    const uint32_t* nonempty, int64_t n_y, hipStream_t s);
-// The quadratic objective of y = alpha * A x on the D w matrix, without y:
-// f = inv_n * sum_r c_r (y_r - p_r)^2 (c NULL: 1) into *f (device), and
-// g_r = two_inv_n * c_r (y_r - p_r) (float32, when g is set).  part: n_seg +
-// n_split doubles of per-segment and per-split-row terms, summed in a fixed
-// order.  With rowmap the matrix has no empty rows: the n_y elements whose
-// bit in nonempty is clear (d = 0) get their terms from a fixed grid of
-// MQI_QUAD_EMPTY_BLOCKS workgroups (part then holds n_seg + n_split +
-// MQI_QUAD_EMPTY_BLOCKS doubles).
+// The quadratic objective of y = alpha * A x on the D w matrices of up to
+// MQI_QUAD_MATS scenarios, without y: f[i] = mean over the n_y elements of
+// c (y_i - p)^2 (c NULL: 1; f on the device) and, for a single matrix, g =
+// 2 / n_y * c (y - p) (float32, when g is set).  terms: n_seg + n_split +
+// MQI_QUAD_EMPTY_BLOCKS + MQI_QUAD_SUM_BLOCKS doubles, the terms of the
+// segments, of the split rows and (rowmap: the matrix has no empty rows) of
+// up to MQI_QUAD_EMPTY_BLOCKS workgroups over the elements whose bit in
+// nonempty is clear (y = 0), summed in a fixed order that depends on the
+// matrix alone.
+#define MQI_QUAD_MATS 16
 #define MQI_QUAD_EMPTY_BLOCKS 2048
-// the terms are summed in MQI_QUAD_SUM_BLOCKS fixed chunks, then the chunk
-// sums (part holds MQI_QUAD_SUM_BLOCKS more doubles for them)
 #define MQI_QUAD_SUM_BLOCKS 256
+#define MQI_QUAD_ONE 32768   // terms that one workgroup sums
 struct quad_obj {
     const double* p;
     const float*  c;
     float*        g;
-    double*       part;
+    double*       part;   // the segments' terms
     double        two_inv_n;
-    int64_t       n_seg;
 };
-int csr_quadratic(const int64_t* indptr, const int32_t* col, const float* val, const float* x, const int64_t* seg_k,
-                  const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-                  double alpha, quad_obj o, double inv_n, double* f, const int32_t* rowmap, const uint32_t* nonempty,
-                  int64_t n_y, hipStream_t s);
-int csr_quadratic16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x,
-                    const int64_t* seg_k, const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg,
-                    int64_t n_split, double* part, double alpha, quad_obj o, double inv_n, double* f,
-                    const int32_t* rowmap, const uint32_t* nonempty, int64_t n_y, hipStream_t s);
+struct quad_mat {
+    const int64_t*  indptr;
+    const void*     col;
+    const float*    val;
+    const int64_t*  seg_k;
+    const uint32_t* seg_info;
+    const int32_t*  split_seg;
+    const int32_t*  rowmap;
+    const uint32_t* nonempty;
+    double *        part, *terms;
+    int64_t         n_seg, n_split;
+    double          alpha;
+    uint32_t        empty;   // workgroups of the elements without a row (set by csr_quadratic)
+};
+int csr_quadratic(const quad_mat* mats, int n, int cols16, const float* x, const double* p, const float* c, float* g,
+                  int64_t n_y, double* f, hipStream_t s);
 // D^T g over column deltas (mqi_aux.hip): the 16-bit deltas of each row's
 // columns (0 at row starts and where a row skips more than 65535 columns,
 // those positions listed in gaps), the column before each piece's first
@@ -131,9 +140,9 @@ struct alignas(16) piece_hdr {
 };
 int pieces_staged(const float* sval, const uint8_t* sd8, const uint16_t* esc, const float* x, const piece_hdr* hdr,
                   int64_t n_p, const int32_t* row_piece, int64_t rows, double* part, void* y, int y_is_double,
-                  double alpha, int accumulate, hipStream_t s);
-// D^T g on compacted x: xc = x[nzvox]
-int gather_x(const float* x, const int32_t* nzvox, int64_t n, float* xc, hipStream_t s);
+                  double alpha, const double* up, int accumulate, hipStream_t s);
+// D^T g on compacted x (float, or double rounded to float): xc = x[nzvox]
+int gather_x(const void* x, int x_double, const int32_t* nzvox, int64_t n, float* xc, hipStream_t s);
 // grouped scoring: out[s][i] += pair[stride i + s] for s < ns, i < n (stride
 // 2 or 4), pair cleared
 int pair_fold(double* const* out, int ns, int stride, double* pair, uint64_t n, hipStream_t s);

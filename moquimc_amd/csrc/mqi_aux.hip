@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
+
 #include "mqi_aux.h"
 #include "mqi_device.hpp"
 #include "mqi_kernels.h"
@@ -584,42 +586,19 @@ static_assert(MQI_SEG_SHORT <= 1024, "packed segments are loaded as at most 256 
 
 // OBJ: instead of y, the quadratic objective of y (quad_obj): per row
 // c_r (y_r - p_r)^2 summed over each packed segment into o.part[s] (0 for a
-// long-row segment, whose rows k_csr_split_rows finishes), and
+// long-row segment, whose rows k_quad_split finishes), and
 // o.g[r] = two_inv_n c_r (y_r - p_r) when o.g is set
 template<typename TY, typename TC, bool OBJ>
-__global__ void __launch_bounds__(64) k_csr_adaptive(const int64_t* __restrict__ indptr,
-                                                     const TC* __restrict__ col,
-                                                     const float* __restrict__ val, const float* __restrict__ x,
-                                                     const int64_t* __restrict__ seg_k,
-                                                     const uint32_t* __restrict__ seg_info, int64_t n_seg,
-                                                     double* __restrict__ part, TY* __restrict__ y, double alpha,
-                                                     int accumulate, quad_obj o,
-                                                     const int32_t* __restrict__ rowmap,
-                                                     const uint32_t* __restrict__ nonempty, int64_t n_y,
-                                                     int zero_blocks) {
+MQI_DI void csr_walk(const int64_t* __restrict__ indptr, const TC* __restrict__ col, const float* __restrict__ val,
+                     const float* __restrict__ x, const int64_t* __restrict__ seg_k,
+                     const uint32_t* __restrict__ seg_info, int64_t first, int64_t stride, int64_t n_seg,
+                     double* __restrict__ part, TY* __restrict__ y, double alpha, const double* __restrict__ up,
+                     int accumulate, const quad_obj& o, const int32_t* __restrict__ rowmap) {
     __shared__ double buf[MQI_SEG_SHORT];
     const int lane = threadIdx.x;
-    // the first zero_blocks workgroups write y = 0 at the elements no row
-    // reaches (bit clear in nonempty), alongside the segments' workgroups
-    if ((int) blockIdx.x < zero_blocks) {
-        // eight elements per lane and pass, their mask words loaded together
-        const int64_t zs = (int64_t) zero_blocks * 64;
-        for (int64_t v0 = (int64_t) blockIdx.x * 64 + lane; v0 < n_y; v0 += 8 * zs) {
-            uint32_t bits[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) bits[j] = (v0 + j * zs < n_y) ? nonempty[(v0 + j * zs) >> 5] : 0xffffffffu;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int64_t v = v0 + j * zs;
-                if (v < n_y && !((bits[j] >> (v & 31)) & 1u)) y[v] = (TY) 0;
-            }
-        }
-        return;
-    }
     // plain grid-stride walk: a remap giving each XCD a contiguous run of
     // segments measured ~7 % slower on the 5000-spot Dij
-    const int64_t stride = (int64_t) gridDim.x - zero_blocks;
-    for (int64_t s = (int64_t) blockIdx.x - zero_blocks; s < n_seg; s += stride) {
+    for (int64_t s = first; s < n_seg; s += stride) {
         const uint32_t info = seg_info[s];
         const int64_t  kb = seg_k[s], ke = seg_k[s + 1];
         if (info >> 31) {
@@ -726,7 +705,7 @@ __global__ void __launch_bounds__(64) k_csr_adaptive(const int64_t* __restrict__
                 }
                 for (int off = L >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
                 if (r < r1 && sub == 0) {
-                    const double out = alpha * acc;
+                    const double out = up ? alpha * acc * *up : alpha * acc;
                     if (OBJ) {
                         const double res = out - pr;
                         obj += cw * res * res;
@@ -745,107 +724,137 @@ __global__ void __launch_bounds__(64) k_csr_adaptive(const int64_t* __restrict__
     }
 }
 
-// rows split over partial segments [split_seg[2i], split_seg[2i+1]):
-// y[r] = alpha * sum of the pieces in order (+ y[r])
-template<typename TY, bool OBJ>
+// up (device): y = alpha * A x * *up, rounded as the two products
+template<typename TY, typename TC>
+__global__ void __launch_bounds__(64) k_csr_adaptive(const int64_t* __restrict__ indptr,
+                                                     const TC* __restrict__ col,
+                                                     const float* __restrict__ val, const float* __restrict__ x,
+                                                     const int64_t* __restrict__ seg_k,
+                                                     const uint32_t* __restrict__ seg_info, int64_t n_seg,
+                                                     double* __restrict__ part, TY* __restrict__ y, double alpha,
+                                                     const double* __restrict__ up, int accumulate,
+                                                     const int32_t* __restrict__ rowmap,
+                                                     const uint32_t* __restrict__ nonempty, int64_t n_y,
+                                                     int zero_blocks) {
+    const int lane = threadIdx.x;
+    // the first zero_blocks workgroups write y = 0 at the elements no row
+    // reaches (bit clear in nonempty), alongside the segments' workgroups
+    if ((int) blockIdx.x < zero_blocks) {
+        // eight elements per lane and pass, their mask words loaded together
+        const int64_t zs = (int64_t) zero_blocks * 64;
+        for (int64_t v0 = (int64_t) blockIdx.x * 64 + lane; v0 < n_y; v0 += 8 * zs) {
+            uint32_t bits[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) bits[j] = (v0 + j * zs < n_y) ? nonempty[(v0 + j * zs) >> 5] : 0xffffffffu;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int64_t v = v0 + j * zs;
+                if (v < n_y && !((bits[j] >> (v & 31)) & 1u)) y[v] = (TY) 0;
+            }
+        }
+        return;
+    }
+    csr_walk<TY, TC, false>(indptr, col, val, x, seg_k, seg_info, (int64_t) blockIdx.x - zero_blocks,
+                            (int64_t) gridDim.x - zero_blocks, n_seg, part, y, alpha, up, accumulate, quad_obj{},
+                            rowmap);
+}
+
+// rows split over partial segments [split_seg[2i], split_seg[2i+1]): their
+// pieces' sum in order
+MQI_DI double split_row(const int32_t* __restrict__ split_seg, int64_t i, const double* __restrict__ part) {
+    double acc = 0.0;
+    for (int32_t s = split_seg[2 * i]; s < split_seg[2 * i + 1]; ++s) acc += part[s];
+    return acc;
+}
+MQI_DI int64_t split_element(const uint32_t* __restrict__ seg_info, const int32_t* __restrict__ split_seg, int64_t i,
+                             const int32_t* __restrict__ rowmap) {
+    const int64_t r = seg_info[split_seg[2 * i]] & 0x7fffffffu;
+    return rowmap ? (int64_t) rowmap[r] : r;
+}
+
+// y[r] = alpha * sum of the pieces (+ y[r])
+template<typename TY>
 __global__ void k_csr_split_rows(const uint32_t* __restrict__ seg_info, const int32_t* __restrict__ split_seg,
                                  int64_t n_split, const double* __restrict__ part, TY* __restrict__ y, double alpha,
-                                 int accumulate, quad_obj o, const int32_t* __restrict__ rowmap) {
+                                 const double* __restrict__ up, int accumulate, const int32_t* __restrict__ rowmap) {
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_split) return;
-    const int32_t s0 = split_seg[2 * i], s1 = split_seg[2 * i + 1];
-    const int64_t rr = seg_info[s0] & 0x7fffffffu;
-    const int64_t r  = rowmap ? (int64_t) rowmap[rr] : rr;   // the element of y
-    double        acc = 0.0;
-    for (int32_t s = s0; s < s1; ++s) acc += part[s];
-    const double out = alpha * acc;
-    if (OBJ) {   // the row's objective term after the packed segments' ones
-        const double res = out - o.p[r];
-        const double cw  = o.c ? (double) o.c[r] : 1.0;
-        o.part[o.n_seg + i] = cw * res * res;
-        if (o.g) o.g[r] = (float) (o.two_inv_n * cw * res);
-    } else {
-        y[r] = accumulate ? (TY) ((double) y[r] + out) : (TY) out;
-    }
-}
-
-// f = inv_n * (o.part[0] + ... + o.part[n - 1]) in a fixed order (one
-// workgroup: strided partial sums, then a block reduction)
-// Fixed-order sum of the objective's terms in two launches: workgroup b
-// sums chunk b of part (each thread its elements in index order, four loads
-// in flight) into out[b]; a single workgroup then sums the
-// MQI_QUAD_SUM_BLOCKS chunk sums and scales by inv_n.
-__global__ void k_quad_chunks(const double* __restrict__ part, int64_t n, double* __restrict__ out) {
-    const int64_t ch = (n + gridDim.x - 1) / gridDim.x;
-    const int64_t b0 = (int64_t) blockIdx.x * ch;
-    const int64_t b1 = b0 + ch < n ? b0 + ch : n;
-    double        acc = 0.0;
-    int64_t       i   = b0 + threadIdx.x;
-    for (; i + 768 < b1; i += 1024) {
-        const double a0 = part[i], a1 = part[i + 256], a2 = part[i + 512], a3 = part[i + 768];
-        acc += a0;
-        acc += a1;
-        acc += a2;
-        acc += a3;
-    }
-    for (; i < b1; i += 256) acc += part[i];
-    typedef hipcub::BlockReduce<double, 256> BR;
-    __shared__ typename BR::TempStorage tmp;
-    const double t = BR(tmp).Sum(acc);
-    if (threadIdx.x == 0) out[blockIdx.x] = t;
-}
-
-__global__ void k_quad_sum(const double* __restrict__ part, int64_t n, double inv_n, double* __restrict__ f) {
-    double acc = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += 256) acc += part[i];
-    typedef hipcub::BlockReduce<double, 256> BR;
-    __shared__ typename BR::TempStorage tmp;
-    const double t = BR(tmp).Sum(acc);
-    if (threadIdx.x == 0) *f = inv_n * t;
+    const int64_t r   = split_element(seg_info, split_seg, i, rowmap);
+    const double  acc = split_row(split_seg, i, part);
+    const double  out = up ? alpha * acc * *up : alpha * acc;
+    y[r]              = accumulate ? (TY) ((double) y[r] + out) : (TY) out;
 }
 
 template<typename TC>
 int
 csr_adaptive_t(const int64_t* indptr, const TC* col, const float* val, const float* x, const int64_t* seg_k,
                const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-               void* y, int y_is_double, double alpha, int accumulate, const int32_t* rowmap,
+               void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
                const uint32_t* nonempty, int64_t n_y, hipStream_t s) {
     if (rowmap && !accumulate && (!nonempty || n_y <= 0)) return (int) hipErrorInvalidValue;
     if (n_seg <= 0) return 0;
     const int blocks = (int) (n_seg < 262144 ? n_seg : 262144);
     const int zb     = (rowmap && !accumulate) ? MQI_ZERO_BLOCKS : 0;
-    const quad_obj o{};
     if (y_is_double)
-        hipLaunchKernelGGL((k_csr_adaptive<double, TC, false>), dim3(blocks + zb), dim3(64), 0, s, indptr, col, val,
-                           x, seg_k, seg_info, n_seg, part, (double*) y, alpha, accumulate, o, rowmap, nonempty, n_y,
-                           zb);
+        hipLaunchKernelGGL((k_csr_adaptive<double, TC>), dim3(blocks + zb), dim3(64), 0, s, indptr, col, val, x, seg_k,
+                           seg_info, n_seg, part, (double*) y, alpha, up, accumulate, rowmap, nonempty, n_y, zb);
     else
-        hipLaunchKernelGGL((k_csr_adaptive<float, TC, false>), dim3(blocks + zb), dim3(64), 0, s, indptr, col, val,
-                           x, seg_k, seg_info, n_seg, part, (float*) y, alpha, accumulate, o, rowmap, nonempty, n_y,
-                           zb);
+        hipLaunchKernelGGL((k_csr_adaptive<float, TC>), dim3(blocks + zb), dim3(64), 0, s, indptr, col, val, x, seg_k,
+                           seg_info, n_seg, part, (float*) y, alpha, up, accumulate, rowmap, nonempty, n_y, zb);
     if (n_split > 0) {
         const int b = (int) ((n_split + 255) / 256);
         if (y_is_double)
-            hipLaunchKernelGGL((k_csr_split_rows<double, false>), dim3(b), dim3(256), 0, s, seg_info, split_seg,
-                               n_split, part, (double*) y, alpha, accumulate, o, rowmap);
+            hipLaunchKernelGGL(k_csr_split_rows<double>, dim3(b), dim3(256), 0, s, seg_info, split_seg, n_split, part,
+                               (double*) y, alpha, up, accumulate, rowmap);
         else
-            hipLaunchKernelGGL((k_csr_split_rows<float, false>), dim3(b), dim3(256), 0, s, seg_info, split_seg,
-                               n_split, part, (float*) y, alpha, accumulate, o, rowmap);
+            hipLaunchKernelGGL(k_csr_split_rows<float>, dim3(b), dim3(256), 0, s, seg_info, split_seg, n_split, part,
+                               (float*) y, alpha, up, accumulate, rowmap);
     }
     return (int) hipGetLastError();
 }
 
+int
+csr_adaptive(const int64_t* indptr, const int32_t* col, const float* val, const float* x, const int64_t* seg_k,
+             const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
+             void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
+             const uint32_t* nonempty, int64_t n_y, hipStream_t s) {
+    return csr_adaptive_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, y, y_is_double,
+                          alpha, up, accumulate, rowmap, nonempty, n_y, s);
+}
+int
+csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, const int64_t* seg_k,
+               const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
+               void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
+               const uint32_t* nonempty, int64_t n_y, hipStream_t s) {
+    return csr_adaptive_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, y, y_is_double,
+                          alpha, up, accumulate, rowmap, nonempty, n_y, s);
+}
+
+// ------------------------------------------------------------------ quadratic objective
+// f_i = inv_n * (sum of c (d_i - p)^2) of up to MQI_QUAD_MATS matrices over one
+// x, p and c.  One launch forms the terms: per matrix, `empty` workgroups take
+// the elements no row reaches (d = 0) and the others its segments, side by
+// side; a second launch sums each matrix' terms.  Four launches per matrix
+// before (elements without a row, segments, chunk sums, sum): each drained
+// the device and cost 4 us and its share of the host's time.
+struct quad_set {
+    int      n;
+    quad_mat m[MQI_QUAD_MATS];
+    uint32_t block0[MQI_QUAD_MATS + 1];   // first workgroup of each matrix
+};
+
 // the objective's terms of the elements of y no row reaches (bit v of
-// nonempty clear): c p^2 per element, summed per workgroup of a fixed grid
-// into part[0 .. MQI_QUAD_EMPTY_BLOCKS), and g = -two_inv_n c p there
-__global__ void k_quad_empty(const uint32_t* __restrict__ nonempty, int64_t n, quad_obj o, double* __restrict__ part) {
-    // eight elements per thread and pass, their loads issued together (one
-    // load in flight per thread left the pass latency-bound); the thread's
-    // sum runs over its elements in index order
+// nonempty clear): c p^2 per element, summed per workgroup into part[b], and
+// g = -two_inv_n c p there
+MQI_DI void quad_empty(const uint32_t* __restrict__ nonempty, int64_t n, const quad_obj& o, uint32_t b,
+                       uint32_t blocks, double* __restrict__ part) {
+    // eight elements per lane and pass, their loads issued together (one load
+    // in flight per lane left the pass latency-bound); the lane's sum runs
+    // over its elements in index order
     constexpr int U      = 8;
-    const int64_t stride = (int64_t) gridDim.x * blockDim.x;
+    const int64_t stride = (int64_t) blocks * 64;
     double        acc    = 0.0;
-    for (int64_t v0 = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; v0 < n; v0 += U * stride) {
+    for (int64_t v0 = (int64_t) b * 64 + threadIdx.x; v0 < n; v0 += U * stride) {
         uint32_t bits[U];
 #pragma unroll
         for (int j = 0; j < U; ++j) {
@@ -868,72 +877,114 @@ __global__ void k_quad_empty(const uint32_t* __restrict__ nonempty, int64_t n, q
             if (o.g) o.g[v] = (float) (-o.two_inv_n * cw[j] * p[j]);
         }
     }
-    typedef hipcub::BlockReduce<double, 256> BR;
-    __shared__ typename BR::TempStorage tmp;
-    const double t = BR(tmp).Sum(acc);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+    if (threadIdx.x == 0) part[b] = acc;
 }
 
 template<typename TC>
-int
-csr_quadratic_t(const int64_t* indptr, const TC* col, const float* val, const float* x, const int64_t* seg_k,
-                const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-                double alpha, quad_obj o, double inv_n, double* f, const int32_t* rowmap, const uint32_t* nonempty,
-                int64_t n_y, hipStream_t s) {
-    if (n_seg <= 0 || !o.part || !o.p || !f) return (int) hipErrorInvalidValue;
-    if (rowmap && !nonempty) return (int) hipErrorInvalidValue;
-    o.n_seg          = n_seg;
-    const int blocks = (int) (n_seg < 262144 ? n_seg : 262144);
-    int64_t   n_part = n_seg + n_split;
-    if (rowmap) {   // the elements without a row first (their g is not written again)
-        hipLaunchKernelGGL(k_quad_empty, dim3(MQI_QUAD_EMPTY_BLOCKS), dim3(256), 0, s, nonempty, n_y, o,
-                           o.part + n_part);
-        n_part += MQI_QUAD_EMPTY_BLOCKS;
+__global__ void __launch_bounds__(64)
+k_quad(quad_set S, const float* __restrict__ x, quad_obj o, int64_t n_y) {
+    int i = 0;
+    while (i + 1 < S.n && blockIdx.x >= S.block0[i + 1]) ++i;
+    const quad_mat& m = S.m[i];
+    const uint32_t  b = blockIdx.x - S.block0[i], nb = S.block0[i + 1] - S.block0[i];
+    o.part            = m.terms;
+    if (b < m.empty)
+        quad_empty(m.nonempty, n_y, o, b, m.empty, m.terms + m.n_seg + m.n_split);
+    else
+        csr_walk<double, TC, true>(m.indptr, (const TC*) m.col, m.val, x, m.seg_k, m.seg_info, b - m.empty,
+                                   nb - m.empty, m.n_seg, m.part, nullptr, m.alpha, nullptr, 0, o, m.rowmap);
+}
+
+// the split rows' terms, after the packed segments' ones (blockIdx.y: matrix)
+__global__ void k_quad_split(quad_set S, quad_obj o) {
+    const quad_mat& m = S.m[blockIdx.y];
+    const int64_t   i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m.n_split) return;
+    const int64_t r   = split_element(m.seg_info, m.split_seg, i, m.rowmap);
+    const double  res = m.alpha * split_row(m.split_seg, i, m.part) - o.p[r];
+    const double  cw  = o.c ? (double) o.c[r] : 1.0;
+    m.terms[m.n_seg + i] = cw * res * res;
+    if (o.g) o.g[r] = (float) (o.two_inv_n * cw * res);
+}
+
+MQI_DI int64_t quad_terms(const quad_mat& m) { return m.n_seg + m.n_split + m.empty; }
+
+// this thread's elements of a[0 .. n) in index order, four loads in flight
+MQI_DI double strided_sum(const double* __restrict__ a, int64_t n, int t) {
+    double  acc = 0.0;
+    int64_t i   = threadIdx.x;
+    for (; i + 3 * t < n; i += 4 * t) {
+        const double a0 = a[i], a1 = a[i + t], a2 = a[i + 2 * t], a3 = a[i + 3 * t];
+        acc += a0;
+        acc += a1;
+        acc += a2;
+        acc += a3;
     }
-    hipLaunchKernelGGL((k_csr_adaptive<double, TC, true>), dim3(blocks), dim3(64), 0, s, indptr, col, val, x, seg_k,
-                       seg_info, n_seg, part, (double*) nullptr, alpha, 0, o, rowmap, (const uint32_t*) nullptr,
-                       (int64_t) 0, 0);
-    if (n_split > 0)
-        hipLaunchKernelGGL((k_csr_split_rows<double, true>), dim3((unsigned) ((n_split + 255) / 256)), dim3(256), 0, s,
-                           seg_info, split_seg, n_split, part, (double*) nullptr, alpha, 0, o, rowmap);
-    double* chunks = o.part + n_seg + n_split + MQI_QUAD_EMPTY_BLOCKS;
-    hipLaunchKernelGGL(k_quad_chunks, dim3(MQI_QUAD_SUM_BLOCKS), dim3(256), 0, s, o.part, n_part, chunks);
-    hipLaunchKernelGGL(k_quad_sum, dim3(1), dim3(256), 0, s, chunks, (int64_t) MQI_QUAD_SUM_BLOCKS, inv_n, f);
+    for (; i < n; i += t) acc += a[i];
+    return acc;
+}
+
+// Fixed-order sums.  A matrix of more than MQI_QUAD_ONE terms has them summed
+// in MQI_QUAD_SUM_BLOCKS chunks by as many workgroups first (one workgroup
+// over the 3.8e5 terms of a 3e8-nonzero matrix took 0.35 ms); one workgroup
+// then sums the chunk sums, or the terms.
+__global__ void __launch_bounds__(256) k_quad_chunks(quad_set S) {
+    const quad_mat& m = S.m[blockIdx.y];
+    const int64_t   n = quad_terms(m);
+    if (n <= MQI_QUAD_ONE) return;
+    const int64_t ch = (n + gridDim.x - 1) / gridDim.x, b0 = (int64_t) blockIdx.x * ch;
+    const int64_t len = b0 + ch < n ? ch : n - b0;
+    const double  acc = strided_sum(m.terms + b0, len, 256);
+    typedef hipcub::BlockReduce<double, 256> BR;
+    __shared__ typename BR::TempStorage tmp;
+    const double t = BR(tmp).Sum(acc);
+    if (threadIdx.x == 0) m.terms[n + blockIdx.x] = t;
+}
+__global__ void __launch_bounds__(1024) k_quad_sum(quad_set S, double inv_n, double* __restrict__ f) {
+    const quad_mat& m   = S.m[blockIdx.x];
+    const int64_t   n   = quad_terms(m);
+    const double    acc = n > MQI_QUAD_ONE ? strided_sum(m.terms + n, MQI_QUAD_SUM_BLOCKS, 1024)
+                                           : strided_sum(m.terms, n, 1024);
+    typedef hipcub::BlockReduce<double, 1024> BR;
+    __shared__ typename BR::TempStorage tmp;
+    const double t = BR(tmp).Sum(acc);
+    if (threadIdx.x == 0) f[blockIdx.x] = inv_n * t;
+}
+
+int
+csr_quadratic(const quad_mat* mats, int n, int cols16, const float* x, const double* p, const float* c, float* g,
+              int64_t n_y, double* f, hipStream_t s) {
+    if (n < 1 || n > MQI_QUAD_MATS || !p || !f || n_y <= 0 || (g && n != 1)) return (int) hipErrorInvalidValue;
+    quad_set S{};
+    S.n            = n;
+    int64_t blocks = 0, split = 0, terms = 0;
+    for (int i = 0; i < n; ++i) {
+        quad_mat& m = S.m[i];
+        m           = mats[i];
+        if (m.n_seg <= 0 || !m.terms || (m.rowmap && !m.nonempty)) return (int) hipErrorInvalidValue;
+        m.empty     = m.rowmap ? (uint32_t) std::min<int64_t>(MQI_QUAD_EMPTY_BLOCKS, (n_y + 511) / 512) : 0;
+        S.block0[i] = (uint32_t) blocks;
+        blocks += m.empty + std::min<int64_t>(m.n_seg, 262144);
+        split = std::max(split, m.n_split);
+        terms = std::max(terms, m.n_seg + m.n_split + (int64_t) m.empty);
+    }
+    S.block0[n] = (uint32_t) blocks;
+    quad_obj o{};
+    o.p         = p;
+    o.c         = c;
+    o.g         = g;
+    o.two_inv_n = 2.0 / (double) n_y;
+    if (cols16)
+        hipLaunchKernelGGL(k_quad<uint16_t>, dim3((unsigned) blocks), dim3(64), 0, s, S, x, o, n_y);
+    else
+        hipLaunchKernelGGL(k_quad<int32_t>, dim3((unsigned) blocks), dim3(64), 0, s, S, x, o, n_y);
+    if (split > 0)
+        hipLaunchKernelGGL(k_quad_split, dim3((unsigned) ((split + 255) / 256), (unsigned) n), dim3(256), 0, s, S, o);
+    if (terms > MQI_QUAD_ONE)
+        hipLaunchKernelGGL(k_quad_chunks, dim3(MQI_QUAD_SUM_BLOCKS, (unsigned) n), dim3(256), 0, s, S);
+    hipLaunchKernelGGL(k_quad_sum, dim3((unsigned) n), dim3(1024), 0, s, S, 1.0 / (double) n_y, f);
     return (int) hipGetLastError();
-}
-
-int
-csr_adaptive(const int64_t* indptr, const int32_t* col, const float* val, const float* x, const int64_t* seg_k,
-             const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-             void* y, int y_is_double, double alpha, int accumulate, const int32_t* rowmap, const uint32_t* nonempty,
-             int64_t n_y, hipStream_t s) {
-    return csr_adaptive_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, y, y_is_double,
-                          alpha, accumulate, rowmap, nonempty, n_y, s);
-}
-int
-csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, const int64_t* seg_k,
-               const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-               void* y, int y_is_double, double alpha, int accumulate, const int32_t* rowmap, const uint32_t* nonempty,
-             int64_t n_y, hipStream_t s) {
-    return csr_adaptive_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, y, y_is_double,
-                          alpha, accumulate, rowmap, nonempty, n_y, s);
-}
-
-int
-csr_quadratic(const int64_t* indptr, const int32_t* col, const float* val, const float* x, const int64_t* seg_k,
-              const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-              double alpha, quad_obj o, double inv_n, double* f, const int32_t* rowmap, const uint32_t* nonempty,
-              int64_t n_y, hipStream_t s) {
-    return csr_quadratic_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, alpha, o, inv_n, f,
-                           rowmap, nonempty, n_y, s);
-}
-int
-csr_quadratic16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, const int64_t* seg_k,
-                const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-                double alpha, quad_obj o, double inv_n, double* f, const int32_t* rowmap, const uint32_t* nonempty,
-                int64_t n_y, hipStream_t s) {
-    return csr_quadratic_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, alpha, o, inv_n, f,
-                           rowmap, nonempty, n_y, s);
 }
 
 // ------------------------------------------------------------------ D^T g over column deltas
@@ -1136,12 +1187,13 @@ __global__ void __launch_bounds__(64 * MQI_PIECE_WAVES)
     }
 }
 
-// y[r] = alpha * (the pieces row_piece[r] .. row_piece[r + 1] - 1) (+ y[r]):
+// y[r] = alpha * (the pieces row_piece[r] .. row_piece[r + 1] - 1) (* *up)
+// (+ y[r]):
 // one wave per row, lane l takes pieces q0 + l + 64 k, the wave adds them in
 // a fixed tree order
 template<typename TY>
 __global__ void k_piece_rows(const int32_t* __restrict__ row_piece, int64_t rows, const double* __restrict__ part,
-                             TY* __restrict__ y, double alpha, int accumulate) {
+                             TY* __restrict__ y, double alpha, const double* __restrict__ up, int accumulate) {
     const int64_t r    = (int64_t) blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int     lane = threadIdx.x & 63;
     if (r >= rows) return;
@@ -1150,7 +1202,7 @@ __global__ void k_piece_rows(const int32_t* __restrict__ row_piece, int64_t rows
     for (int32_t q = q0 + lane; q < q1; q += 64) acc += part[q];
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
     if (lane == 0) {
-        const double out = alpha * acc;
+        const double out = up ? alpha * acc * *up : alpha * acc;
         y[r]             = accumulate ? (TY) ((double) y[r] + out) : (TY) out;
     }
 }
@@ -1194,7 +1246,7 @@ stage_pieces(const float* val, const uint16_t* dcol, const int64_t* pk, const in
 int
 pieces_staged(const float* sval, const uint8_t* sd8, const uint16_t* esc, const float* x, const piece_hdr* hdr,
               int64_t n_p, const int32_t* row_piece, int64_t rows, double* part, void* y, int y_is_double,
-              double alpha, int accumulate, hipStream_t s) {
+              double alpha, const double* up, int accumulate, hipStream_t s) {
     if (n_p > 0) {
         const int64_t b = (n_p + MQI_PIECE_WAVES - 1) / MQI_PIECE_WAVES;
         hipLaunchKernelGGL(k_pieces_staged, dim3((unsigned) (b < 65536 ? b : 65536)), dim3(64 * MQI_PIECE_WAVES), 0,
@@ -1204,37 +1256,43 @@ pieces_staged(const float* sval, const uint8_t* sd8, const uint16_t* esc, const 
         const unsigned b = (unsigned) ((rows + 3) / 4);
         if (y_is_double)
             hipLaunchKernelGGL(k_piece_rows<double>, dim3(b), dim3(256), 0, s, row_piece, rows, part, (double*) y,
-                               alpha, accumulate);
+                               alpha, up, accumulate);
         else
             hipLaunchKernelGGL(k_piece_rows<float>, dim3(b), dim3(256), 0, s, row_piece, rows, part, (float*) y,
-                               alpha, accumulate);
+                               alpha, up, accumulate);
     }
     return (int) hipGetLastError();
 }
 
 // Compacted x for D^T g: xc[i] = x[nzvox[i]] (nzvox: the voxels that appear
-// in some row, ascending).
+// in some row, ascending), rounded to float here if x is double: a conversion
+// of the whole vector first reads and writes every voxel (20 us for 8.4 M).
 // four entries per thread: 16-byte index loads and stores
-__global__ void k_gather_x(const float* __restrict__ x, const int32_t* __restrict__ nzvox, int64_t n,
+template<typename TX>
+__global__ void k_gather_x(const TX* __restrict__ x, const int32_t* __restrict__ nzvox, int64_t n,
                            float* __restrict__ xc) {
     const int64_t n4 = n >> 2;
     for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t) gridDim.x * blockDim.x) {
         const i32x4 v = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(nzvox) + i);
         f32x4       o;
-        o.x = x[v.x];
-        o.y = x[v.y];
-        o.z = x[v.z];
-        o.w = x[v.w];
+        o.x = (float) x[v.x];
+        o.y = (float) x[v.y];
+        o.z = (float) x[v.z];
+        o.w = (float) x[v.w];
         __builtin_nontemporal_store(o, reinterpret_cast<f32x4*>(xc) + i);
     }
     const int64_t t = (n4 << 2) + (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.x == 0 && t < n) xc[t] = x[nzvox[t]];
+    if (blockIdx.x == 0 && t < n) xc[t] = (float) x[nzvox[t]];
 }
 
 int
-gather_x(const float* x, const int32_t* nzvox, int64_t n, float* xc, hipStream_t s) {
+gather_x(const void* x, int x_double, const int32_t* nzvox, int64_t n, float* xc, hipStream_t s) {
     if (n <= 0) return 0;
-    hipLaunchKernelGGL(k_gather_x, dim3(grid_for((uint64_t) (n + 3) / 4)), dim3(256), 0, s, x, nzvox, n, xc);
+    const dim3 g(grid_for((uint64_t) (n + 3) / 4));
+    if (x_double)
+        hipLaunchKernelGGL(k_gather_x<double>, g, dim3(256), 0, s, (const double*) x, nzvox, n, xc);
+    else
+        hipLaunchKernelGGL(k_gather_x<float>, g, dim3(256), 0, s, (const float*) x, nzvox, n, xc);
     return (int) hipGetLastError();
 }
 

@@ -41,21 +41,28 @@ class DijMatrix:
             raise ValueError("the sparse products take device tensors")
         return x.detach().to(torch.float32).contiguous()
 
-    def _product(self, transpose, x, n_out, out_dtype):
-        y = torch.empty(n_out, dtype=torch.float64, device=x.device)
-        stream = torch.cuda.current_stream(x.device).cuda_stream
-        self.ctx.dij_matvec(self.scenario, int(transpose), x.data_ptr(), y.data_ptr(), y_double=True,
-                            alpha=self.scale, stream=stream)
-        return y if out_dtype == torch.float64 else y.to(out_dtype)
-
     def matvec(self, w, out_dtype=torch.float64):
         """Dose scale * D w (n_voxels)."""
-        return self._product(False, self._vec(w, self.n_spots), self.n_voxels, out_dtype)
+        x = self._vec(w, self.n_spots)
+        y = torch.empty(self.n_voxels, dtype=torch.float64, device=x.device)
+        stream = torch.cuda.current_stream(x.device).cuda_stream
+        self.ctx.dij_matvec(self.scenario, 0, x.data_ptr(), y.data_ptr(), y_double=True, alpha=self.scale,
+                            stream=stream)
+        return y if out_dtype == torch.float64 else y.to(out_dtype)
 
     def quadratic(self, w, prescription, voxel_weights=None, want_grad=True):
         """f = mean_v c_v (scale (D w)_v - p_v)^2 as a device scalar (float64)
         and, with want_grad, df/dd = 2 c (d - p) / n_voxels (float32, the
         input of rmatvec), in one pass over the matrix (mqi_dij_quadratic)."""
+        w, p, c = self._objective_inputs(w, prescription, voxel_weights)
+        f = torch.empty((), dtype=torch.float64, device=w.device)
+        g = torch.empty(self.n_voxels, dtype=torch.float32, device=w.device) if want_grad else None
+        stream = torch.cuda.current_stream(w.device).cuda_stream
+        self.ctx.dij_quadratic(self.scenario, w.data_ptr(), p.data_ptr(), c.data_ptr() if c is not None else 0,
+                               self.scale, g.data_ptr() if g is not None else 0, f.data_ptr(), stream=stream)
+        return f, g
+
+    def _objective_inputs(self, w, prescription, voxel_weights):
         w = self._vec(w, self.n_spots)
         p = prescription.detach().to(device=w.device, dtype=torch.float64).contiguous()
         if p.dim() != 1 or p.numel() != self.n_voxels:
@@ -65,16 +72,24 @@ class DijMatrix:
             c = voxel_weights.detach().to(device=w.device, dtype=torch.float32).contiguous()
             if c.dim() != 1 or c.numel() != self.n_voxels:
                 raise ValueError("expected voxel weights of %d voxels" % self.n_voxels)
-        f = torch.empty((), dtype=torch.float64, device=w.device)
-        g = torch.empty(self.n_voxels, dtype=torch.float32, device=w.device) if want_grad else None
-        stream = torch.cuda.current_stream(w.device).cuda_stream
-        self.ctx.dij_quadratic(self.scenario, w.data_ptr(), p.data_ptr(), c.data_ptr() if c is not None else 0,
-                               self.scale, g.data_ptr() if g is not None else 0, f.data_ptr(), stream=stream)
-        return f, g
+        return w, p, c
 
     def rmatvec(self, g, out_dtype=torch.float64):
         """scale * D^T g (n_spots)."""
-        return self._product(True, self._vec(g, self.n_voxels), self.n_spots, out_dtype)
+        return self._adjoint(g, out_dtype)
+
+    def _adjoint(self, g, out_dtype, up=0):
+        """scale * D^T g in out_dtype, times the device double at up (unless
+        0).  A float64 g is rounded to float32 where the product reads it."""
+        double = (g.dtype == torch.float64 and g.dim() == 1 and g.numel() == self.n_voxels and g.is_cuda and
+                  g.is_contiguous() and not g.is_neg())
+        x = g.detach() if double else self._vec(g, self.n_voxels)
+        y_dtype = torch.float32 if out_dtype == torch.float32 else torch.float64
+        y = torch.empty(self.n_spots, dtype=y_dtype, device=x.device)
+        stream = torch.cuda.current_stream(x.device).cuda_stream
+        self.ctx.dij_adjoint(self.scenario, x.data_ptr(), double, up, self.scale, y.data_ptr(),
+                             y_dtype == torch.float64, stream=stream)
+        return y if y_dtype == out_dtype else y.to(out_dtype)
 
 
 class _Dose(torch.autograd.Function):
@@ -86,8 +101,7 @@ class _Dose(torch.autograd.Function):
 
     @staticmethod
     def backward(fctx, grad_dose):
-        grad_w = fctx.mat.rmatvec(grad_dose, torch.float64)
-        return grad_w.to(fctx.w_dtype), None
+        return fctx.mat.rmatvec(grad_dose, fctx.w_dtype), None
 
 
 def dose(mat, w):
@@ -108,8 +122,25 @@ class _Quadratic(torch.autograd.Function):
     @staticmethod
     def backward(fctx, grad_f):
         (g,) = fctx.saved_tensors
+        up = _device_scalar(grad_f, g)
+        if up:
+            return fctx.mat._adjoint(g, fctx.w_dtype, up), None, None, None
         grad_w = fctx.mat.rmatvec(g, torch.float64) * grad_f
         return grad_w.to(fctx.w_dtype), None, None, None
+
+
+def _device_scalar(s, like):
+    """Address of s when it is a plain float64 scalar on like's device that
+    the product may take by its address, else 0: a graph through s (create_graph)
+    or a batch of scalars (is_grads_batched, without storage of its own) takes
+    torch's product."""
+    if (s.dtype != torch.float64 or s.numel() != 1 or s.device != like.device or s.is_neg() or
+            (torch.is_grad_enabled() and s.requires_grad)):
+        return 0
+    try:
+        return s.data_ptr()
+    except RuntimeError:
+        return 0
 
 
 def quadratic_objective(mat, w, prescription, voxel_weights=None):
@@ -117,6 +148,22 @@ def quadratic_objective(mat, w, prescription, voxel_weights=None):
     one pass over the matrix (the dose is not formed); the gradient is
     D^T (2 c (D w - p) / n)."""
     return _Quadratic.apply(w, mat, prescription, voxel_weights)
+
+
+def _values(mats, w, prescription, voxel_weights):
+    """The objective of every scenario (float64 vector), in one pass of
+    launches where the scenarios are distinct ones of one context and size."""
+    first = mats[0] if mats else None
+    if (len({m.scenario for m in mats}) < len(mats) or not mats or
+            any(m.ctx is not first.ctx or type(m) is not DijMatrix or m.n_spots != first.n_spots or
+                m.n_voxels != first.n_voxels for m in mats)):
+        return torch.stack([m.quadratic(w, prescription, voxel_weights, want_grad=False)[0] for m in mats])
+    w, p, c = first._objective_inputs(w, prescription, voxel_weights)
+    f = torch.empty(len(mats), dtype=torch.float64, device=w.device)
+    stream = torch.cuda.current_stream(w.device).cuda_stream
+    first.ctx.dij_quadratics([m.scenario for m in mats], [m.scale for m in mats], w.data_ptr(), p.data_ptr(),
+                             c.data_ptr() if c is not None else 0, f.data_ptr(), stream=stream)
+    return f
 
 
 def worst_case_objective(mats, w, prescription, voxel_weights=None):
@@ -128,6 +175,6 @@ def worst_case_objective(mats, w, prescription, voxel_weights=None):
     would carry zero gradients through the others).  The products are
     deterministic: the returned maximum equals its entry in the values."""
     with torch.no_grad():
-        vals = torch.stack([m.quadratic(w, prescription, voxel_weights, want_grad=False)[0] for m in mats])
+        vals = _values(mats, w, prescription, voxel_weights)
     k = int(torch.argmax(vals).item())
     return quadratic_objective(mats[k], w, prescription, voxel_weights), vals
