@@ -1769,8 +1769,9 @@ prepare_products(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& indptr, bui
     HIPCHK(c, hipMemcpy(&n_nz, ws.heads + (m.nnz + MQI_TILE - 1) / MQI_TILE, sizeof n_nz, hipMemcpyDeviceToHost));
     m.n_nz = (int64_t) n_nz;
     // D w over 16-bit spot columns where they fit
-    if ((r = m.rows <= 65536 ? dalloc(c, &m.tcol16, m.nnz) : dalloc(c, &m.tcol, m.nnz)) ||
-        (r = dalloc(c, &m.tval, m.nnz)) || (r = dalloc(c, &m.tindptr, m.n_nz + 1)) ||
+    const size_t padded = (size_t) m.nnz + MQI_SEG_PAD;
+    if ((r = m.rows <= 65536 ? dalloc(c, &m.tcol16, padded) : dalloc(c, &m.tcol, padded)) ||
+        (r = dalloc(c, &m.tval, padded)) || (r = dalloc(c, &m.tindptr, m.n_nz + 1)) ||
         (r = dalloc(c, &m.tnonempty, (m.cols + 31) / 32)) || (r = dalloc(c, &m.nzvox, m.n_nz)) ||
         (r = dalloc(c, &m.xc, m.n_nz)))
         return r;
@@ -1784,7 +1785,7 @@ prepare_products(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& indptr, bui
         std::swap(ws.packed, ws.packed2);
     }
     // long rows (the Dij of pencil beams): D^T g over byte column deltas
-    const bool pieces = m.nnz >= (int64_t) MQI_SEG_SHORT * m.rows;
+    const bool pieces = m.nnz >= 1024 * m.rows;
     if (!pieces && (r = dalloc(c, &m.ccol, m.nnz))) return r;
     KCHK(c, mqi_aux::spot_rows(ws.packed, m.nzvox, m.nnz, m.col, pieces ? (int32_t*) ws.vox : m.ccol, m.val,
                                c->stream));
@@ -2159,9 +2160,9 @@ mqi_dij_matvec(mqi_ctx* c, int s, int transpose, const float* x, void* y, int y_
         // zeros at the others
         const csr_plan& p = m.tplan;
         if (m.tcol16)
-            KCHK(c, mqi_aux::csr_adaptive16(m.tindptr, m.tcol16, m.tval, x, p.seg_k, p.seg_info, p.n_seg,
-                                            p.split_seg, p.n_split, p.part, y, y_double, alpha, nullptr, accumulate,
-                                            m.nzvox, m.tnonempty, m.cols, st));
+            KCHK(c, mqi_aux::csr_adaptive16(m.tindptr, m.tcol16, m.tval, x, m.rows, p.seg_k, p.seg_info, p.n_seg,
+                                            p.split_seg, p.n_split, p.part, y, y_double, alpha, accumulate, m.nzvox,
+                                            m.tnonempty, m.cols, st));
         else
             KCHK(c, mqi_aux::csr_adaptive(m.tindptr, m.tcol, m.tval, x, p.seg_k, p.seg_info, p.n_seg, p.split_seg,
                                           p.n_split, p.part, y, y_double, alpha, nullptr, accumulate, m.nzvox,
@@ -2198,7 +2199,7 @@ mqi_dij_quadratic(mqi_ctx* c, int s, const float* w, const double* p, const floa
     const csr_dev& m  = c->dij[s];
     hipStream_t    st = stream ? (hipStream_t) stream : c->stream;
     HIPCHK(c, hipEventRecord(c->ev_mv0, st));
-    KCHK(c, mqi_aux::csr_quadratic(&q, 1, m.tcol16 != nullptr, w, p, cw, g, m.cols, f, st));
+    KCHK(c, mqi_aux::csr_quadratic(&q, 1, m.tcol16 != nullptr, w, m.rows, p, cw, g, m.cols, f, st));
     HIPCHK(c, hipEventRecord(c->ev_mv1, st));
     c->matvec_pending = true;
     return 0;
@@ -2222,7 +2223,7 @@ mqi_dij_quadratics(mqi_ctx* c, int n, const int32_t* scenarios, const double* al
     hipStream_t    st = stream ? (hipStream_t) stream : c->stream;
     HIPCHK(c, hipEventRecord(c->ev_mv0, st));
     for (int i = 0; i < n; i += MQI_QUAD_MATS)
-        KCHK(c, mqi_aux::csr_quadratic(q.data() + i, std::min(n - i, MQI_QUAD_MATS), m.tcol16 != nullptr, w, p, cw,
+        KCHK(c, mqi_aux::csr_quadratic(q.data() + i, std::min(n - i, MQI_QUAD_MATS), m.tcol16 != nullptr, w, m.rows, p, cw,
                                        nullptr, m.cols, f + i, st));
     HIPCHK(c, hipEventRecord(c->ev_mv1, st));
     c->matvec_pending = true;

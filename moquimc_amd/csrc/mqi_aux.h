@@ -55,9 +55,10 @@ int spot_rows(const uint64_t* ranked, const int32_t* nzvox, int64_t n, int32_t* 
 // CSR-Adaptive segment sizes (entries of one long-row piece; entries and rows
 // of one packed segment)
 #define MQI_SEG_LONG 16384
-#ifndef MQI_SEG_SHORT
-#define MQI_SEG_SHORT 1024
-#endif
+#define MQI_SEG_SHORT 1016
+#define MQI_SEG_BUF 1024   // entries of the vectors that cover a packed segment
+// entries behind the last one that the products' vectors may cover (zero)
+#define MQI_SEG_PAD 4
 #define MQI_SEG_ROWS 1024
 // rowmap: the element of y each row writes (NULL: row r writes y[r]).  A
 // matrix stored without its empty rows (rowmap set) writes y = 0 at the n_y
@@ -69,11 +70,18 @@ int csr_adaptive(const int64_t* indptr, const int32_t* col, const float* val, co
                  const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
                  void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
                  const uint32_t* nonempty, int64_t n_y, hipStream_t s);
-// the same over 16-bit columns (D w of a Dij with at most 65536 spots)
-int csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, const int64_t* seg_k,
-                   const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-                   void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
-                   const uint32_t* nonempty, int64_t n_y, hipStream_t s);
+// The same over 16-bit columns (D w of a Dij with at most 65536 spots).  From
+// MQI_LDS_SEGS segments on its workgroups keep x (n_x entries) in LDS, where
+// that leaves room for MQI_LDS_WAVES waves of a CU (24576 entries): 200 spots
+// (8.4 M entries) took 43.9 us without and 42.1 with, 150 spots 40.5 without.
+#define MQI_LDS 163840   // bytes of LDS of a CU and of a workgroup
+#define MQI_CUS 256
+#define MQI_LDS_WAVES 8
+#define MQI_LDS_SEGS 8192
+int csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, int64_t n_x,
+                   const int64_t* seg_k, const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg,
+                   int64_t n_split, double* part, void* y, int y_is_double, double alpha, int accumulate,
+                   const int32_t* rowmap, const uint32_t* nonempty, int64_t n_y, hipStream_t s);
 // The quadratic objective of y = alpha * A x on the D w matrices of up to
 // MQI_QUAD_MATS scenarios, without y: f[i] = mean over the n_y elements of
 // c (y_i - p)^2 (c NULL: 1; f on the device) and, for a single matrix, g =
@@ -84,7 +92,7 @@ int csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val,
 // nonempty is clear (y = 0), summed in a fixed order that depends on the
 // matrix alone.
 #define MQI_QUAD_MATS 16
-#define MQI_QUAD_EMPTY_BLOCKS 2048
+#define MQI_QUAD_EMPTY_BLOCKS 4096
 #define MQI_QUAD_SUM_BLOCKS 256
 #define MQI_QUAD_ONE 32768   // terms that one workgroup sums
 struct quad_obj {
@@ -108,8 +116,8 @@ struct quad_mat {
     double          alpha;
     uint32_t        empty;   // workgroups of the elements without a row (set by csr_quadratic)
 };
-int csr_quadratic(const quad_mat* mats, int n, int cols16, const float* x, const double* p, const float* c, float* g,
-                  int64_t n_y, double* f, hipStream_t s);
+int csr_quadratic(const quad_mat* mats, int n, int cols16, const float* x, int64_t n_x, const double* p,
+                  const float* c, float* g, int64_t n_y, double* f, hipStream_t s);
 // D^T g over column deltas (mqi_aux.hip): the 16-bit deltas of each row's
 // columns (0 at row starts and where a row skips more than 65535 columns,
 // those positions listed in gaps), the column before each piece's first

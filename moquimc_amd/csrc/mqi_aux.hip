@@ -513,6 +513,10 @@ k_voxel_rows(const uint32_t* __restrict__ key, const uint64_t* __restrict__ pack
         if (i == n - 1) {
             tptr[row + 1]   = n;
             tptr32[row + 1] = (uint32_t) n;
+            for (int k = 0; k < MQI_SEG_PAD; ++k) {
+                tcol[n + k] = (T) 0;
+                tval[n + k] = 0.0f;
+            }
         }
     }
 }
@@ -581,9 +585,17 @@ template<typename TC> struct col4;
 template<> struct col4<int32_t> { typedef i32x4 type; };
 template<> struct col4<uint16_t> { typedef u16x4 type; };
 
-// a packed segment is loaded as at most 4 x 64 vectors of four entries
-static_assert(MQI_SEG_SHORT <= 1024, "packed segments are loaded as at most 256 vectors");
+// a packed segment is loaded as at most 4 x 64 vectors of four entries, which
+// may begin up to three entries before it
+static_assert(MQI_SEG_SHORT + 3 <= MQI_SEG_BUF && MQI_SEG_BUF == 1024, "segments are loaded as at most 256 vectors");
 
+// a wave's LDS accesses are performed in order: only the compiler must keep it
+MQI_DI void lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One wave's walk over segments, with MQI_SEG_SHORT doubles of LDS of its own.
 // OBJ: instead of y, the quadratic objective of y (quad_obj): per row
 // c_r (y_r - p_r)^2 summed over each packed segment into o.part[s] (0 for a
 // long-row segment, whose rows k_quad_split finishes), and
@@ -593,9 +605,8 @@ MQI_DI void csr_walk(const int64_t* __restrict__ indptr, const TC* __restrict__ 
                      const float* __restrict__ x, const int64_t* __restrict__ seg_k,
                      const uint32_t* __restrict__ seg_info, int64_t first, int64_t stride, int64_t n_seg,
                      double* __restrict__ part, TY* __restrict__ y, double alpha, const double* __restrict__ up,
-                     int accumulate, const quad_obj& o, const int32_t* __restrict__ rowmap) {
-    __shared__ double buf[MQI_SEG_SHORT];
-    const int lane = threadIdx.x;
+                     int accumulate, const quad_obj& o, const int32_t* __restrict__ rowmap, double* buf) {
+    const int lane = threadIdx.x & 63;
     // plain grid-stride walk: a remap giving each XCD a contiguous run of
     // segments measured ~7 % slower on the 5000-spot Dij
     for (int64_t s = first; s < n_seg; s += stride) {
@@ -678,7 +689,7 @@ MQI_DI void csr_walk(const int64_t* __restrict__ indptr, const TC* __restrict__ 
                     b[3]      = (double) v[u].w * (double) x[c[u].w];
                 }
             }
-            __syncthreads();
+            lds_fence();
             // L lanes per row (a power of two, L * rows <= 64): each sums a
             // strided part, then the group adds its parts with shuffles
             const int64_t nr = r1 - r0;
@@ -719,9 +730,37 @@ MQI_DI void csr_walk(const int64_t* __restrict__ indptr, const TC* __restrict__ 
                 for (int off = 32; off > 0; off >>= 1) obj += __shfl_xor(obj, off);
                 if (lane == 0) o.part[s] = obj;
             }
-            __syncthreads();
+            lds_fence();
         }
     }
+}
+
+// y = 0 at the elements no row reaches (bit clear in nonempty): part b of n
+template<typename TY>
+MQI_DI void zero_empty(const uint32_t* __restrict__ nonempty, int64_t n_y, TY* __restrict__ y, int b, int n) {
+    // eight elements per lane and pass, their mask words loaded together
+    const int64_t zs = (int64_t) n * 64;
+    for (int64_t v0 = (int64_t) b * 64 + (threadIdx.x & 63); v0 < n_y; v0 += 8 * zs) {
+        uint32_t bits[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bits[j] = (v0 + j * zs < n_y) ? nonempty[(v0 + j * zs) >> 5] : 0xffffffffu;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int64_t v = v0 + j * zs;
+            if (v < n_y && !((bits[j] >> (v & 31)) & 1u)) y[v] = (TY) 0;
+        }
+    }
+}
+
+// x behind the waves' buffers, and the wave's index in the grid (a scalar)
+MQI_DI const float* stage_x(const float* __restrict__ x, int n_x, double* lds) {
+    float* xs = (float*) (lds + (blockDim.x >> 6) * MQI_SEG_BUF);
+    for (int i = threadIdx.x; i < n_x; i += blockDim.x) xs[i] = x[i];
+    __syncthreads();
+    return xs;
+}
+MQI_DI int64_t wave_index() {
+    return (int64_t) blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
 }
 
 // up (device): y = alpha * A x * *up, rounded as the two products
@@ -736,27 +775,173 @@ __global__ void __launch_bounds__(64) k_csr_adaptive(const int64_t* __restrict__
                                                      const int32_t* __restrict__ rowmap,
                                                      const uint32_t* __restrict__ nonempty, int64_t n_y,
                                                      int zero_blocks) {
-    const int lane = threadIdx.x;
+    __shared__ double buf[MQI_SEG_BUF];
     // the first zero_blocks workgroups write y = 0 at the elements no row
-    // reaches (bit clear in nonempty), alongside the segments' workgroups
+    // reaches, alongside the segments' workgroups
     if ((int) blockIdx.x < zero_blocks) {
-        // eight elements per lane and pass, their mask words loaded together
-        const int64_t zs = (int64_t) zero_blocks * 64;
-        for (int64_t v0 = (int64_t) blockIdx.x * 64 + lane; v0 < n_y; v0 += 8 * zs) {
-            uint32_t bits[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) bits[j] = (v0 + j * zs < n_y) ? nonempty[(v0 + j * zs) >> 5] : 0xffffffffu;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int64_t v = v0 + j * zs;
-                if (v < n_y && !((bits[j] >> (v & 31)) & 1u)) y[v] = (TY) 0;
-            }
-        }
+        zero_empty(nonempty, n_y, y, blockIdx.x, zero_blocks);
         return;
     }
     csr_walk<TY, TC, false>(indptr, col, val, x, seg_k, seg_info, (int64_t) blockIdx.x - zero_blocks,
                             (int64_t) gridDim.x - zero_blocks, n_seg, part, y, alpha, up, accumulate, quad_obj{},
-                            rowmap);
+                            rowmap, buf);
+}
+
+// ------------------------------------------------------------------ D w, large matrices
+// The same with x in LDS and the next segment under way, for 16-bit columns.
+// k_csr_adaptive's waves load, gather, sum and write one segment after
+// another, and their gathers of x (64 lanes, as many lines of the vector
+// cache) take about a clock a lane: 6 bytes an entry at 2.2 to 2.8 TB/s.  Here
+// workgroups of 8 to 16 waves share a copy of x and stay; a wave loads its
+// next segment's entries, row pointers and voxels once this segment's products
+// are in LDS, before it sums them.  D w of 1000 spots on 8.4 M voxels (42 M
+// entries) 116 -> 91 us, 8000 spots (219 M) 465 -> 356, 24576 spots (672 M)
+// 1755 -> 1431; their objective with weights and gradient 156 -> 127, 514 ->
+// 377 and 1816 -> 1414.  (The loads alone stream 6.8 TB/s, with sums of rows
+// of 27 entries and the gathers 5.2; what is left between is the row data, the
+// scattered writes and the last, partly filled round of segments.)
+//
+// A segment's entries are read as the whole 16-byte vectors that cover it: at
+// most 256, as a packed segment has at most MQI_SEG_SHORT entries; what is
+// read around it belongs to its neighbours or to the arrays' padding.
+struct seg_rows {   // a packed segment, as a wave holds it
+    int64_t kb, r0;
+    int     n4, nr, L;          // vectors, rows, lanes per row
+    int     ea, eb;             // the lane's first row: its entries in the buffer
+    int32_t va;                 // and its element of y
+};
+struct seg_data {
+    f32x4 v[4];
+    u16x4 c[4];
+};
+MQI_DI void seg_load(const int64_t* __restrict__ indptr, const uint16_t* __restrict__ col,
+                     const float* __restrict__ val, int64_t kb, int64_t ke, int64_t r0, int64_t r1,
+                     const int32_t* __restrict__ rowmap, seg_rows& q, seg_data& d) {
+    const int lane = threadIdx.x & 63;
+    q.kb           = kb & ~(int64_t) 3;
+    q.r0           = r0;
+    q.n4           = (int) ((ke + 3 - q.kb) >> 2);
+    q.nr           = (int) (r1 - r0);
+    q.L            = 1;
+    while (q.L < 64 && 2 * q.L * q.nr <= 64) q.L *= 2;
+    const f32x4* v4 = reinterpret_cast<const f32x4*>(val + q.kb);
+    const u16x4* c4 = reinterpret_cast<const u16x4*>(col + q.kb);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        if (lane + 64 * u < q.n4) {
+            d.v[u] = __builtin_nontemporal_load(v4 + lane + 64 * u);
+            d.c[u] = __builtin_nontemporal_load(c4 + lane + 64 * u);
+        }
+    const int ra = lane / q.L;
+    if (ra < q.nr) {
+        q.ea = (int) (indptr[r0 + ra] - q.kb);
+        q.eb = (int) (indptr[r0 + ra + 1] - q.kb);
+        q.va = rowmap ? rowmap[r0 + ra] : (int32_t) (r0 + ra);
+    }
+}
+
+// wave `wave` of `waves`' segments of a matrix: as csr_walk
+template<typename TY, bool OBJ>
+MQI_DI void csr_stream(const int64_t* __restrict__ indptr, const uint16_t* __restrict__ col,
+                       const float* __restrict__ val, const float* xs, const int64_t* __restrict__ seg_k,
+                       const uint32_t* __restrict__ seg_info, int64_t wave, int64_t waves, int64_t n_seg,
+                       double* __restrict__ part, TY* __restrict__ y, double alpha, int accumulate, const quad_obj& o,
+                       const int32_t* __restrict__ rowmap, double* buf) {
+    const int lane = threadIdx.x & 63;
+    seg_rows  q;
+    seg_data  d;
+    bool      loaded = false;
+    for (int64_t s = wave; s < n_seg; s += waves) {
+        const uint32_t info = seg_info[s];
+        if (info >> 31) {   // a piece of a long row
+            csr_walk<TY, uint16_t, OBJ>(indptr, col, val, xs, seg_k, seg_info, s, 1, s + 1, part, y, alpha, nullptr,
+                                        accumulate, o, rowmap, buf);
+            continue;
+        }
+        if (!loaded)
+            seg_load(indptr, col, val, seg_k[s], seg_k[s + 1], info, seg_info[s + 1] & 0x7fffffffu, rowmap, q, d);
+        const seg_rows h  = q;
+        const int      ra = lane / h.L, sub = lane & (h.L - 1);
+        double         pa = 0.0, ca = 1.0;
+        if (OBJ && ra < h.nr && sub == 0) {
+            pa = o.p[h.va];
+            if (o.c) ca = (double) o.c[h.va];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (lane + 64 * u < h.n4) {
+                double* b = buf + 4 * (lane + 64 * u);
+                b[0]      = (double) d.v[u].x * (double) xs[d.c[u].x];
+                b[1]      = (double) d.v[u].y * (double) xs[d.c[u].y];
+                b[2]      = (double) d.v[u].z * (double) xs[d.c[u].z];
+                b[3]      = (double) d.v[u].w * (double) xs[d.c[u].w];
+            }
+        const int64_t  nx = s + waves;
+        const uint32_t ni = nx < n_seg ? seg_info[nx] : 1u << 31;
+        loaded            = !(ni >> 31);
+        if (loaded)
+            seg_load(indptr, col, val, seg_k[nx], seg_k[nx + 1], ni, seg_info[nx + 1] & 0x7fffffffu, rowmap, q, d);
+        lds_fence();
+        double obj = 0.0;   // this lane's rows' objective terms, in row order
+        for (int rb = 0; rb < h.nr; rb += 64 / h.L) {
+            const int r   = rb + ra;
+            double    acc = 0.0, pr = pa, cw = ca;
+            int       i = h.ea, e = h.eb;
+            int32_t   v = h.va;
+            if (rb > 0 && r < h.nr) {
+                i = (int) (indptr[h.r0 + r] - h.kb);
+                e = (int) (indptr[h.r0 + r + 1] - h.kb);
+                v = rowmap ? rowmap[h.r0 + r] : (int32_t) (h.r0 + r);
+                if (OBJ && sub == 0) {
+                    pr = o.p[v];
+                    if (o.c) cw = (double) o.c[v];
+                }
+            }
+            if (r < h.nr) {
+                // in order, four LDS reads in flight
+                i += sub;
+                for (; i + 3 * h.L < e; i += 4 * h.L) {
+                    const double a0 = buf[i], a1 = buf[i + h.L], a2 = buf[i + 2 * h.L], a3 = buf[i + 3 * h.L];
+                    acc += a0;
+                    acc += a1;
+                    acc += a2;
+                    acc += a3;
+                }
+                for (; i < e; i += h.L) acc += buf[i];
+            }
+            for (int off = h.L >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+            if (r < h.nr && sub == 0) {
+                const double out = alpha * acc;
+                if (OBJ) {
+                    const double res = out - pr;
+                    obj += cw * res * res;
+                    if (o.g) o.g[v] = (float) (o.two_inv_n * cw * res);
+                } else {
+                    y[v] = accumulate ? (TY) ((double) y[v] + out) : (TY) out;
+                }
+            }
+        }
+        if (OBJ) {
+            for (int off = 32; off > 0; off >>= 1) obj += __shfl_xor(obj, off);
+            if (lane == 0) o.part[s] = obj;
+        }
+        lds_fence();
+    }
+}
+
+template<typename TY>
+__global__ void __launch_bounds__(1024)
+k_csr_lds(const int64_t* __restrict__ indptr, const uint16_t* __restrict__ col, const float* __restrict__ val,
+          const float* __restrict__ x, int n_x, const int64_t* __restrict__ seg_k,
+          const uint32_t* __restrict__ seg_info, int64_t n_seg, double* __restrict__ part, TY* __restrict__ y,
+          double alpha, int accumulate, const int32_t* __restrict__ rowmap, const uint32_t* __restrict__ nonempty,
+          int64_t n_y, int zero) {
+    extern __shared__ double lds[];
+    const float*  xs    = stage_x(x, n_x, lds);
+    const int64_t waves = (int64_t) gridDim.x * (blockDim.x >> 6), wave = wave_index();
+    if (zero) zero_empty(nonempty, n_y, y, (int) wave, (int) waves);
+    csr_stream<TY, false>(indptr, col, val, xs, seg_k, seg_info, wave, waves, n_seg, part, y, alpha, accumulate,
+                              quad_obj{}, rowmap, lds + (threadIdx.x >> 6) * MQI_SEG_BUF);
 }
 
 // rows split over partial segments [split_seg[2i], split_seg[2i+1]): their
@@ -785,6 +970,38 @@ __global__ void k_csr_split_rows(const uint32_t* __restrict__ seg_info, const in
     y[r]              = accumulate ? (TY) ((double) y[r] + out) : (TY) out;
 }
 
+int
+csr_split_rows(const uint32_t* seg_info, const int32_t* split_seg, int64_t n_split, double* part, void* y,
+               int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap, hipStream_t s) {
+    if (n_split > 0) {
+        const int b = (int) ((n_split + 255) / 256);
+        if (y_is_double)
+            hipLaunchKernelGGL(k_csr_split_rows<double>, dim3(b), dim3(256), 0, s, seg_info, split_seg, n_split, part,
+                               (double*) y, alpha, up, accumulate, rowmap);
+        else
+            hipLaunchKernelGGL(k_csr_split_rows<float>, dim3(b), dim3(256), 0, s, seg_info, split_seg, n_split, part,
+                               (float*) y, alpha, up, accumulate, rowmap);
+    }
+    return (int) hipGetLastError();
+}
+
+// Workgroups with x in LDS: waves a group, groups and LDS bytes; false where
+// the segments are too few to stay for, or too few waves would share a CU with
+// x (the kernels' registers allow 16).
+struct lds_shape {
+    int    waves, blocks;
+    size_t bytes;
+};
+bool
+lds_launch(int64_t n_x, int64_t n_seg, lds_shape& L) {
+    const int64_t w = std::min<int64_t>(16, (MQI_LDS - 4 * n_x) / (8 * MQI_SEG_BUF));
+    if (n_x <= 0 || w < MQI_LDS_WAVES || n_seg < MQI_LDS_SEGS) return false;
+    L.waves  = (int) w;
+    L.bytes  = (size_t) (8 * MQI_SEG_BUF * w + 4 * n_x);
+    L.blocks = MQI_CUS;
+    return true;
+}
+
 template<typename TC>
 int
 csr_adaptive_t(const int64_t* indptr, const TC* col, const float* val, const float* x, const int64_t* seg_k,
@@ -801,16 +1018,7 @@ csr_adaptive_t(const int64_t* indptr, const TC* col, const float* val, const flo
     else
         hipLaunchKernelGGL((k_csr_adaptive<float, TC>), dim3(blocks + zb), dim3(64), 0, s, indptr, col, val, x, seg_k,
                            seg_info, n_seg, part, (float*) y, alpha, up, accumulate, rowmap, nonempty, n_y, zb);
-    if (n_split > 0) {
-        const int b = (int) ((n_split + 255) / 256);
-        if (y_is_double)
-            hipLaunchKernelGGL(k_csr_split_rows<double>, dim3(b), dim3(256), 0, s, seg_info, split_seg, n_split, part,
-                               (double*) y, alpha, up, accumulate, rowmap);
-        else
-            hipLaunchKernelGGL(k_csr_split_rows<float>, dim3(b), dim3(256), 0, s, seg_info, split_seg, n_split, part,
-                               (float*) y, alpha, up, accumulate, rowmap);
-    }
-    return (int) hipGetLastError();
+    return csr_split_rows(seg_info, split_seg, n_split, part, y, y_is_double, alpha, up, accumulate, rowmap, s);
 }
 
 int
@@ -822,12 +1030,25 @@ csr_adaptive(const int64_t* indptr, const int32_t* col, const float* val, const 
                           alpha, up, accumulate, rowmap, nonempty, n_y, s);
 }
 int
-csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, const int64_t* seg_k,
-               const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg, int64_t n_split, double* part,
-               void* y, int y_is_double, double alpha, const double* up, int accumulate, const int32_t* rowmap,
-               const uint32_t* nonempty, int64_t n_y, hipStream_t s) {
-    return csr_adaptive_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, y, y_is_double,
-                          alpha, up, accumulate, rowmap, nonempty, n_y, s);
+csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, const float* x, int64_t n_x,
+               const int64_t* seg_k, const uint32_t* seg_info, int64_t n_seg, const int32_t* split_seg,
+               int64_t n_split, double* part, void* y, int y_is_double, double alpha, int accumulate,
+               const int32_t* rowmap, const uint32_t* nonempty, int64_t n_y, hipStream_t s) {
+    lds_shape L;
+    if (!lds_launch(n_x, n_seg, L))
+        return csr_adaptive_t(indptr, col, val, x, seg_k, seg_info, n_seg, split_seg, n_split, part, y, y_is_double,
+                              alpha, nullptr, accumulate, rowmap, nonempty, n_y, s);
+    const int zero = rowmap && !accumulate;
+    if (zero && (!nonempty || n_y <= 0)) return (int) hipErrorInvalidValue;
+    if (y_is_double)
+        hipLaunchKernelGGL(k_csr_lds<double>, dim3(L.blocks), dim3(64 * L.waves), L.bytes, s, indptr, col, val, x,
+                           (int) n_x, seg_k, seg_info, n_seg, part, (double*) y, alpha, accumulate, rowmap, nonempty,
+                           n_y, zero);
+    else
+        hipLaunchKernelGGL(k_csr_lds<float>, dim3(L.blocks), dim3(64 * L.waves), L.bytes, s, indptr, col, val, x,
+                           (int) n_x, seg_k, seg_info, n_seg, part, (float*) y, alpha, accumulate, rowmap, nonempty,
+                           n_y, zero);
+    return csr_split_rows(seg_info, split_seg, n_split, part, y, y_is_double, alpha, nullptr, accumulate, rowmap, s);
 }
 
 // ------------------------------------------------------------------ quadratic objective
@@ -840,7 +1061,7 @@ csr_adaptive16(const int64_t* indptr, const uint16_t* col, const float* val, con
 struct quad_set {
     int      n;
     quad_mat m[MQI_QUAD_MATS];
-    uint32_t block0[MQI_QUAD_MATS + 1];   // first workgroup of each matrix
+    uint32_t unit0[MQI_QUAD_MATS + 1];   // first unit of each matrix
 };
 
 // the objective's terms of the elements of y no row reaches (bit v of
@@ -854,7 +1075,7 @@ MQI_DI void quad_empty(const uint32_t* __restrict__ nonempty, int64_t n, const q
     constexpr int U      = 8;
     const int64_t stride = (int64_t) blocks * 64;
     double        acc    = 0.0;
-    for (int64_t v0 = (int64_t) b * 64 + threadIdx.x; v0 < n; v0 += U * stride) {
+    for (int64_t v0 = (int64_t) b * 64 + (threadIdx.x & 63); v0 < n; v0 += U * stride) {
         uint32_t bits[U];
 #pragma unroll
         for (int j = 0; j < U; ++j) {
@@ -878,22 +1099,48 @@ MQI_DI void quad_empty(const uint32_t* __restrict__ nonempty, int64_t n, const q
         }
     }
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-    if (threadIdx.x == 0) part[b] = acc;
+    if ((threadIdx.x & 63) == 0) part[b] = acc;
 }
 
+// unit `u` of the set: a part of a matrix' elements without a row, or a segment
 template<typename TC>
-__global__ void __launch_bounds__(64)
-k_quad(quad_set S, const float* __restrict__ x, quad_obj o, int64_t n_y) {
+MQI_DI void quad_unit(const quad_set& S, const float* __restrict__ x, quad_obj& o, int64_t n_y, uint32_t u,
+                      double* buf) {
     int i = 0;
-    while (i + 1 < S.n && blockIdx.x >= S.block0[i + 1]) ++i;
+    while (i + 1 < S.n && u >= S.unit0[i + 1]) ++i;
     const quad_mat& m = S.m[i];
-    const uint32_t  b = blockIdx.x - S.block0[i], nb = S.block0[i + 1] - S.block0[i];
+    const uint32_t  b = u - S.unit0[i];
     o.part            = m.terms;
     if (b < m.empty)
         quad_empty(m.nonempty, n_y, o, b, m.empty, m.terms + m.n_seg + m.n_split);
     else
-        csr_walk<double, TC, true>(m.indptr, (const TC*) m.col, m.val, x, m.seg_k, m.seg_info, b - m.empty,
-                                   nb - m.empty, m.n_seg, m.part, nullptr, m.alpha, nullptr, 0, o, m.rowmap);
+        csr_walk<double, TC, true>(m.indptr, (const TC*) m.col, m.val, x, m.seg_k, m.seg_info, b - m.empty, 1,
+                                   b - m.empty + 1, m.part, nullptr, m.alpha, nullptr, 0, o, m.rowmap, buf);
+}
+template<typename TC>
+__global__ void __launch_bounds__(64)
+k_quad(quad_set S, const float* __restrict__ x, quad_obj o, int64_t n_y) {
+    __shared__ double buf[MQI_SEG_BUF];
+    for (uint32_t u = blockIdx.x; u < S.unit0[S.n]; u += gridDim.x) quad_unit<TC>(S, x, o, n_y, u, buf);
+}
+// with x in LDS (k_csr_lds); block0: the first workgroup of each matrix
+struct quad_blocks {
+    uint32_t b[MQI_QUAD_MATS + 1];
+};
+__global__ void __launch_bounds__(1024)
+k_quad_lds(quad_set S, quad_blocks block0, const float* __restrict__ x, int n_x, quad_obj o, int64_t n_y) {
+    extern __shared__ double lds[];
+    const float* xs = stage_x(x, n_x, lds);
+    int          i  = 0;
+    while (i + 1 < S.n && blockIdx.x >= block0.b[i + 1]) ++i;
+    const quad_mat& m     = S.m[i];
+    const int64_t   waves = (int64_t) (block0.b[i + 1] - block0.b[i]) * (blockDim.x >> 6);
+    const int64_t   wave  = wave_index() - (int64_t) block0.b[i] * (blockDim.x >> 6);
+    o.part                = m.terms;
+    for (int64_t b = wave; b < m.empty; b += waves)
+        quad_empty(m.nonempty, n_y, o, (uint32_t) b, m.empty, m.terms + m.n_seg + m.n_split);
+    csr_stream<double, true>(m.indptr, (const uint16_t*) m.col, m.val, xs, m.seg_k, m.seg_info, wave, waves, m.n_seg,
+                             m.part, nullptr, m.alpha, 0, o, m.rowmap, lds + (threadIdx.x >> 6) * MQI_SEG_BUF);
 }
 
 // the split rows' terms, after the packed segments' ones (blockIdx.y: matrix)
@@ -953,32 +1200,43 @@ __global__ void __launch_bounds__(1024) k_quad_sum(quad_set S, double inv_n, dou
 }
 
 int
-csr_quadratic(const quad_mat* mats, int n, int cols16, const float* x, const double* p, const float* c, float* g,
-              int64_t n_y, double* f, hipStream_t s) {
+csr_quadratic(const quad_mat* mats, int n, int cols16, const float* x, int64_t n_x, const double* p, const float* c,
+              float* g, int64_t n_y, double* f, hipStream_t s) {
     if (n < 1 || n > MQI_QUAD_MATS || !p || !f || n_y <= 0 || (g && n != 1)) return (int) hipErrorInvalidValue;
     quad_set S{};
     S.n            = n;
-    int64_t blocks = 0, split = 0, terms = 0;
+    int64_t units = 0, segs = 0, split = 0, terms = 0;
     for (int i = 0; i < n; ++i) {
         quad_mat& m = S.m[i];
         m           = mats[i];
         if (m.n_seg <= 0 || !m.terms || (m.rowmap && !m.nonempty)) return (int) hipErrorInvalidValue;
         m.empty     = m.rowmap ? (uint32_t) std::min<int64_t>(MQI_QUAD_EMPTY_BLOCKS, (n_y + 511) / 512) : 0;
-        S.block0[i] = (uint32_t) blocks;
-        blocks += m.empty + std::min<int64_t>(m.n_seg, 262144);
+        S.unit0[i]  = (uint32_t) units;
+        units += m.empty + m.n_seg;
+        segs += m.n_seg;
         split = std::max(split, m.n_split);
         terms = std::max(terms, m.n_seg + m.n_split + (int64_t) m.empty);
     }
-    S.block0[n] = (uint32_t) blocks;
+    if (units > (int64_t) UINT32_MAX) return (int) hipErrorInvalidValue;
+    S.unit0[n] = (uint32_t) units;
     quad_obj o{};
     o.p         = p;
     o.c         = c;
     o.g         = g;
     o.two_inv_n = 2.0 / (double) n_y;
-    if (cols16)
-        hipLaunchKernelGGL(k_quad<uint16_t>, dim3((unsigned) blocks), dim3(64), 0, s, S, x, o, n_y);
+    lds_shape  L;
+    const dim3 blocks((unsigned) std::min<int64_t>(units, 262144));
+    if (cols16 && lds_launch(n_x, segs, L)) {
+        // workgroups by the matrices' work, at least one each
+        quad_blocks bl{};
+        for (int i = 0; i < n; ++i)
+            bl.b[i + 1] = bl.b[i] + (uint32_t) std::max<int64_t>(
+                                        1, (int64_t) L.blocks * (S.unit0[i + 1] - S.unit0[i]) / units);
+        hipLaunchKernelGGL(k_quad_lds, dim3(bl.b[n]), dim3(64 * L.waves), L.bytes, s, S, bl, x, (int) n_x, o, n_y);
+    } else if (cols16)
+        hipLaunchKernelGGL(k_quad<uint16_t>, blocks, dim3(64), 0, s, S, x, o, n_y);
     else
-        hipLaunchKernelGGL(k_quad<int32_t>, dim3((unsigned) blocks), dim3(64), 0, s, S, x, o, n_y);
+        hipLaunchKernelGGL(k_quad<int32_t>, blocks, dim3(64), 0, s, S, x, o, n_y);
     if (split > 0)
         hipLaunchKernelGGL(k_quad_split, dim3((unsigned) ((split + 255) / 256), (unsigned) n), dim3(256), 0, s, S, o);
     if (terms > MQI_QUAD_ONE)

@@ -128,3 +128,58 @@ def test_quadratic_backward_forms(ctx):
         v = torch.linspace(1.0, 2.0, 40, device="cuda", dtype=dt)
         (du,) = torch.autograd.grad((gu * v).sum(), up)
         assert torch.allclose(du, (g1.double() * v.double()).sum(), rtol=40 * 2.0 ** -23, atol=0)
+
+
+def _big(spots, voxels, seed):
+    """Voxel v in (a_v + 7 j) mod spots, j < k_v: 1 to 250 spots, all of them
+    (a row split over pieces) in some, none in every tenth."""
+    rng = np.random.default_rng(seed)
+    k = rng.integers(1, 251, voxels)
+    k[::1000] = min(spots, 1300)
+    k[5::10] = 0
+    k[-1] = 3
+    row = np.repeat(np.arange(voxels), k)
+    j = np.arange(k.sum()) - np.repeat(np.cumsum(k) - k, k)
+    col = (rng.integers(0, spots, voxels)[row] + 7 * j) % spots
+    m = sps.csr_matrix((rng.uniform(0.1, 1.0, len(row)).astype(np.float32), (col, row)), shape=(spots, voxels))
+    m.sort_indices()
+    return m
+
+
+@pytest.mark.parametrize("spots", [1300, 24576, 24577, 66000])   # x in LDS up to 24576; 32-bit columns from 65537
+def test_large_matrices(ctx, spots):
+    """More segments than the least for which workgroups stay."""
+    import torch
+    m = _big(spots, 100003, spots)
+    assert m.nnz > 8192 * 1100
+    (mat,) = _set(ctx, [m])
+    rng = np.random.default_rng(9)
+    w_np = rng.uniform(0.5, 1.5, spots).astype(np.float32)
+    w = torch.tensor(w_np, device="cuda")
+    ref = m.T.astype(np.float64) @ w_np.astype(np.float64) * mat.scale
+    # up to 1300 positive FP64 terms a voxel
+    tol = 1300 * 2.0 ** -52
+    y = mat.matvec(w)
+    np.testing.assert_allclose(y.cpu().numpy(), ref, rtol=tol, atol=0)
+    st = torch.cuda.current_stream().cuda_stream
+    y2 = y.clone()
+    ctx.dij_matvec(0, 0, w.data_ptr(), y2.data_ptr(), alpha=mat.scale, accumulate=True, stream=st)
+    np.testing.assert_allclose(y2.cpu().numpy(), 2 * ref, rtol=2 * tol, atol=0)
+    y3 = torch.full((m.shape[1],), 7.0, dtype=torch.float32, device="cuda")
+    ctx.dij_matvec(0, 0, w.data_ptr(), y3.data_ptr(), y_double=False, alpha=mat.scale, stream=st)
+    assert torch.equal(y3, y.to(torch.float32))
+    p_np, c_np = rng.uniform(0.0, 200.0, m.shape[1]), rng.uniform(0.0, 2.0, m.shape[1]).astype(np.float32)
+    p, c = torch.tensor(p_np, device="cuda"), torch.tensor(c_np, device="cuda")
+    for cc, c64 in ((None, 1.0), (c, c_np.astype(np.float64))):
+        f, g = mat.quadratic(w, p, cc)
+        r = y.cpu().numpy() - p_np
+        assert abs(f.item() - np.mean(c64 * r * r)) <= 1e5 * 2.0 ** -52 * np.mean(c64 * r * r)
+        # the rounded residual of a d and p that may cancel, then one rounding to float
+        err = 2.0 / m.shape[1] * c64 * (tol * (np.abs(ref) + p_np) + 2.0 ** -23 * np.abs(r))
+        assert np.all(np.abs(g.cpu().numpy() - 2.0 / m.shape[1] * c64 * r) <= err + 1e-37)
+    # two matrices side by side: the bits of one
+    from moquimc_amd import dij
+    mats = _set(ctx, [m, m])
+    got = dij._values(mats, w, p, c)
+    assert got[0].item() == mats[0].quadratic(w, p, c, want_grad=False)[0].item()
+    assert got[1].item() == mats[1].quadratic(w, p, c, want_grad=False)[0].item()
