@@ -12,9 +12,11 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <new>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/mqi_hip.h"
@@ -154,6 +156,8 @@ struct mqi_ctx {
     size_t                dij_items   = 0;
     std::vector<uint64_t> dij_off;                 // host copy of the offsets of the last run
     std::vector<csr_dev> dij;
+    std::unordered_map<void*, size_t> mat_bytes;   // the matrices' arrays
+    std::multimap<size_t, void*>      spare;       // during a build: the last one's arrays by size
 
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev_mv0 = nullptr, ev_mv1 = nullptr;   // around the last sparse product
@@ -264,41 +268,86 @@ dfree(T*& p) {
     p = nullptr;
 }
 
+// the device arrays of a matrix
+std::vector<void*>
+csr_arrays(const csr_dev& m) {
+    std::vector<void*> a = { m.indptr, m.col, m.val, m.tindptr, m.tnonempty, m.tcol, m.tval, m.nzvox, m.ccol, m.xc,
+                             m.sval, m.sd8, m.pesc, m.phdr, m.row_piece, m.ppart, m.tcol16 };
+    for (const csr_plan* p : {&m.plan, &m.tplan})
+        a.insert(a.end(), { p->seg_k, p->seg_info, p->split_seg, p->part, p->qpart });
+    return a;
+}
+
 void
-free_csr(csr_dev& m) {
-    {
-        dfree(m.indptr);
-        dfree(m.col);
-        dfree(m.val);
-        dfree(m.tindptr);
-        dfree(m.tnonempty);
-        dfree(m.tcol);
-        dfree(m.tval);
-        dfree(m.nzvox);
-        dfree(m.ccol);
-        dfree(m.xc);
-        dfree(m.sval);
-        dfree(m.sd8);
-        dfree(m.pesc);
-        dfree(m.phdr);
-        dfree(m.row_piece);
-        dfree(m.ppart);
-        dfree(m.tcol16);
-        for (csr_plan* p : {&m.plan, &m.tplan}) {
-            dfree(p->seg_k);
-            dfree(p->seg_info);
-            dfree(p->split_seg);
-            dfree(p->part);
-            dfree(p->qpart);
+free_csr(mqi_ctx* c, csr_dev& m) {
+    for (void* a : csr_arrays(m))
+        if (a) {
+            c->mat_bytes.erase(a);
+            hipFree(a);
         }
-    }
     m = csr_dev();
 }
 
 void
+free_spare(mqi_ctx* c) {
+    for (auto& a : c->spare) hipFree(a.second);
+    c->spare.clear();
+}
+
+void
 free_dij(mqi_ctx* c) {
-    for (auto& m : c->dij) free_csr(m);
+    for (auto& m : c->dij) free_csr(c, m);
     c->dij.clear();
+}
+
+// An array of a matrix: during a build one of the last build's of nearly the
+// same size (a build of nine scenarios frees and allocates some 150 arrays,
+// each hipFree waiting for the device), else a new one, its size rounded up
+// by at most a sixteenth so that the next build's nonzeros fit it too.
+template<typename T>
+int
+mat_alloc(mqi_ctx* c, T** p, size_t count) {
+    *p = nullptr;
+    if (count == 0) return 0;
+    const size_t need = count * sizeof(T);
+    size_t       unit = 256;
+    while (unit * 32 <= need) unit *= 2;
+    const size_t bytes = (need + unit - 1) / unit * unit;
+    const auto   it    = c->spare.lower_bound(need);
+    if (it != c->spare.end() && it->first <= bytes + unit) {
+        *p               = (T*) it->second;
+        c->mat_bytes[*p] = it->first;
+        c->spare.erase(it);
+        return 0;
+    }
+    hipError_t e = hipMalloc((void**) p, bytes);
+    if (e != hipSuccess && !c->spare.empty()) {
+        (void) hipGetLastError();
+        free_spare(c);
+        e = hipMalloc((void**) p, bytes);
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        return fail(c, MQI_E_MEMORY, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+    }
+    c->mat_bytes[*p] = bytes;
+    return 0;
+}
+
+// the matrices' arrays become the next build's; nothing still reads them
+int
+spare_dij(mqi_ctx* c) {
+    HIPCHK(c, hipDeviceSynchronize());
+    for (auto& m : c->dij) {
+        for (void* a : csr_arrays(m))
+            if (a) {
+                c->spare.emplace(c->mat_bytes[a], a);
+                c->mat_bytes.erase(a);
+            }
+        m = csr_dev();
+    }
+    c->dij.clear();
+    return 0;
 }
 
 // CSR-Adaptive segmentation of a row pointer array (cut_segments)
@@ -316,9 +365,9 @@ build_plan(mqi_ctx* c, const std::vector<Idx>& ip, csr_plan& P) {
     P.n_seg   = (int64_t) sk.size() - 1;
     P.n_split = (int64_t) split.size() / 2;
     int e;
-    if ((e = dalloc(c, &P.seg_k, sk.size())) || (e = dalloc(c, &P.seg_info, si.size())) ||
-        (e = dalloc(c, &P.split_seg, std::max<size_t>(split.size(), 1))) ||
-        (e = dalloc(c, &P.part, std::max<size_t>(P.n_seg, 1))))
+    if ((e = mat_alloc(c, &P.seg_k, sk.size())) || (e = mat_alloc(c, &P.seg_info, si.size())) ||
+        (e = mat_alloc(c, &P.split_seg, std::max<size_t>(split.size(), 1))) ||
+        (e = mat_alloc(c, &P.part, std::max<size_t>(P.n_seg, 1))))
         return e;
     HIPCHK(c, hipMemcpy(P.seg_k, sk.data(), sizeof(int64_t) * sk.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(P.seg_info, si.data(), sizeof(uint32_t) * si.size(), hipMemcpyHostToDevice));
@@ -424,9 +473,9 @@ build_pieces(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& ip, const build
     int32_t*     d_base = (int32_t*) (d_pb + np + 1);
     uint32_t*    d_ecnt = (uint32_t*) d_base + np;
     const size_t np1    = std::max<size_t>(np, 1);
-    if ((r = dalloc(c, &m.row_piece, rows + 1)) || (r = dalloc(c, &m.ppart, np1)) ||
-        (r = dalloc(c, &m.sval, std::max<int64_t>(staged, 1))) ||
-        (r = dalloc(c, &m.sd8, std::max<int64_t>(staged, 1))) || (r = dalloc(c, &m.phdr, np1)))
+    if ((r = mat_alloc(c, &m.row_piece, rows + 1)) || (r = mat_alloc(c, &m.ppart, np1)) ||
+        (r = mat_alloc(c, &m.sval, std::max<int64_t>(staged, 1))) ||
+        (r = mat_alloc(c, &m.sd8, std::max<int64_t>(staged, 1))) || (r = mat_alloc(c, &m.phdr, np1)))
         return r;
     HIPCHK(c, hipMemcpy(d_pk, pk.data(), sizeof(int64_t) * pk.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(m.row_piece, row_piece.data(), sizeof(int32_t) * (rows + 1), hipMemcpyHostToDevice));
@@ -448,7 +497,7 @@ build_pieces(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& ip, const build
     }
     if (n_esc + 64 > (uint64_t) UINT32_MAX) return fail(c, MQI_E_CAPACITY, "too many Dij escapes");
     const uint64_t n_esc_alloc = (n_esc + 64 + 1) & ~(uint64_t) 1;
-    if ((r = dalloc(c, &m.pesc, n_esc_alloc))) return r;
+    if ((r = mat_alloc(c, &m.pesc, n_esc_alloc))) return r;
     KCHK(c, mqi_aux::fill_u32(m.pesc, 0u, n_esc_alloc / 2, c->stream));
     if (np) HIPCHK(c, hipMemcpy(d_ecnt, ebase.data(), sizeof(uint32_t) * np, hipMemcpyHostToDevice));
     KCHK(c, mqi_aux::stage_pieces(m.val, d_dcol, d_pk, d_pb, d_ecnt, m.n_piece, m.sval, m.sd8, m.pesc, c->stream));
@@ -1770,10 +1819,10 @@ prepare_products(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& indptr, bui
     m.n_nz = (int64_t) n_nz;
     // D w over 16-bit spot columns where they fit
     const size_t padded = (size_t) m.nnz + MQI_SEG_PAD;
-    if ((r = m.rows <= 65536 ? dalloc(c, &m.tcol16, padded) : dalloc(c, &m.tcol, padded)) ||
-        (r = dalloc(c, &m.tval, padded)) || (r = dalloc(c, &m.tindptr, m.n_nz + 1)) ||
-        (r = dalloc(c, &m.tnonempty, (m.cols + 31) / 32)) || (r = dalloc(c, &m.nzvox, m.n_nz)) ||
-        (r = dalloc(c, &m.xc, m.n_nz)))
+    if ((r = m.rows <= 65536 ? mat_alloc(c, &m.tcol16, padded) : mat_alloc(c, &m.tcol, padded)) ||
+        (r = mat_alloc(c, &m.tval, padded)) || (r = mat_alloc(c, &m.tindptr, m.n_nz + 1)) ||
+        (r = mat_alloc(c, &m.tnonempty, (m.cols + 31) / 32)) || (r = mat_alloc(c, &m.nzvox, m.n_nz)) ||
+        (r = mat_alloc(c, &m.xc, m.n_nz)))
         return r;
     KCHK(c, mqi_aux::voxel_rows(ws.vox, ws.packed, m.nnz, ws.heads, m.nzvox, m.tindptr, ws.tptr32, m.tnonempty,
                                 m.cols, m.tcol16, m.tcol, m.tval, ws.vox2, ws.packed2, c->stream));
@@ -1786,7 +1835,7 @@ prepare_products(mqi_ctx* c, csr_dev& m, const std::vector<int64_t>& indptr, bui
     }
     // long rows (the Dij of pencil beams): D^T g over byte column deltas
     const bool pieces = m.nnz >= 1024 * m.rows;
-    if (!pieces && (r = dalloc(c, &m.ccol, m.nnz))) return r;
+    if (!pieces && (r = mat_alloc(c, &m.ccol, m.nnz))) return r;
     KCHK(c, mqi_aux::spot_rows(ws.packed, m.nzvox, m.nnz, m.col, pieces ? (int32_t*) ws.vox : m.ccol, m.val,
                                c->stream));
     std::vector<uint32_t> tptr(m.n_nz + 1);
@@ -1804,7 +1853,11 @@ mqi_dij_build(mqi_ctx* c, double rel_thr) {
     if (c->dij_items != (size_t) c->n_scen * c->spots.size())
         return fail(c, MQI_E_STATE, "the spots or scenarios changed since the run that scored the Dij tables");
     hipSetDevice(c->device);
-    free_dij(c);
+    if ((r = spare_dij(c))) return r;
+    struct spare_guard {
+        mqi_ctx* c;
+        ~spare_guard() { free_spare(c); }
+    } sg{c};
     const uint32_t n_items = (uint32_t) c->dij_items, n_spots = (uint32_t) c->spots.size();
     const uint32_t chunks  = dij_chunks(c);
     struct tables {
@@ -1842,15 +1895,19 @@ mqi_dij_build(mqi_ctx* c, double rel_thr) {
     }
     HIPCHK(c, hipMemcpy(d.count, cnt.data(), sizeof(uint32_t) * n_chunks, hipMemcpyHostToDevice));
     build_ws ws;
-    if (most && (r = build_scratch(c, ws, n_spots, (int64_t) nvox(c), most))) return r;
+    if (most && (r = build_scratch(c, ws, n_spots, (int64_t) nvox(c), most))) {
+        (void) hipGetLastError();
+        free_spare(c);
+        if ((r = build_scratch(c, ws, n_spots, (int64_t) nvox(c), most))) return r;
+    }
     c->dij.resize(c->n_scen);
     for (int s = 0; s < c->n_scen; ++s) {
         csr_dev& m = c->dij[s];
         m.rows     = n_spots;
         m.cols     = (int64_t) nvox(c);
         m.nnz      = indptr[s][n_spots];
-        if ((r = dalloc(c, &m.indptr, n_spots + 1)) || (r = dalloc(c, &m.col, std::max<int64_t>(1, m.nnz))) ||
-            (r = dalloc(c, &m.val, std::max<int64_t>(1, m.nnz))))
+        if ((r = mat_alloc(c, &m.indptr, n_spots + 1)) || (r = mat_alloc(c, &m.col, std::max<int64_t>(1, m.nnz))) ||
+            (r = mat_alloc(c, &m.val, std::max<int64_t>(1, m.nnz))))
             break;
         hipError_t e = hipMemcpy(m.indptr, indptr[s].data(), sizeof(int64_t) * (n_spots + 1), hipMemcpyHostToDevice);
         if (e == hipSuccess && m.nnz)
@@ -1889,19 +1946,19 @@ mqi_dij_set_csr(mqi_ctx* c, int s, int64_t rows, int64_t cols, const int64_t* in
     hipSetDevice(c->device);
     if ((int) c->dij.size() <= s) c->dij.resize(s + 1);
     csr_dev& m = c->dij[s];
-    free_csr(m);
+    free_csr(c, m);
     m.rows = rows;
     m.cols = cols;
     m.nnz  = nnz;
-    if ((r = dalloc(c, &m.indptr, rows + 1)) || (r = dalloc(c, &m.col, std::max<int64_t>(1, nnz))) ||
-        (r = dalloc(c, &m.val, std::max<int64_t>(1, nnz))))
+    if ((r = mat_alloc(c, &m.indptr, rows + 1)) || (r = mat_alloc(c, &m.col, std::max<int64_t>(1, nnz))) ||
+        (r = mat_alloc(c, &m.val, std::max<int64_t>(1, nnz))))
         return r;
     std::vector<int64_t> ip(indptr, indptr + rows + 1);
     HIPCHK(c, hipMemcpy(m.indptr, ip.data(), sizeof(int64_t) * (rows + 1), hipMemcpyHostToDevice));
     build_ws ws;
     if (nnz) {
         if ((r = build_scratch(c, ws, rows, cols, nnz))) {
-            free_csr(m);
+            free_csr(c, m);
             return r;
         }
         HIPCHK(c, hipMemcpy(ws.vox, indices, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
@@ -1909,7 +1966,7 @@ mqi_dij_set_csr(mqi_ctx* c, int s, int64_t rows, int64_t cols, const int64_t* in
         KCHK(c, mqi_aux::pack_rows(m.indptr, m.val, rows, ws.packed, c->stream));
     }
     if ((r = prepare_products(c, m, ip, ws))) {
-        free_csr(m);
+        free_csr(c, m);
         return r;
     }
     return 0;
@@ -2128,7 +2185,7 @@ quad_matrix(mqi_ctx* c, int s, double alpha, mqi_aux::quad_mat& q) {
     csr_plan& P = m.tplan;
     int       r = 0;
     if (!P.qpart &&
-        (r = dalloc(c, &P.qpart, P.n_seg + P.n_split + MQI_QUAD_EMPTY_BLOCKS + MQI_QUAD_SUM_BLOCKS)))
+        (r = mat_alloc(c, &P.qpart, P.n_seg + P.n_split + MQI_QUAD_EMPTY_BLOCKS + MQI_QUAD_SUM_BLOCKS)))
         return r;
     q = { m.tindptr, m.tcol16 ? (const void*) m.tcol16 : (const void*) m.tcol, m.tval, P.seg_k, P.seg_info,
           P.split_seg, m.nzvox, m.tnonempty, P.part, P.qpart, P.n_seg, P.n_split, alpha, 0 };
