@@ -79,9 +79,9 @@ def transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling):
                                                   "device, this run (clustered streams run faster: "
                                                   "profiles/atomic_probes.md)"),
                                   "counter_source": COUNTER_SOURCE}
-    out["limiter"] = ("VALU issue (valu_issue_frac of the issue slots busy); the FP64 atomic requests of the "
-                      "paired scorers run below the device's random-atomic rate (atomic_roofline) and HBM "
-                      "bandwidth is far from its ceiling (" + COUNTER_SOURCE + ")")
+    out["limiter"] = ("the FP64 atomic requests of the paired scorers, near the device's random-atomic rate "
+                      "(atomic_roofline); VALU issue at valu_issue_frac of its slots and HBM bandwidth far from "
+                      "its ceiling (" + COUNTER_SOURCE + ")")
     return out
 
 
