@@ -749,6 +749,9 @@ launch_bound(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int dyn
         return (int) hipErrorInvalidValue;
     pack_scoring(P);
     const size_t sh = shmem_bytes(c, cfg, threads, &P.dij_queued);
+    // the queue's lanes read the offsets of any (scenario, spot) of the plan
+    if (P.dij_queued && (!P.dij_off || c->dij_items != (size_t) c->n_scen * c->spots.size()))
+        return (int) hipErrorInvalidValue;
     if (dynamic) {
         const int e = mqi_aux::queue_init(P.queue, P.total, c->stream);
         if (e) return e;
@@ -1716,6 +1719,12 @@ mqi_trace(mqi_ctx* c, const mqi_run_config* cfg_in, const float* vertices, uint6
     hipSetDevice(c->device);
     mqi_run_config cfg = *cfg_in;
     if ((r = check_tuning(c, cfg))) return r;
+    // A trace scores nothing, and the Dij tables are those of the last Dij
+    // run, which may have had fewer spots or scenarios: the launch must not
+    // look into them (the production kernels read a voxel's key on every step).
+    if (cfg.dij && (!c->d_dij_keys || !c->d_dij_vals))
+        return fail(c, MQI_E_STATE, "trace: a Dij config needs an earlier Dij run");
+    cfg.dij = 0;
     run_plan       p;
     float*         d_v = nullptr;
     if (vertices) {
