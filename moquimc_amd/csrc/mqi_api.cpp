@@ -95,6 +95,7 @@ struct mqi_ctx {
     // doubles per element, zero between passes) and the arrays it folds into
     double*               d_pair     = nullptr;
     size_t                pair_cap   = 0;   // doubles
+    bool                  pair_optional = false;   // allocated by a pass that could do without
     size_t                pair_n     = 0;   // elements of the current pass (0: not grouped)
     int                   pair_ns = 0, pair_stride = 0;
     double*               pair_real[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -772,9 +773,26 @@ launch_bound(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int dyn
 // one atomic instruction from the group, folded into their arrays after the
 // pass.  The fold reads the whole array (4 to 8 ps per voxel), the groups save
 // some 5 to 10 ns per history, so a pass of less than a history per
-// MQI_PAIR_VOXELS voxels scores ungrouped, as does (optional) one whose array
-// the device has no memory for.
+// MQI_PAIR_VOXELS voxels scores ungrouped.  So does (optional) a plain pass or
+// one of caller-made vertices that would have to allocate more for the array
+// than MQI_PAIR_BYTES or a sixteenth of the device's free memory: with nine
+// scenarios of three scorers on 512x512x200 voxels it is 15 GB, which those
+// passes do not need.  An array they did allocate goes with the scorers.
 #define MQI_PAIR_VOXELS 1024
+#define MQI_PAIR_BYTES (1ull << 30)
+bool
+pair_room(size_t bytes) {
+    size_t free_b = 0, total_b = 0;
+    return bytes <= MQI_PAIR_BYTES && hipMemGetInfo(&free_b, &total_b) == hipSuccess && bytes <= free_b / 16;
+}
+
+void
+drop_pair(mqi_ctx* c) {
+    dfree(c->d_pair);
+    c->pair_cap      = 0;
+    c->pair_optional = false;
+}
+
 int
 pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, uint64_t histories, bool optional) {
     c->pair_n = 0;
@@ -786,8 +804,8 @@ pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, uint64_t 
     const size_t n      = (size_t) nvox(c) * (c->per_scen ? (size_t) c->n_scen : 1u);
     if (histories * MQI_PAIR_VOXELS < n) return 0;
     if (stride * n > c->pair_cap) {
-        dfree(c->d_pair);
-        c->pair_cap = 0;
+        if (optional && !pair_room(sizeof(double) * stride * n)) return 0;
+        drop_pair(c);
         int r = dalloc(c, &c->d_pair, stride * n);
         if (r && optional) {
             (void) hipGetLastError();
@@ -795,7 +813,8 @@ pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, uint64_t 
         }
         if (r) return r;
         KCHK(c, mqi_aux::fill_u64(c->d_pair, 0ull, stride * n, c->stream));
-        c->pair_cap = stride * n;
+        c->pair_cap      = stride * n;
+        c->pair_optional = optional;
     }
     for (int s = 0; s < ns; ++s) c->pair_real[s] = P.out[s];
     c->pair_n      = n;
@@ -1334,6 +1353,7 @@ mqi_set_scorers(mqi_ctx* c, int mask, int per_scenario) {
         c->kinds.push_back(MQI_KIND_STAT_DOSE);
         c->kinds.push_back(MQI_KIND_STAT_DOSE2);
     }
+    if (c->pair_optional) drop_pair(c);
     const uint64_t n = nvox(c) * (c->per_scen ? (uint64_t) c->n_scen : 1ull);
     for (int k = 0; k < MQI_MAX_SCORERS; ++k) {
         if (k < (int) c->kinds.size()) {
