@@ -101,7 +101,9 @@ class _Dose(torch.autograd.Function):
 
     @staticmethod
     def backward(fctx, grad_dose):
-        return fctx.mat.rmatvec(grad_dose, fctx.w_dtype), None
+        if type(fctx.mat) is DijMatrix:
+            return fctx.mat.rmatvec(grad_dose, fctx.w_dtype), None
+        return fctx.mat.rmatvec(grad_dose, torch.float64).to(fctx.w_dtype), None
 
 
 def dose(mat, w):
@@ -122,7 +124,9 @@ class _Quadratic(torch.autograd.Function):
     @staticmethod
     def backward(fctx, grad_f):
         (g,) = fctx.saved_tensors
-        up = _device_scalar(grad_f, g)
+        # the upstream factor goes into the product, unless the matrix has a
+        # product of its own
+        up = _device_scalar(grad_f, g) if type(fctx.mat) is DijMatrix else 0
         if up:
             return fctx.mat._adjoint(g, fctx.w_dtype, up), None, None, None
         grad_w = fctx.mat.rmatvec(g, torch.float64) * grad_f
@@ -153,10 +157,9 @@ def quadratic_objective(mat, w, prescription, voxel_weights=None):
 def _values(mats, w, prescription, voxel_weights):
     """The objective of every scenario (float64 vector), in one pass of
     launches where the scenarios are distinct ones of one context and size."""
-    first = mats[0] if mats else None
-    if (len({m.scenario for m in mats}) < len(mats) or not mats or
-            any(m.ctx is not first.ctx or type(m) is not DijMatrix or m.n_spots != first.n_spots or
-                m.n_voxels != first.n_voxels for m in mats)):
+    first = mats[0] if len(mats) else None
+    if (first is None or any(type(m) is not DijMatrix for m in mats) or len({m.scenario for m in mats}) < len(mats) or
+            any(m.ctx is not first.ctx or m.n_spots != first.n_spots or m.n_voxels != first.n_voxels for m in mats)):
         return torch.stack([m.quadratic(w, prescription, voxel_weights, want_grad=False)[0] for m in mats])
     w, p, c = first._objective_inputs(w, prescription, voxel_weights)
     f = torch.empty(len(mats), dtype=torch.float64, device=w.device)
