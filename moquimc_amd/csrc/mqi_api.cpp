@@ -96,6 +96,7 @@ struct mqi_ctx {
     double*               d_pair     = nullptr;
     size_t                pair_cap   = 0;   // doubles
     bool                  pair_optional = false;   // allocated by a pass that could do without
+    bool                  pair_dirty    = false;   // a pass that scores into it has not folded it yet
     size_t                pair_n     = 0;   // elements of the current pass (0: not grouped)
     int                   pair_ns = 0, pair_stride = 0;
     double*               pair_real[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -790,7 +791,7 @@ void
 drop_pair(mqi_ctx* c) {
     dfree(c->d_pair);
     c->pair_cap      = 0;
-    c->pair_optional = false;
+    c->pair_optional = c->pair_dirty = false;
 }
 
 int
@@ -815,7 +816,11 @@ pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, uint64_t 
         KCHK(c, mqi_aux::fill_u64(c->d_pair, 0ull, stride * n, c->stream));
         c->pair_cap      = stride * n;
         c->pair_optional = optional;
+    } else if (c->pair_dirty) {
+        // the last pass failed between its launches: its sums are not this one's
+        KCHK(c, mqi_aux::fill_u64(c->d_pair, 0ull, c->pair_cap, c->stream));
     }
+    c->pair_dirty = true;
     for (int s = 0; s < ns; ++s) c->pair_real[s] = P.out[s];
     c->pair_n      = n;
     c->pair_ns     = ns;
@@ -828,8 +833,10 @@ pair_setup(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, uint64_t 
 
 int
 pair_fold(mqi_ctx* c) {
-    if (c->pair_n)
+    if (c->pair_n) {
         KCHK(c, mqi_aux::pair_fold(c->pair_real, c->pair_ns, c->pair_stride, c->d_pair, c->pair_n, c->stream));
+        c->pair_dirty = false;
+    }
     return 0;
 }
 
