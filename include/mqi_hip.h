@@ -311,7 +311,10 @@ int mqi_last_matvec_ms(mqi_ctx* ctx, double* ms);
 
 /* Verification: the portable math functions on the device (fn 0 log, 1 exp,
  * 2 pow, 3 sin, 4 cos, 5 acos, 6 sqrt, 7 float divide, 8 double divide,
- * 9 float sqrt) on n host inputs. */
+ * 9 float sqrt) on n host inputs; and the production step's arithmetic: 10
+ * float quotient, 11 square root, 12 logarithm, 13 correctly rounded float
+ * quotient, 14 double quotient, 15 double square root, and the production
+ * build's own float division (16), square root (17) and logarithm (18). */
 int mqi_math_probe(mqi_ctx* ctx, int fn, const double* x, const double* y, int64_t n, double* out);
 
 /* Verification: the material and physics functions as the transport kernels

@@ -2344,7 +2344,10 @@ mqi_math_probe(mqi_ctx* c, int fn, const double* x, const double* y, int64_t n, 
     if ((r = dalloc(c, &dx, n)) || (r = dalloc(c, &dy, n)) || (r = dalloc(c, &dout, n))) return r;
     HIPCHK(c, hipMemcpy(dx, x, sizeof(double) * n, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(dy, y ? y : x, sizeof(double) * n, hipMemcpyHostToDevice));
-    KCHK(c, mqi_aux::math_probe(fn, dx, dy, dout, n, c->stream));
+    if (fn >= 10 && fn <= 18)
+        KCHK(c, mqi_fast::arith_probe(fn, dx, dy, dout, n, c->stream));
+    else
+        KCHK(c, mqi_aux::math_probe(fn, dx, dy, dout, n, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, hipMemcpy(out, dout, sizeof(double) * n, hipMemcpyDeviceToHost));
     hipFree(dx);

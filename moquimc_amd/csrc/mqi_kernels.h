@@ -183,6 +183,7 @@ int launch_transport(const transport_params& P, int debug, int dynamic, int trac
                      int threads, size_t shmem, hipStream_t stream);
 int occupancy(int debug, int dynamic, int trace, int waves, int threads, size_t shmem);
 int physics_probe(int debug, int fn, const float* rho, const float* ek, int64_t n, float* out, hipStream_t stream);
+int arith_probe(int fn, const double* x, const double* y, double* out, int64_t n, hipStream_t stream);
 }
 namespace mqi_fast6   // the production kernels with every scorer slot summed per voxel
 {

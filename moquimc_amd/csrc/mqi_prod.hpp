@@ -3,19 +3,20 @@
 // launch with fewer histories than lanes by the length of one wave's
 // instruction stream, so both run at the rate of the instructions per step.
 //
-// Every value is the one the expression-by-expression code of
-// mqi_transport.hip / mqi_device.hpp gives in this build: the same operations
-// are rounded in the same order, with the fused multiply-adds spelled out
-// (contraction is off here, so the code around an inlined call cannot change
-// them).  What is left out is work whose result is known: range scaling of
+// Every value is the one that the expressions of the verification build gave
+// when this build compiled them too: the same operations are rounded in the
+// same order, with the fused multiply-adds spelled out (contraction is off
+// here, so the code around an inlined call cannot change them).  What is left out is work whose result is known: range scaling of
 // divisions and square roots whose operands are nowhere near the ends of the
 // float range, products with the zeros and ones of a rotation's matrices, a
 // conversion to double around an operation that is exact in float, a table
-// index formed once per table.  Measured against the expression-by-expression
-// step: 2000-spot CT plan (512x512x200, dose and statistics) 437 -> 354 ms,
-// 25-spot slab phantom (dose and LETd, 2.5e6 histories) 49.6 -> 39.8 ms, one
-// 200 MeV spot of 1e5 histories in water 7.57 -> 6.11 ms, one launch per spot
-// 138 -> 103 ms for 40 spots.
+// index formed once per table.  The helpers are compared with IEEE results and
+// with this build's own operations on the device (mqi_math_probe 10 - 18).
+//
+// Measured against the expressions: 2000-spot CT plan (512x512x200, dose and
+// statistics) 437 -> 354 ms, 25-spot slab phantom (dose and LETd, 2.5e6
+// histories) 49.6 -> 39.8 ms, one 200 MeV spot of 1e5 histories in water 7.57
+// -> 6.11 ms, one launch per spot 138 -> 103 ms for 40 spots.
 #ifndef MQI_PROD_HPP
 #define MQI_PROD_HPP
 
@@ -39,12 +40,12 @@ constexpr float at_most(double c) {    // the largest float <= c, c > 0
 // a / b as this build's float division gives it (hardware reciprocal, one
 // multiplication), without the exponent handling the compiler wraps around
 // it (8 instructions): bit for bit the same for operands and results within
-// 2^-60 .. 2^60, checked on the device over 2^32 pairs
+// 2^-60 .. 2^60
 MQI_DI float q_div(float a, float b) {
     MQI_NO_CONTRACT
     return a * __builtin_amdgcn_rcpf(b);
 }
-// the same for the square root (arguments of 2^-96 and more, and 0); the
+// the same for the square root (arguments of 2^-96 .. 2^60, and 0); the
 // empty asm keeps the compiler from making one reciprocal square root, which
 // rounds differently, of a division by it
 MQI_DI float q_sqrt(float a) {
@@ -52,8 +53,11 @@ MQI_DI float q_sqrt(float a) {
     asm("" : "+v"(r));
     return r;
 }
-// natural logarithm of a normal, positive, finite float (hardware log2, ln 2
-// in two parts), as logf of this build without its denormal and infinity cases
+// natural logarithm of a normal, positive, finite float, bit for bit logf of
+// this build: the hardware's log2 times ln 2 as the sum of two floats, the
+// low part and the rounding error of the product added on (the last fused
+// multiply-add is what contraction makes of that addition: the error counts
+// twice, half an ulp at most)
 MQI_DI float q_log(float a) {
     MQI_NO_CONTRACT
     const float y  = __builtin_amdgcn_logf(a);
@@ -62,8 +66,10 @@ MQI_DI float q_log(float a) {
     e              = __builtin_fmaf(y, lo, e);
     return __builtin_fmaf(y, hi, e);
 }
-// correctly rounded a / b (the geometry): the compiler's sequence without its
-// range scaling, for |b| in 2^-13 .. 2^13 and |a| up to 2^60
+// correctly rounded a / b (the geometry) for |b| in 2^-13 .. 2^13 and a = 0 or
+// |a| in 2^-60 .. 2^60: the reciprocal after one Newton-Raphson step, the
+// quotient corrected by its residual, which a fused multiply-add gives exactly
+// (P. W. Markstein, IBM J. Res. Dev. 34 (1990) 111); no range scaling
 MQI_DI float r_div(float a, float b) {
     MQI_NO_CONTRACT
     float r = __builtin_amdgcn_rcpf(b);
@@ -72,8 +78,9 @@ MQI_DI float r_div(float a, float b) {
     q       = __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
     return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
 }
-// reciprocal and quotient in double to the same end: the correctly rounded
-// a / b is d_quot(a, b, d_recip(b)) for operands far from the range's ends
+// the same in double, from a hardware reciprocal of half the digits: the
+// correctly rounded a / b is d_quot(a, b, d_recip(b)) for operands within
+// 2^-200 .. 2^200 (and a = 0)
 MQI_DI double d_recip(double b) {
     MQI_NO_CONTRACT
     double r = __builtin_amdgcn_rcp(b);
@@ -86,8 +93,10 @@ MQI_DI double d_quot(double a, double b, double r) {
     return __builtin_fma(__builtin_fma(-b, q, a), r, q);
 }
 
-// correctly rounded square root in double of a normal a > 0 (the compiler's
-// sequence without its range scaling)
+// correctly rounded square root in double of a in 2^-700 .. 2^700:
+// Goldschmidt's iteration on sqrt(a) and 1 / (2 sqrt(a)) together, from the
+// hardware reciprocal square root, then two corrections by the residual
+// (Markstein, as above); no range scaling
 MQI_DI double d_sqrt(double a) {
     MQI_NO_CONTRACT
     const double y = __builtin_amdgcn_rsq(a);

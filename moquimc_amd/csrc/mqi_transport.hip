@@ -1939,6 +1939,39 @@ physics_probe(int debug, int fn, const float* rho, const float* ek, int64_t n, f
     return (int) hipGetLastError();
 }
 
+#if !MQI_EXACT
+// Verification probe of the step's arithmetic (mqi_prod.hpp) as this build
+// compiles it: fn 10 q_div, 11 q_sqrt, 12 q_log, 13 r_div (floats), 14 d_quot
+// by d_recip, 15 d_sqrt (doubles), and what the build's own float division
+// (16), square root (17) and logarithm (18) give.
+__global__ void __launch_bounds__(256)
+k_arith_probe(int fn, const double* x, const double* y, double* out, int64_t n) {
+    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float a = (float) x[i], b = (float) y[i];
+    double      r = 0.0;
+    switch (fn) {
+    case 10: r = (double) q_div(a, b); break;
+    case 11: r = (double) q_sqrt(a); break;
+    case 12: r = (double) q_log(a); break;
+    case 13: r = (double) r_div(a, b); break;
+    case 14: r = d_quot(x[i], y[i], d_recip(y[i])); break;
+    case 15: r = d_sqrt(x[i]); break;
+    case 16: r = (double) (a / b); break;
+    case 17: r = (double) sqrtf(a); break;
+    default: r = (double) logf(a); break;
+    }
+    out[i] = r;
+}
+
+int
+arith_probe(int fn, const double* x, const double* y, double* out, int64_t n, hipStream_t stream) {
+    if (n <= 0) return 0;
+    hipLaunchKernelGGL(k_arith_probe, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, stream, fn, x, y, out, n);
+    return (int) hipGetLastError();
+}
+#endif
+
 #endif
 
 // resident workgroups per CU of one instantiation
