@@ -874,15 +874,25 @@ check_tuning(mqi_ctx* c, const mqi_run_config& cfg) {
     return 0;
 }
 
-// waves_per_simd 0: 4 for a launch of more histories than the lanes of 3 hold,
-// 3 for a smaller one, which the longest track bounds: its wave runs alone on
-// a SIMD at the end, and the register budget of 3 spills nothing.  Slab
-// phantom (2.5e6 histories) 28.9 ms with 4 against 30.5 with 3, 2000-spot CT
-// 355 / 360, nine Dij scenarios (1.2e6) 8.9 / 9.8, Dij field (2e6) 14.6 /
-// 15.7; water spot (1e5) 5.20 / 5.12, small CT field (1.3e5) 2.83 / 2.84.
+// waves_per_simd 0: 4 for a launch of more histories than the lanes of 3 hold
+// (196,608), 3 for a smaller one, which the longest track bounds: its wave
+// runs alone on a SIMD at the end, and the register budget of 3 spills
+// nothing.  Ratio of the kernel's times with 3 and with 4, by histories (above
+// 1: 4 is faster):
+//                              1e5   1.95e5  2.15e5  2.6e5   4e5   1.5e6  3e6
+//   water spot, dose           0.95   0.91    1.13   1.16   1.00   1.11  1.13
+//   slabs, dose                0.96   0.97    1.01   1.13   0.99   1.10  1.13
+//   slabs, dose and LETd       0.97   0.97    0.99   1.12   1.01   1.10  1.12
+//   CT, dose                   0.94   0.93    0.99   1.04   1.01   0.98  1.07
+//   CT, dose and statistics    0.96   0.97    0.95   0.94   0.98   1.01  1.03
+//   CT, Dij                    0.98   0.96    0.97   1.04   1.06   1.08  1.11
+// The kernels of five and six scorers (mqi_fast6) spill with 4: 0.88 to 0.98
+// at every count from 5e4 to 3e6, for plans and vertices (six scorers in
+// slabs, 2.6e5 of a plan: 1.05), so they keep 3.
 int
-waves_for(const mqi_ctx* c, const mqi_run_config& cfg, uint64_t histories) {
+waves_for(const mqi_ctx* c, const mqi_run_config& cfg, uint64_t histories, int threads) {
     if (cfg.exact || cfg.waves_per_simd) return cfg.waves_per_simd;
+    if (deferred_slots(c, cfg, threads) > MQI_DEFER) return 3;
     return histories > (uint64_t) c->n_cu * 4 * 3 * 64 ? 4 : 3;
 }
 
@@ -975,7 +985,7 @@ transport_pass(mqi_ctx* c, const mqi_run_config& cfg_in, uint64_t hoff, double* 
         if (p.total == 0) return 0;
         P.n_items      = (int) p.item_end.size();
         P.total        = p.total;
-        cfg.waves_per_simd = waves_for(c, cfg, p.total);
+        cfg.waves_per_simd = waves_for(c, cfg, p.total, threads);
         const int blocks = persistent_blocks(c, cfg, threads, 0);
         if ((r = ensure_stack(c, lane_bytes * (size_t) blocks * threads))) return r;
         P.stack = c->d_stack;
@@ -1005,7 +1015,7 @@ transport_pass(mqi_ctx* c, const mqi_run_config& cfg_in, uint64_t hoff, double* 
         if ((r = upload_plan(c, p))) return r;
         P.n_items    = (int) p.item_end.size();
         P.total      = p.total;
-        cfg.waves_per_simd = waves_for(c, cfg_in, p.total);
+        cfg.waves_per_simd = waves_for(c, cfg_in, p.total, threads);
         uint64_t lanes = std::min<uint64_t>(p.total, max_lanes);
         int      blocks = (int) ((lanes + threads - 1) / threads);   // <= max_blocks
         HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1603,7 +1613,8 @@ mqi_run_vertices(mqi_ctx* c, const float* vtx, uint64_t n, const uint32_t* spot_
     mqi_run_config cfg = *cfg_in;
     if ((r = check_tuning(c, cfg))) return r;
     if (cfg.dij) return fail(c, MQI_E_ARG, "Dij scoring needs a spot table (mqi_run)");
-    cfg.waves_per_simd = waves_for(c, cfg, n);
+    const int threads  = cfg.block_size > 0 ? cfg.block_size : 256;
+    cfg.waves_per_simd = waves_for(c, cfg, n, threads);
     float*    d_v = nullptr;
     uint32_t* d_s = nullptr;
     if ((r = dalloc(c, &d_v, 7 * n))) return r;
@@ -1627,7 +1638,6 @@ mqi_run_vertices(mqi_ctx* c, const float* vtx, uint64_t n, const uint32_t* spot_
     KCHK(c, mqi_aux::fill_u64(c->d_counters, 0ull, 4, c->stream));
     KCHK(c, mqi_aux::fill_u32(c->d_status, 0u, 1, c->stream));
     KCHK(c, mqi_aux::fill_u64(c->d_hoff, cfg.hist_offset, 1, c->stream));
-    const int threads = cfg.block_size > 0 ? cfg.block_size : 256;
     int       blocks;
     if (cfg.batched) {
         blocks = persistent_blocks(c, cfg, threads, 0);

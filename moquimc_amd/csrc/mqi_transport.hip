@@ -17,9 +17,9 @@
 // (namespace mqi_fast, device math library, FMA contraction), and the latter
 // again with MQI_DEFER=6 (namespace mqi_fast6) for launches of five or six
 // scorers.  A fifth scorer added on every step cost 2.5 ms of the 11.9 of 3e5
-// histories with dose and four LET scorers (9.4 with its sum in LDS too);
-// built into mqi_fast the two slots cost every launch registers (143 -> 153
-// VGPRs, Dij field 18.9 -> 20.1 ms).
+// histories with dose and four LET scorers (9.4 with its sum in LDS too, 8.5
+// with the register budget of 3 waves/SIMD); built into mqi_fast the two slots
+// cost every launch registers (143 -> 153 VGPRs, Dij field 18.9 -> 20.1 ms).
 #include "mqi_device.hpp"
 #include "mqi_kernels.h"
 #if MQI_EXACT
@@ -1833,8 +1833,9 @@ variant pick_waves(int waves) {
     return make<D, Y, T, 0>();
 #else
     if (T) return make<D, Y, T, 0>();
-    // the callers choose between 3 and 4 (the budgets without spills in the
-    // step; 5 spills and is slower everywhere); 2: the compiler's own budget
+    // by default the callers choose between 3 and 4 (the budgets without spills
+    // in the step, 3 where it sums six scorers; 5 spills and is slower
+    // everywhere), a caller's config any of them; 2: the compiler's own budget
     switch (waves) {
     case 2: return make<D, Y, T, 0>();
     case 4: return make<D, Y, T, 4>();
