@@ -133,7 +133,7 @@ struct transport_params {
     uint64_t out_scenario_stride;   // 0: scenarios share the arrays; else per-scenario offset (elements)
     int      loops;
     uint32_t kind_word;   // kinds[], four bits each
-    uint32_t mode_word;   // MQI_MODE_*
+    uint32_t mode_word;   // mqi_mode
     // Grouped scoring (production kernels, each-scorer-once, no Dij): the
     // leading group_ns scorers (2 .. 4) add into one interleaved array with
     // pair (2 or 4; 0: off) doubles per element, element i of scorer s at

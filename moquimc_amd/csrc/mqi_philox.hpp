@@ -118,18 +118,6 @@ struct stream {
         return (float) ((w >> 8) + 1u) * (1.0f / 16777216.0f);
     }
 
-    // block `b` of this history's stream for another purpose (same key and
-    // history, spot, scenario)
-    MQI_HD u32x4
-    block_of(uint32_t purpose, uint32_t b) const {
-        u32x4 c;
-        c.v[0] = b;
-        c.v[1] = c1;
-        c.v[2] = c2;
-        c.v[3] = (c3 & ~0xffu) | purpose;
-        return philox4x32_10(c, key0, key1);
-    }
-
     // Standard normal variate in double (Box-Muller pair, second one cached).
     MQI_HD double
     gauss() {
