@@ -79,9 +79,11 @@ def transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling):
                                                   "device, this run (clustered streams run faster: "
                                                   "profiles/atomic_probes.md)"),
                                   "counter_source": COUNTER_SOURCE}
-    out["limiter"] = ("the FP64 atomic requests of the paired scorers, near the device's random-atomic rate "
-                      "(atomic_roofline); VALU issue at valu_issue_frac of its slots and HBM bandwidth far from "
-                      "its ceiling (" + COUNTER_SOURCE + ")")
+    if m and sq:   # the counters' launch shape; their shares are not those of another one
+        out["counter_launch"] = m["launch"]
+    out["limiter"] = ("VALU issue (valu_issue_frac of the slots) and the FP64 atomic requests of the paired scorers "
+                      "together: the requests run at the rate of uniformly random atomics (atomic_roofline), which "
+                      "clustered ones may exceed; HBM bandwidth is far from its ceiling (" + COUNTER_SOURCE + ")")
     return out
 
 
@@ -295,7 +297,7 @@ def phantom_bench(ctx_cls, reps=3):
     return {"phantoms": out}
 
 
-def transport_pass(waves=3, block=128, fetch=1, refill=4):
+def transport_pass(waves, block, fetch, refill):
     """One production batched pass of the 2000-spot CT plan (dose + the
     statistics pair) with a fixed launch shape: a single k_transport dispatch
     for the counter runs."""
@@ -426,6 +428,9 @@ def main():
                     help="only the FP64 atomic rate, uniform and clustered (mqi_atomic_probe)")
     ap.add_argument("--transport-pass", action="store_true",
                     help="only one production pass of the CT plan with a fixed launch shape (the counter runs)")
+    ap.add_argument("--launch", default="4,256,2,64", metavar="W,B,F,R",
+                    help="its waves/SIMD, workgroup size, histories per fetch and refill lanes; the default is the "
+                         "autotuner's pick (4,256,1,4: an untuned launch's)")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (each GPU would take its own slice "
@@ -436,7 +441,7 @@ def main():
         copy_calibration()
         return
     if args.transport_pass:
-        transport_pass()
+        transport_pass(*(int(x) for x in args.launch.split(",")))
         return
     if args.atomic_probes:
         atomic_probes()
