@@ -44,7 +44,7 @@ def measured_traffic(key):
         return None
 
 
-def transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling):
+def transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling, refill):
     """Algorithmic bytes of the transport: per voxel step one density load
     (4 B) and one FP64 read-modify-write per scorer (8 B each), over the
     average duration of one persistent launch (HIP events on its stream).
@@ -52,7 +52,9 @@ def transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling):
     and lane activity of the pass (SQ counters), and its FP64 atomic rate
     (TCC_ATOMIC per voxel step from the counter run, scaled to this launch)
     against the rate mqi_atomic_probe measures for random FP64 atomics on
-    this device (atomic_ceiling, atomics/s, None when not measured)."""
+    this device (atomic_ceiling, atomics/s, None when not measured).  The
+    counters are those of whole-wave refills or of small ones, as the launch
+    refills (refill: its lanes); counter_launch names their launch."""
     bytes_per_step = 4.0 + 8.0 * n_scorers
     per_launch = steps / launches * bytes_per_step
     ms_per_launch = kernel_ms / launches
@@ -66,21 +68,19 @@ def transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling):
            "kernel": "k_transport<release, dynamic> (persistent)", "launch_ms": round(ms_per_launch, 3),
            "voxel_steps_per_launch": int(steps / launches), "bytes_per_step": bytes_per_step,
            "scorer_deposits_per_s": round(steps * n_scorers / (kernel_ms * 1e-3), 1)}
-    sq = measured_traffic("k_transport_sq")
-    if sq:
-        out["valu_issue_frac"] = sq["valu_issue_frac"]
-        out["valu_lanes_active"] = sq["valu_lanes_active"]
-    if m and "atomics" in m:
-        rate = m["atomics"] / m["voxel_steps"] * steps / launches / (ms_per_launch * 1e-3)
+    c = measured_traffic("k_transport_whole_wave" if refill >= 60 else "k_transport_untuned")
+    if c:
+        out["counter_launch"] = c["launch"]
+        out["valu_issue_frac"] = c["valu_issue_frac"]
+        out["valu_lanes_active"] = c["valu_lanes_active"]
+        rate = c["atomics"] / c["voxel_steps"] * steps / launches / (ms_per_launch * 1e-3)
         out["atomic_roofline"] = {"achieved": float("%.4g" % rate), "peak": atomic_ceiling, "unit": "atomics/s",
                                   "frac": round(rate / atomic_ceiling, 4) if atomic_ceiling else None,
-                                  "atomics_per_voxel_step": round(m["atomics"] / m["voxel_steps"], 4),
+                                  "atomics_per_voxel_step": round(c["atomics"] / c["voxel_steps"], 4),
                                   "peak_source": ("mqi_atomic_probe, uniformly random FP64 atomic adds on this "
                                                   "device, this run (clustered streams run faster: "
                                                   "profiles/atomic_probes.md)"),
                                   "counter_source": COUNTER_SOURCE}
-    if m and sq:   # the counters' launch shape; their shares are not those of another one
-        out["counter_launch"] = m["launch"]
     out["limiter"] = ("VALU issue (valu_issue_frac of the slots) and the FP64 atomic requests of the paired scorers "
                       "together: the requests run at the rate of uniformly random atomics (atomic_roofline), which "
                       "clustered ones may exceed; HBM bandwidth is far from its ceiling (" + COUNTER_SOURCE + ")")
@@ -541,7 +541,7 @@ def main():
            "batched_vs_plain_dose": agree,
            "secondaries_dropped_per_step": round(dropped / args.steps, 1),
            "steps_per_history": round(steps / max(1, hist), 1),
-           "roofline": transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling(ctx))}
+           "roofline": transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling(ctx), cfg.refill_lanes)}
     ctx.close()
     if not args.no_adjoint:
         try:
