@@ -82,7 +82,7 @@ def transport_roofline(steps, kernel_ms, launches, n_scorers, atomic_ceiling, re
                                                   "profiles/atomic_probes.md)"),
                                   "counter_source": COUNTER_SOURCE}
     out["limiter"] = ("VALU issue (valu_issue_frac of the slots) and the FP64 atomic requests of the paired scorers "
-                      "together: the requests run at the rate of uniformly random atomics (atomic_roofline), which "
+                      "together: the requests run near the rate of uniformly random atomics (atomic_roofline), which "
                       "clustered ones may exceed; HBM bandwidth is far from its ceiling (" + COUNTER_SOURCE + ")")
     return out
 

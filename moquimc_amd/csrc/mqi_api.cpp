@@ -767,8 +767,8 @@ launch_bound(mqi_ctx* c, transport_params& P, const mqi_run_config& cfg, int dyn
                                       c->stream);
 }
 
-// Grouped scoring for a batched pass of the production kernels with each
-// scorer scored once, no Dij and at least two scorers: the leading deferred
+// Grouped scoring for a pass of the production kernels with each scorer
+// scored once, no Dij and at least two scorers: the leading deferred
 // scorers (two: pairs of lanes; three or four: groups of four lanes) add
 // into one interleaved array, all sums of a voxel in one line and added by
 // one atomic instruction from the group, folded into their arrays after the
